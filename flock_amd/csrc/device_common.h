@@ -43,6 +43,9 @@ constexpr int32_t kPadCost = 1 << 30;
 __device__ __forceinline__ int32_t imin(int32_t a, int32_t b) { return a < b ? a : b; }
 constexpr uint64_t kNoKey = ~0ull;
 
+// Keeps the instruction scheduler from moving anything across this point.
+__device__ __forceinline__ void sched_fence() { __builtin_amdgcn_sched_barrier(0); }
+
 // Per-instance descriptor in device memory.  Inputs are written by the host before a
 // launch; outputs (objective .. status) and the basis/dual arrays are written by the
 // engine.  Matrices are row-major with a padded pitch (multiple of 4 int32 = 16 bytes):

@@ -27,8 +27,15 @@ namespace flock {
 // ---------------------------------------------------------------------------
 // groups
 // ---------------------------------------------------------------------------
+// The rank is opaque to the compiler at each call: values derived from it are computed
+// again in the phase that uses them, where the optimiser would otherwise hoist them to the
+// kernel's entry and spill them (up to 40 registers in the work-queue kernels).
 template <int G>
-__device__ __forceinline__ int grank() { return (int)(threadIdx.x % G); }
+__device__ __forceinline__ int grank() {
+  int r = (int)(threadIdx.x % G);
+  asm volatile("" : "+v"(r));
+  return r;
+}
 
 template <int G>
 __device__ __forceinline__ void gsync() {
@@ -984,22 +991,41 @@ __device__ bool build_tree(const Ctx& C, gcint* brow, gcint* bcol, gcint* bflow,
 // Reduced-cost sweep fused with the argmin (computeReducedCosts + thrust::min_element,
 // parallel_kernels.cu:329-353 and uv_model_parallel.cu:169; host scan :184-194):
 // r_ij = c_ij - u_i - v_j over all cells, minimum r, ties -> lowest row-major index.
-// The padded matrix is walked as a flat array of 16-byte vectors; rank t takes
-// vectors t, t+G, t+2G, ... in increasing order, kSweepUnroll loads in flight at a time.
-// The rank's vectors are dealt round-robin to K slots (slot = position in the unrolled
-// batch mod K); a strict `<` keeps each slot's first minimum, so the least (r, index)
-// key over the slots is the rank's, and the group min over ranks finishes the argmin.
-// Each slot's best cell is also a pricing candidate (K per rank).
+// The padded matrix is walked in blocks of kSlots * G 16-byte vectors that are whole rows:
+// slot s of rank t holds position p = t + s*G of the block, i.e. column vector p % w and
+// row p / w of the block's h = kSlots*G / w rows (w vectors per row), and the next block
+// is h rows further down.  A slot's columns never change, so their four duals stay in
+// registers and its next address is one uniform step away: per vector one LDS read (u),
+// the four subtractions and the running minimum remain, 11 vector-ALU instructions.
+// (Vectors dealt to ranks by flat index took 23: a 40-bit multiply for the row, both
+// addresses and an LDS read of the four duals each time.)  The load of a slot's next
+// vector is issued as soon as its present one is consumed, so kSlots loads stay in flight
+// across blocks.  Positions past the block or the matrix repeat the last one.
+// A strict `<` keeps each slot's first minimum (rows only grow), so the least
+// (r, row, column) key over the slots is the rank's, and the group min over ranks finishes
+// the argmin.  With K = kSlots each slot's best cell is also a pricing candidate; with
+// K = 1 (one pivot per sweep) the rank's single best cell is, and only its vector is read
+// again to find the column inside it.
+// Bound: one compute unit's cache bandwidth (about 64 bytes a clock, 150 GB/s) for large
+// matrices, load latency and the closing minimum for small ones.  A sweep of 500x480 at
+// 512 threads went from 15.1 to 8.2 us (64 -> 117 GB/s), one of 100x100 at 256 threads from
+// 3.0 to 1.8 us; the 4096-instance batch from 10.2 to 9.43 ms (candidates) and from 58 to
+// 38 ms (Dantzig).
 // ---------------------------------------------------------------------------
 // 16-byte loads in flight per rank: 8 for workgroup groups, 4 for wavefront groups
 template <int G>
-struct SweepUnroll { static constexpr int value = G == kWave ? 4 : 8; };
+struct SweepSlots { static constexpr int value = G == kWave ? 4 : 8; };
 // candidates per rank: 8 for workgroup groups (2048 at 256 threads, 8192 at 1024; more
 // candidates measured fewer sweeps and pivots at every group size: at 1024 threads an
 // 1800x1800 instance needs 1645 sweeps instead of 7692 with one per rank), 4 for
 // wavefront groups
 template <int G>
 struct CandsPerRank { static constexpr int value = G == kWave ? 4 : 8; };
+
+// Cell (row, col) as one word whose order is row-major order (m+n <= 16383)
+__device__ __forceinline__ uint32_t cell_id(uint32_t row, uint32_t col) { return (row << 16) | col; }
+__device__ __forceinline__ int cell_row(uint64_t key) { return (int)((uint32_t)key >> 16); }
+__device__ __forceinline__ int cell_col(uint64_t key) { return (int)((uint32_t)key & 0xffffu); }
 
 struct Cand {
   int32_t row, col, cost;
@@ -1026,80 +1052,165 @@ struct CandSet {
   }
 };
 
+// Shape of a sweep over w column vectors: a block is h rows, the matrix `full` whole
+// blocks and `rest` rows.  p / w is the high word of p * magic, exact while p * w < 2^32
+// (both are at most kSlots * G <= 8192).
+struct SweepShape {
+  uint32_t w, magic, h, full, rest;
+  __device__ __forceinline__ uint32_t div(uint32_t p) const {
+    return w > 1 ? (uint32_t)(((uint64_t)p * magic) >> 32) : p;
+  }
+};
+template <int G>
+__device__ __forceinline__ SweepShape sweep_shape(int m, int w) {
+  SweepShape s;
+  s.w = (uint32_t)w;
+  s.magic = w > 1 ? 0xffffffffu / (uint32_t)w + 1 : 0;
+  s.h = s.div((uint32_t)(SweepSlots<G>::value * G));
+  s.full = (uint32_t)m / s.h;
+  s.rest = (uint32_t)m - s.full * s.h;
+  return s;
+}
+// whether a row can be longer than one block (wavefront groups with n > 1024 only: a
+// workgroup's block is at least 8192 columns, more than m+n of any instance in LDS)
+template <int G>
+struct SweepChunks { static constexpr bool value = SweepSlots<G>::value * G * 4 < 8000; };
+
+// shape: sweep_shape<G> of the whole row (used unless SweepChunks)
 template <int G, int K>
-__device__ uint64_t sweep_argmin(const Ctx& C, const TreeLds& t, Shared& S, CandSet<K>& mine) {
-  const uint32_t vpr = (uint32_t)C.ld >> 2;
-  const uint32_t nvec = (uint32_t)C.m * vpr;
-  // q / vpr as (q * magic) >> 40 with magic = floor(2^40 / vpr) + 1: the error term is
-  // below q / 2^40 < 2^-16 while the fractional part of q / vpr is at most
-  // 1 - 1/vpr, so the quotient is exact for q < 2^24 and vpr <= 2^11 (m*n <= 2^26).
-  const uint64_t magic = (0x10000000000ull / vpr) + 1;
-  const uint32_t ld = (uint32_t)C.ld;
-  constexpr int kSweepUnroll = SweepUnroll<G>::value;
-  static_assert(kSweepUnroll % K == 0, "slots must divide the unrolled batch");
-  // per vector only its minimum reduced cost is compared (strict <, so the slot's first
-  // minimum vector wins); the winning cell inside that vector is recovered once at the end
-  int32_t bestR[K];
-  uint32_t bestQ[K];
+__device__ uint64_t sweep_argmin(const Ctx& C, const TreeLds& t, Shared& S, const SweepShape& shape, CandSet<K>& mine) {
+  constexpr int kSlots = SweepSlots<G>::value;
+  static_assert(K == 1 || K == kSlots, "one candidate per rank or one per slot");
+  constexpr bool kChunks = SweepChunks<G>::value;
+  // the rank index, opaque to the compiler here: the slots' positions depend on nothing
+  // else, and kept across the pivots between two sweeps they would spill
+  int tidr = grank<G>();
+  asm volatile("" : "+v"(tidr));
+  const uint32_t tid = (uint32_t)tidr;
+  const uint32_t m = (uint32_t)C.m, ld = (uint32_t)C.ld;
+  const uint32_t vpr = ld >> 2;
+  typedef const FLOCK_GLOBAL char gcbyte;
+  int32_t bestR[kSlots];
+  uint32_t bestRow[kSlots], col[kSlots];
 #pragma unroll
-  for (int k = 0; k < K; ++k) { bestR[k] = kBig; bestQ[k] = 0xffffffffu; }
-  for (uint32_t q0 = (uint32_t)grank<G>(); q0 < nvec; q0 += kSweepUnroll * G) {
-    i32x4 cv[kSweepUnroll];
-    uint32_t rw[kSweepUnroll], c4[kSweepUnroll];
-    // addresses first, loads unconditional (out-of-range slots re-read vector 0), so all
-    // kSweepUnroll loads are in flight together
+  for (int s = 0; s < kSlots; ++s) { bestR[s] = kBig; bestRow[s] = 0; col[s] = 0; }
+  uint32_t c0 = 0;
+  do {
+    const SweepShape sh =
+        kChunks ? sweep_shape<G>((int)m, (int)(vpr - c0 < (uint32_t)(kSlots * G) ? vpr - c0 : (uint32_t)(kSlots * G)))
+                : shape;
+    const uint32_t rowBytes = 4 * ld, blockBytes = sh.h * rowBytes;
+    // row and column of a slot's position in a block
+    auto place = [&](uint32_t rank, int s, uint32_t* row, uint32_t* cc) {
+      uint32_t p = rank + (uint32_t)(s * G);
+      p = p < sh.h * sh.w ? p : sh.h * sh.w - 1;
+      *row = sh.div(p);
+      *cc = 4 * (c0 + p - *row * sh.w);
+    };
+    uint32_t row[kSlots], off[kSlots];  // off: byte offset of the slot's vector in the block at hand
+    i32x4 dv[kSlots], cv[kSlots];
 #pragma unroll
-    for (int k = 0; k < kSweepUnroll; ++k) {
-      const uint32_t q = q0 + (uint32_t)k * G;
-      const uint32_t qq = q < nvec ? q : nvec - 1;  // slots past the matrix repeat the last vector
-      const uint32_t r = (uint32_t)(((uint64_t)qq * magic) >> 40);
-      rw[k] = r; c4[k] = qq - r * vpr;
-      cv[k] = *(const FLOCK_GLOBAL i32x4*)(C.cost + (r * ld + 4 * c4[k]));
+    for (int s = 0; s < kSlots; ++s) {
+      uint32_t cc;
+      place(tid, s, &row[s], &cc);
+      off[s] = row[s] * rowBytes + 4 * cc;
+      const uint32_t back = row[s] < m ? 0 : row[s] - (m - 1);  // rows past the matrix repeat the last
+      cv[s] = *(const FLOCK_GLOBAL i32x4*)((gcbyte*)C.cost + (off[s] - back * rowBytes));
+      dv[s] = *(const i32x4*)(t.dv + cc);
+    }
+    auto take = [&](int s, uint32_t r, const i32x4& c) {
+      const int32_t u = t.du[r];
+      const int32_t mn = imin(imin(c.x - dv[s].x, c.y - dv[s].y), imin(c.z - dv[s].z, c.w - dv[s].w)) - u;
+      bool better = mn < bestR[s];
+      if constexpr (kChunks) {
+        uint32_t rr, cc;
+        place(tid, s, &rr, &cc);
+        better = better | ((mn == bestR[s]) & (cell_id(r, cc) < cell_id(bestRow[s], col[s])));
+        col[s] = better ? cc : col[s];
+      }
+      bestR[s] = better ? mn : bestR[s];
+      bestRow[s] = better ? r : bestRow[s];
+    };
+    const uint32_t blocks = sh.full + (sh.rest ? 1u : 0u);
+    uint32_t b = 0;
+    gcbyte* next = (gcbyte*)C.cost + blockBytes;
+    for (; b + 1 < sh.full; ++b) {  // this block and the next are whole
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        take(s, b * sh.h + row[s], cv[s]);
+        cv[s] = *(const FLOCK_GLOBAL i32x4*)(next + off[s]);
+        sched_fence();  // keep one vector per slot in registers, not two
+      }
+      next += blockBytes;
+    }
+    if (b + 1 < blocks) {  // the last whole block, then the partial one
+      const uint32_t left = m - (b + 1) * sh.h;  // rows of the partial block
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        take(s, b * sh.h + row[s], cv[s]);
+        const uint32_t back = row[s] < left ? 0 : row[s] - (left - 1);
+        cv[s] = *(const FLOCK_GLOBAL i32x4*)(next + (off[s] - back * rowBytes));
+        sched_fence();
+      }
+      ++b;
     }
 #pragma unroll
-    for (int k = 0; k < kSweepUnroll; ++k) {
-      const uint32_t q = q0 + (uint32_t)k * G;
-      const uint32_t qq = q < nvec ? q : nvec - 1;
-      const i32x4 vv = *(const i32x4*)(t.dv + 4 * c4[k]);
-      const int32_t u = t.du[rw[k]];
-      // min over the vector of c - v, then - u once (the row is the vector's); padding
-      // cells (cost kPadCost, dual 0) price positive and never hold a negative minimum.
-      // A repeated last vector has the same (r, index) keys as the original.
-      const int32_t mn = imin(imin(cv[k].x - vv.x, cv[k].y - vv.y), imin(cv[k].z - vv.z, cv[k].w - vv.w)) - u;
-      const bool better = mn < bestR[k % K];
-      bestR[k % K] = better ? mn : bestR[k % K];
-      bestQ[k % K] = better ? qq : bestQ[k % K];
+    for (int s = 0; s < kSlots; ++s) {
+      const uint32_t r = b * sh.h + row[s];
+      take(s, r < m ? r : m - 1, cv[s]);
     }
-  }
-  // recover each slot's cell (its vector reloaded; the K loads in flight together)
-  i32x4 cv[K];
-  uint32_t rr[K], cc4[K];
+    if constexpr (!kChunks) {
+      // the slots' columns, computed again rather than kept through the loop
+      int tide = grank<G>();
+      asm volatile("" : "+v"(tide));
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const uint32_t q = bestQ[k] != 0xffffffffu ? bestQ[k] : 0u;
-    rr[k] = (uint32_t)(((uint64_t)q * magic) >> 40);
-    cc4[k] = q - rr[k] * vpr;
-    cv[k] = *(const FLOCK_GLOBAL i32x4*)(C.cost + (rr[k] * ld + 4 * cc4[k]));
-  }
+      for (int s = 0; s < kSlots; ++s) {
+        uint32_t rr;
+        place((uint32_t)tide, s, &rr, &col[s]);
+      }
+    }
+    c0 += (uint32_t)(kSlots * G);
+  } while (kChunks && c0 < vpr);
+  // A real cell's c - v is at most V * max cost < 2^30, so a padding cell (cost 2^30,
+  // dual 0) is never its vector's minimum.
   uint64_t key = kNoKey;
+  if constexpr (K == 1) {
+    // the rank's least (r, row, first column of the vector), then the vector's first cell
+    // at the minimum: the vectors are disjoint and ordered, so this is row-major order
+    int32_t r = kBig;
+    uint32_t id = ~0u;
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const bool none = bestQ[k] == 0xffffffffu;
-    const uint32_t r = rr[k], c = cc4[k];
-    const int32_t u = t.du[r];
-    const i32x4 vv = *(const i32x4*)(t.dv + 4 * c);
-    const int32_t cc[4] = {cv[k].x, cv[k].y, cv[k].z, cv[k].w};
-    const int32_t dv[4] = {vv.x, vv.y, vv.z, vv.w};
-    int e = 3;
+    for (int s = 0; s < kSlots; ++s) {
+      const uint32_t is = cell_id(bestRow[s], col[s]);
+      const bool better = (bestR[s] < r) | ((bestR[s] == r) & (is < id));
+      r = better ? bestR[s] : r;
+      id = better ? is : id;
+    }
+    const uint32_t br = id >> 16, bc = id & 0xffffu;
+    const i32x4 c = *(const FLOCK_GLOBAL i32x4*)((gcbyte*)C.cost + 4 * (br * ld + bc));
+    const int32_t u = t.du[br];
+    const i32x4 vv = *(const i32x4*)(t.dv + bc);
+    const int e = c.x - vv.x - u == r ? 0 : c.y - vv.y - u == r ? 1 : c.z - vv.z - u == r ? 2 : 3;
+    mine.rc[0] = (int32_t)(id + (uint32_t)e);
+    mine.cost[0] = e == 0 ? c.x : e == 1 ? c.y : e == 2 ? c.z : c.w;
+    key = pack_vi(r, id + (uint32_t)e);
+  } else {
+    // each slot's first cell at its minimum (its vector reloaded; the K loads together)
+    i32x4 cv[K];
 #pragma unroll
-    for (int j = 3; j >= 0; --j)  // first cell at the minimum
-      e = (4 * (int)c + j < C.n && cc[j] - u - dv[j] == bestR[k]) ? j : e;
-    const int32_t ce = e == 0 ? cc[0] : e == 1 ? cc[1] : e == 2 ? cc[2] : cc[3];
-    const uint32_t col = 4 * c + (uint32_t)e;
-    mine.rc[k] = none ? -1 : (int32_t)((r << 16) | col);
-    mine.cost[k] = none ? 0 : ce;
-    const uint64_t kk = none ? kNoKey : pack_vi(bestR[k], r * (uint32_t)C.n + col);
-    key = kk < key ? kk : key;
+    for (int k = 0; k < K; ++k) cv[k] = *(const FLOCK_GLOBAL i32x4*)((gcbyte*)C.cost + 4 * (bestRow[k] * ld + col[k]));
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int32_t u = t.du[bestRow[k]];
+      const i32x4 vv = *(const i32x4*)(t.dv + col[k]);
+      const i32x4 c = cv[k];
+      const int e = c.x - vv.x - u == bestR[k] ? 0 : c.y - vv.y - u == bestR[k] ? 1 : c.z - vv.z - u == bestR[k] ? 2 : 3;
+      const uint32_t id = cell_id(bestRow[k], col[k] + (uint32_t)e);
+      mine.rc[k] = (int32_t)id;
+      mine.cost[k] = e == 0 ? c.x : e == 1 ? c.y : e == 2 ? c.z : c.w;
+      const uint64_t kk = pack_vi(bestR[k], id);
+      key = kk < key ? kk : key;
+    }
   }
   return group_min1_u64<G, 2>(key, S);
 }
@@ -1115,7 +1226,7 @@ __device__ __forceinline__ uint64_t reprice_set(const Ctx& C, const TreeLds& t, 
     const int row = rc < 0 ? 0 : (rc >> 16), col = rc < 0 ? 0 : (rc & 0xffff);
     const int32_t r = cs.cost[k] - t.du[row] - t.dv[col];
     // an empty slot ORs in all ones (kNoKey) instead of branching
-    const uint64_t kk = pack_vi(r, (uint32_t)row * (uint32_t)C.n + (uint32_t)col) | (rc < 0 ? kNoKey : 0ull);
+    const uint64_t kk = pack_vi(r, (uint32_t)rc) | (rc < 0 ? kNoKey : 0ull);
     key = kk < key ? kk : key;
   }
   return key;
@@ -1125,7 +1236,7 @@ __device__ __forceinline__ uint64_t reprice_set(const Ctx& C, const TreeLds& t, 
 __device__ __forceinline__ uint64_t reprice(const Ctx& C, const TreeLds& t, const Cand& c) {
   if (c.row < 0) return kNoKey;
   const int32_t r = c.cost - t.du[c.row] - t.dv[c.col];
-  return pack_vi(r, (uint32_t)c.row * (uint32_t)C.n + (uint32_t)c.col);
+  return pack_vi(r, cell_id((uint32_t)c.row, (uint32_t)c.col));
 }
 
 // ---------------------------------------------------------------------------
@@ -1162,7 +1273,10 @@ __device__ void sweep_tile(const SweepArgs& A, uint32_t tile, Shared& S) {
   const int m = A.m, n = A.n, nLast = A.n - 1;
   const uint32_t vpr = (uint32_t)A.ld >> 2;
   const uint32_t nvec = (uint32_t)m * vpr;
-  const uint64_t magic = (0x10000000000ull / vpr) + 1;  // exact quotient, as in sweep_argmin
+  // q / vpr as (q * magic) >> 40 with magic = floor(2^40 / vpr) + 1: the error term is
+  // below q / 2^40 < 2^-16 while the fractional part of q / vpr is at most
+  // 1 - 1/vpr, so the quotient is exact for q < 2^24 and vpr <= 2^11 (m*n <= 2^26).
+  const uint64_t magic = (0x10000000000ull / vpr) + 1;
   const uint32_t ld = (uint32_t)A.ld;
   const uint32_t v0 = tile * A.vpt;
   const uint32_t v1 = v0 + A.vpt < nvec ? v0 + A.vpt : nvec;
@@ -1218,7 +1332,7 @@ __device__ void sweep_tile(const SweepArgs& A, uint32_t tile, Shared& S) {
   }
   const int32_t ce = e == 0 ? cc[0] : e == 1 ? cc[1] : e == 2 ? cc[2] : cc[3];
   const uint32_t colb = 4 * cb + (uint32_t)e;
-  const uint64_t key = none ? kNoKey : pack_vi(bestR, rb * (uint32_t)n + colb);
+  const uint64_t key = none ? kNoKey : pack_vi(bestR, cell_id(rb, colb));
   // one candidate per 16-lane row of each wavefront (kTileCands per tile): the row's
   // least key by DPP row shifts lands in the row's lane 15
   uint64_t rk = key;
@@ -1588,7 +1702,7 @@ __device__ __attribute__((noinline)) int multi_pivot(const Ctx& C, const TreeLds
   const int m = C.m, V = C.V, tid = grank<G>();
   constexpr uint32_t kRange = (1u << 22) - 1;
   const int I = cand.row, J = m + cand.col;
-  const uint32_t mine = (uint32_t)cand.row * (uint32_t)C.n + (uint32_t)cand.col;
+  const uint32_t mine = cell_id((uint32_t)cand.row, (uint32_t)cand.col);
   bool spent = cand.row < 0;  // this rank's candidate has entered the basis
   int done = 0;
   for (int round = 0; round < rounds && iter + done < maxIt; ++round) {
@@ -1620,10 +1734,8 @@ __device__ __attribute__((noinline)) int multi_pivot(const Ctx& C, const TreeLds
     while (iter + done < maxIt) {
       const uint64_t k = group_min_u64<G>(accepted ? reprice(C, t, cand) : kNoKey, S);
       if (k == kNoKey || key_val(k) >= 0) break;
-      const uint32_t cell = key_idx(k);
-      if (accepted && cell == mine) { accepted = false; spent = true; }
-      const int ei = (int)(cell / (uint32_t)C.n), ej = (int)(cell - (uint32_t)ei * (uint32_t)C.n);
-      pivot<G>(C, t, sn, S, ei, ej, key_val(k));
+      if (accepted && key_idx(k) == mine) { accepted = false; spent = true; }
+      pivot<G>(C, t, sn, S, cell_row(k), cell_col(k), key_val(k));
       if (S.status != 0) return done;
       ++done; ++inRound;
     }
@@ -1699,9 +1811,11 @@ __device__ void write_outputs(const Ctx& C, const TreeLds& t, DevInstance& D, Sh
 // Solve (or advance) one instance with one group.  `region` is the group's LDS region
 // of `region_bytes` bytes, starting with its Shared block.
 // ---------------------------------------------------------------------------
-// kMulti: this instantiation carries the multi-pivot rule (kernels launched for it);
-// the others leave its code out, which keeps their register count down.
-template <int G, bool kMulti>
+// kRule: the pricing rule this instantiation carries (kernels are launched for one rule, so
+// each keeps only its own state in registers: one kernel for Dantzig and candidates kept
+// the candidate set alive through Dantzig's sweeps).
+enum { kRuleDantzig = 0, kRuleCandidates = 1, kRuleMulti = 2 };
+template <int G, int kRule>
 __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes, const EngineParams& P) {
   if (D.phase == 2) return;
   Shared& S = *(Shared*)region;
@@ -1726,6 +1840,7 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
   // 256- and 512-thread engines keep the pivot's snapshot in LDS only (one pivot code
   // path, fewer live registers); the host gives them only instances whose tree and
   // snapshot fit their LDS
+  constexpr bool kMulti = kRule == kRuleMulti, kCands = kRule == kRuleCandidates;
   constexpr bool kSnapLdsOnly = (G == 256 || G == 512) && !kMulti;
   if constexpr (kSnapLdsOnly) {
     if (!auxLds) {
@@ -1733,19 +1848,17 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
       return;
     }
   }
-  int64_t iter = D.iterations;
-  int64_t sweeps = D.sweeps;
-  int32_t mode = D.phase == 0 ? 0 : D.mode;  // switch rule: 1 once multi-pivoting stopped
+  const bool fresh = D.phase == 0;
+  int32_t mode = fresh ? 0 : uniform(D.mode);  // switch rule: 1 once multi-pivoting stopped
   const bool lead = grank<G>() == 0;
   if (lead) {
     S.status = 0;
-    for (int k = 0; k < 6; ++k) S.tk[k] = D.phase == 0 ? 0 : D.ticks[k];
-    if (D.phase == 0) D.t_start = now_ticks();
+    for (int k = 0; k < 6; ++k) S.tk[k] = fresh ? 0 : D.ticks[k];
+    if (fresh) D.t_start = now_ticks();
   }
   uint64_t tp = now_ticks();
   gsync<G>();
-  if (D.phase == 0) {
-    iter = 0; sweeps = 0;
+  if (fresh) {
     // Vogel and the tree build cannot stop at a slice deadline: count this group as busy
     // meanwhile (relaxed device-scope counter; it only decides when pivoting groups stop)
     if (P.busy && lead) __hip_atomic_fetch_add(P.busy, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1782,34 +1895,38 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
   }
   for (int j = n + grank<G>(); j < C.ld; j += G) t.dv[j] = 0;  // padding duals (published below)
   tree_index<G>(C, t, S);
+  // pivots still allowed (this call counts in 32 bits; D.iterations holds the earlier ones)
+  const int64_t iter0 = fresh ? 0 : D.iterations;
   const int64_t maxIt = P.max_iterations > 0 ? P.max_iterations : 50LL * V + 100000;
+  const int32_t budget = uniform((int32_t)(maxIt - iter0 < 0x7fffffff ? maxIt - iter0 : 0x7fffffff));
   int32_t status = 0;
   bool finished = false;
-  int64_t stepDone = 0;
-  constexpr int K = kMulti ? 1 : CandsPerRank<G>::value;
+  int32_t done = 0, sweeps = 0;  // pivots and full sweeps of this call
+  constexpr int K = kCands ? CandsPerRank<G>::value : 1;
   CandSet<K> cands;
   cands.clear();
+  const SweepShape shape = sweep_shape<G>(m, C.ld >> 2);
   int minor = 0;
   bool haveList = false;
   for (;;) {
     uint64_t key;
     tp = now_ticks();
-    if (P.pricing == 1 && haveList && minor < P.minor_limit) {
+    if (kCands && haveList && minor < P.minor_limit) {
       key = group_min1_u64<G, 0>(reprice_set(C, t, cands), S);
       if (lead) S.tk[3] += (int64_t)(now_ticks() - tp);
       if (key == kNoKey || key_val(key) >= 0) { haveList = false; continue; }
       ++minor;
     } else {
-      key = sweep_argmin<G, K>(C, t, S, cands);
+      key = sweep_argmin<G, K>(C, t, S, shape, cands);
       if (lead) S.tk[2] += (int64_t)(now_ticks() - tp);
       ++sweeps;
-      haveList = P.pricing == 1;
+      haveList = kCands;
       minor = 0;
       if (key == kNoKey || key_val(key) >= 0) { finished = true; break; }
     }
-    if (iter >= maxIt) { status = 1; finished = true; break; }
-    if (P.step_pivots > 0 && stepDone >= P.step_pivots) break;
-    if (P.deadline && stepDone > 0) {  // one decision for the whole group; >= 1 pivot per call
+    if (done >= budget) { status = 1; finished = true; break; }
+    if (P.step_pivots > 0 && done >= P.step_pivots) break;
+    if (P.deadline && done > 0) {  // one decision for the whole group; >= 1 pivot per call
       if (lead)
         S.stop = now_ticks() >= P.deadline &&
                  (!P.busy || __hip_atomic_load(P.busy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0);
@@ -1821,29 +1938,32 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
         // the switch rule makes one claim round per sweep and leaves multi-pivoting for
         // good once a round pivots fewer than 10 times (switch_model_parallel.cu:182-184)
         const bool sw = P.pricing == 4;
-        const int done = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cands.get(0), iter, maxIt,
+        const int made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cands.get(0), done, budget,
                                         sw ? 1 : P.minor_limit);
         if (S.status != 0) { status = S.status; finished = true; break; }
-        iter += done; stepDone += done;
-        if (sw && done < 10) mode = 1;
+        done = uniform(done + made);
+        if (sw && made < 10) mode = 1;
         continue;
       }
     }
-    const uint32_t cell = key_idx(key);
-    const int ei = (int)(cell / (uint32_t)n), ej = (int)(cell - (uint32_t)ei * (uint32_t)n);
+    const int ei = cell_row(key), ej = cell_col(key);
     if (kSnapLdsOnly || auxLds) pivot<G, (G < 1024)>(C, t, snL, S, ei, ej, key_val(key));
     else pivot<G, (G < 1024)>(C, t, sn, S, ei, ej, key_val(key));
     if (S.status != 0) { status = S.status; finished = true; break; }
-    ++iter; ++stepDone;
+    ++done;
   }
   if (finished) {
     write_outputs<G>(C, t, D, S);
-    if (grank<G>() == 0) { D.status = status; D.phase = 2; D.iterations = iter; D.sweeps = sweeps; D.mode = mode; }
   } else {
     save_state<G>(C, t, gl(uniform_ptr(D.state)));
-    if (grank<G>() == 0) { D.phase = 1; D.iterations = iter; D.sweeps = sweeps; D.mode = mode; }
   }
   if (lead) {
+    // a fresh instance's counters start at zero (the launch's reset cleared them)
+    if (finished) D.status = status;
+    D.phase = finished ? 2 : 1;
+    D.iterations = iter0 + done;
+    D.sweeps = (fresh ? 0 : D.sweeps) + sweeps;
+    D.mode = mode;
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
     if (finished) D.t_done = now_ticks();
   }
@@ -1988,9 +2108,8 @@ __device__ void large_round(DevInstance& D, char* region, size_t region_bytes, c
   // least once whatever tiles the ranks' candidates came from (the grid can have more
   // tiles than a rank per wavefront candidate)
   if ((P.pricing == 2 || P.pricing == 4) && tid == 0 && key != kNoKey && key_val(key) < 0) {
-    const uint32_t cell = key_idx(key);
-    cand.row = (int)(cell / (uint32_t)n);
-    cand.col = (int)(cell - (uint32_t)cand.row * (uint32_t)n);
+    cand.row = cell_row(key);
+    cand.col = cell_col(key);
     cand.cost = cost_at(C, cand.row, cand.col);
   }
   int64_t iter = D.iterations;
@@ -2016,8 +2135,7 @@ __device__ void large_round(DevInstance& D, char* region, size_t region_bytes, c
     int minor = 0;
     for (;;) {
       if (iter >= maxIt) { status = 1; finished = true; break; }
-      const uint32_t cell = key_idx(key);
-      const int ei = (int)(cell / (uint32_t)n), ej = (int)(cell - (uint32_t)ei * (uint32_t)n);
+      const int ei = cell_row(key), ej = cell_col(key);
       if (auxLds) pivot<G, true>(C, t, snL, S, ei, ej, key_val(key));
       else pivot<G, true>(C, t, sn, S, ei, ej, key_val(key));
       if (S.status != 0) { status = S.status; finished = true; break; }
@@ -2061,7 +2179,7 @@ __host__ __device__ inline SweepArgs sweep_args(const DevInstance& D, int V, uin
 // instance indices from `head` and solves them one after another.  With a slice
 // deadline no instance is started after it.
 // ---------------------------------------------------------------------------
-template <int T, int G, bool kMulti>
+template <int T, int G, int kRule>
 __device__ void queue_worker(DevInstance* insts, const int32_t* order, int32_t count, int32_t* head,
                              const EngineParams& P, char* smem) {
   const size_t region_bytes = (size_t)P.lds_bytes;
@@ -2081,12 +2199,13 @@ __device__ void queue_worker(DevInstance* insts, const int32_t* order, int32_t c
       idx = S.idx;
       __syncthreads();
     }
+    idx = uniform(idx);
     if (idx >= count) break;
     // the largest instances set the launch's makespan: their waves get issue priority
     // over co-resident workgroups' (uniform per group)
     if (idx < Q.prio_count) __builtin_amdgcn_s_setprio(3);
     else __builtin_amdgcn_s_setprio(0);
-    solve_instance<G, kMulti>(insts[order[idx]], region, region_bytes, Q);
+    solve_instance<G, kRule>(*uniform_ptr(insts + order[idx]), region, region_bytes, Q);
   }
 }
 

@@ -26,13 +26,13 @@ using namespace flock;
 // instance configurations of up to 512 threads are held to 168 VGPRs, i.e. three waves
 // per SIMD; the few values that spill are stored at kernel entry and reloaded once per
 // instance, outside the pivot loop.
-template <int T, int G, bool M>
-struct QueueWaves { static constexpr int value = (G == T && T <= 512 && !M) ? 3 : 1; };
-template <int T, int G, bool M>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(QueueWaves<T, G, M>::value))) void k_solve_queue(DevInstance* insts, const int32_t* order, int32_t count,
+template <int T, int G, int R>
+struct QueueWaves { static constexpr int value = (G == T && T <= 512 && R != kRuleMulti) ? 3 : 1; };
+template <int T, int G, int R>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(QueueWaves<T, G, R>::value))) void k_solve_queue(DevInstance* insts, const int32_t* order, int32_t count,
                                                    int32_t* head, EngineParams P) {
   extern __shared__ __align__(16) char smem[];
-  queue_worker<T, G, M>(insts, order, count, head, P, smem);
+  queue_worker<T, G, R>(insts, order, count, head, P, smem);
 }
 
 // Large-instance path (bodies in engine.h): setup and rounds run on one workgroup of
@@ -196,12 +196,13 @@ struct KernelCfg {
   int threads;  // workgroup size
   int group;    // threads per instance (64 = one wavefront per instance)
   int max_v;    // largest m+n the configuration accepts
-  const void* fn;        // Dantzig and candidate-list rules
-  const void* fn_multi;  // multi-pivot rule
+  const void* fn[3];  // by pricing rule: Dantzig, candidate list, multi-pivot
 };
 
 static const KernelCfg kCfgs[] = {
-#define FLOCK_CFG(T, G, MAXV) {T, G, MAXV, (const void*)k_solve_queue<T, G, false>, (const void*)k_solve_queue<T, G, true>}
+#define FLOCK_CFG(T, G, MAXV)                                                                                   \
+  {T, G, MAXV, {(const void*)k_solve_queue<T, G, kRuleDantzig>, (const void*)k_solve_queue<T, G, kRuleCandidates>, \
+                (const void*)k_solve_queue<T, G, kRuleMulti>}}
     FLOCK_CFG(256, 64, 2048),
     FLOCK_CFG(128, 64, 2048),
     FLOCK_CFG(64, 64, 2048),
@@ -297,7 +298,7 @@ int launch_queue_on(int cfg, DevInstance* d_insts, const int32_t* d_order, int32
   const int gpw = K.threads / K.group;
   const size_t lds = group_bytes * gpw;
   if (lds > g_lds_max) return set_error(FLOCK_E_TOO_LARGE, "LDS need %zu exceeds %zu", lds, g_lds_max);
-  const void* fn = (P.pricing == 2 || P.pricing == 4) ? K.fn_multi : K.fn;
+  const void* fn = K.fn[(P.pricing == 2 || P.pricing == 4) ? kRuleMulti : P.pricing == 1 ? kRuleCandidates : kRuleDantzig];
   if (lds > 65536) HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   int occ = 0;
   HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, K.threads, lds));

@@ -99,8 +99,9 @@ void run_group(DevInstance& D, char* region, size_t region_bytes, const EnginePa
     f->stack.resize(1 << 18);
     f->lane = emu::Lane{(unsigned)t, &block, waves[t / 64], xchg[t / 64].data()};
     f->body = [&D, region, region_bytes, &P] {
-      if (P.pricing == 2 || P.pricing == 4) solve_instance<G, true>(D, region, region_bytes, P);
-      else solve_instance<G, false>(D, region, region_bytes, P);
+      if (P.pricing == 2 || P.pricing == 4) solve_instance<G, kRuleMulti>(D, region, region_bytes, P);
+      else if (P.pricing == 1) solve_instance<G, kRuleCandidates>(D, region, region_bytes, P);
+      else solve_instance<G, kRuleDantzig>(D, region, region_bytes, P);
     };
     getcontext(&f->ctx);
     f->ctx.uc_stack.ss_sp = f->stack.data();
@@ -126,8 +127,9 @@ void run_group(DevInstance& D, char* region, size_t region_bytes, const EnginePa
   for (int t = 0; t < G; ++t) {
     th.emplace_back([&, t] {
       emu::lane_ctx = emu::Lane{(unsigned)t, &block, waves[t / 64], xchg[t / 64].data()};
-      if (P.pricing == 2 || P.pricing == 4) solve_instance<G, true>(D, region, region_bytes, P);
-      else solve_instance<G, false>(D, region, region_bytes, P);
+      if (P.pricing == 2 || P.pricing == 4) solve_instance<G, kRuleMulti>(D, region, region_bytes, P);
+      else if (P.pricing == 1) solve_instance<G, kRuleCandidates>(D, region, region_bytes, P);
+      else solve_instance<G, kRuleDantzig>(D, region, region_bytes, P);
     });
   }
   for (auto& x : th) x.join();
@@ -144,7 +146,7 @@ T* exact(size_t count) {
 
 // One launch of the persistent work-queue kernel: `wgs` workgroups of T lanes, all of
 // them running at the same time (fibers of one scheduler, or one OS thread per lane),
-// each executing the kernel body queue_worker<T, G, multi> with its own LDS block.
+// each executing the kernel body queue_worker<T, G, rule> with its own LDS block.
 template <int T, int G>
 void run_launch(DevInstance* insts, const int32_t* order, int32_t count, int32_t* head, const EngineParams& P,
                 int wgs, size_t lds_bytes) {
@@ -171,8 +173,9 @@ void run_launch(DevInstance* insts, const int32_t* order, int32_t count, int32_t
       f->lane = emu::Lane{(unsigned)t, g[b].block, g[b].waves[t / 64], g[b].xchg[t / 64].data()};
       char* smem = g[b].smem;
       f->body = [=, &P] {
-        if (P.pricing == 2 || P.pricing == 4) queue_worker<T, G, true>(insts, order, count, head, P, smem);
-        else queue_worker<T, G, false>(insts, order, count, head, P, smem);
+        if (P.pricing == 2 || P.pricing == 4) queue_worker<T, G, kRuleMulti>(insts, order, count, head, P, smem);
+        else if (P.pricing == 1) queue_worker<T, G, kRuleCandidates>(insts, order, count, head, P, smem);
+        else queue_worker<T, G, kRuleDantzig>(insts, order, count, head, P, smem);
       };
       getcontext(&f->ctx);
       f->ctx.uc_stack.ss_sp = f->stack.data();
@@ -190,8 +193,9 @@ void run_launch(DevInstance* insts, const int32_t* order, int32_t count, int32_t
     for (int t = 0; t < T; ++t)
       th.emplace_back([&, b, t] {
         emu::lane_ctx = emu::Lane{(unsigned)t, g[b].block, g[b].waves[t / 64], g[b].xchg[t / 64].data()};
-        if (P.pricing == 2 || P.pricing == 4) queue_worker<T, G, true>(insts, order, count, head, P, g[b].smem);
-        else queue_worker<T, G, false>(insts, order, count, head, P, g[b].smem);
+        if (P.pricing == 2 || P.pricing == 4) queue_worker<T, G, kRuleMulti>(insts, order, count, head, P, g[b].smem);
+        else if (P.pricing == 1) queue_worker<T, G, kRuleCandidates>(insts, order, count, head, P, g[b].smem);
+        else queue_worker<T, G, kRuleDantzig>(insts, order, count, head, P, g[b].smem);
       });
   for (auto& x : th) x.join();
 #endif

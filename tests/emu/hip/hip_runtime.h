@@ -158,6 +158,8 @@ namespace emu {
 void lane_yield();
 }
 #define __builtin_amdgcn_s_sleep(n) (emu::lane_yield())
+// instruction scheduling fence: nothing to order on the CPU
+#define __builtin_amdgcn_sched_barrier(m) ((void)0)
 // wave issue priority: no scheduling effect on the CPU
 #define __builtin_amdgcn_s_setprio(n) ((void)0)
 template <class T>

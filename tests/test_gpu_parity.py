@@ -189,6 +189,29 @@ def test_every_kernel_configuration_exact(threads, team):
             assert c.objective == o.objective and certify(inst, c)[0] == 0, pricing
 
 
+# (m, n) at the edges of a sweep block of kSlots * threads vectors (2048 at 256 threads,
+# 256 for a wavefront): one vector per row with one block, one row more or less; whole
+# blocks; a last block of one row; rows longer than a wavefront's block
+SWEEP_EDGES = {64: [(255, 3), (257, 4), (63, 16), (65, 16), (3, 1024), (4, 1025), (2, 1540)],
+               256: [(2047, 4), (2049, 3), (255, 32), (257, 30), (512, 32), (31, 260), (32, 258), (63, 260)],
+               512: [(511, 32), (513, 31), (62, 260), (63, 257)],
+               1024: [(1023, 32), (1025, 29), (127, 257)]}
+
+
+@pytest.mark.parametrize("threads", sorted(SWEEP_EDGES))
+def test_sweep_block_edges_exact(threads):
+    """The sweep's argmin and ties at block edges: the whole Dantzig sequence equals the
+    oracle's (integers, no tolerance); candidate pricing reaches the same objective."""
+    rng = np.random.default_rng(77 + threads)
+    for k, (m, n) in enumerate(SWEEP_EDGES[threads]):
+        inst = _rand(rng, m, n, cmax=(3, 50, 9000)[k % 3], zeros=n > 20 * m)
+        say("sweep edge", threads, m, n)
+        o = oracle.solve(inst.cost, inst.supply, inst.demand)
+        assert_same_as_oracle(inst, F.solve(inst, pricing="dantzig", threads=threads), o, exact_sequence=True)
+        c = F.solve(inst, pricing="candidates", threads=threads)
+        assert c.objective == o.objective and certify(inst, c)[0] == 0
+
+
 def test_batch_mixed_configurations():
     """One batch mixing wavefront and workgroup classes, candidates pricing."""
     rng = np.random.default_rng(8)
