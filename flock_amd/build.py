@@ -14,8 +14,9 @@ ROOT = os.path.dirname(HERE)
 LIB_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIB_DIR, "libflock_amd.so")
 CLI = os.path.join(LIB_DIR, "flock")
-SOURCES = ["csrc/runtime.hip", "csrc/server.hip", "csrc/uv_model.hip", "csrc/noalloc.hip"]
-HEADERS = ["csrc/device_common.h", "csrc/engine.h", "csrc/runtime_internal.h",
+SOURCES = ["csrc/queue_512.hip", "csrc/queue_1024.hip", "csrc/queue_256.hip", "csrc/queue_wave.hip",
+           "csrc/large.hip", "csrc/runtime.hip", "csrc/server.hip", "csrc/uv_model.hip", "csrc/noalloc.hip"]
+HEADERS = ["csrc/device_common.h", "csrc/engine.h", "csrc/kernels.h", "csrc/queue_kernel.h", "csrc/runtime_internal.h",
            "../include/flock_amd.h", "../include/flock/structs.h", "../include/flock/uv_model_parallel.h"]
 
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -47,7 +48,7 @@ def build(verbose: bool = False) -> str:
         r = subprocess.run(cmd, capture_output=True, text=True)
         return obj, r
 
-    with ThreadPoolExecutor(max_workers=min(4, len(srcs))) as pool:
+    with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as pool:
         results = list(pool.map(compile_one, srcs))
     for obj, r in results:
         if r.returncode != 0:

@@ -19,6 +19,10 @@
 //   y is an ancestor-or-self of x  <=>  pre[y] <= pre[x] < pre[y] + size[y].
 // That O(1) test is what makes cycle discovery and subtree identification
 // embarrassingly parallel over vertices.
+//
+// Every device function here is forced inline: an outlined one takes generic pointers, so
+// its LDS accesses become flat ones, and its caller keeps a stack (Vogel's register mode
+// outlined in the set-up kernel, for one).
 #pragma once
 #include "device_common.h"
 
@@ -170,7 +174,7 @@ __host__ __device__ inline size_t group_lds_bytes(int m, int n, size_t cap, bool
   return part;
 }
 
-__device__ inline TreeLds carve_tree(char* base, int m, int n) {
+__device__ __forceinline__ TreeLds carve_tree(char* base, int m, int n) {
   const int V = m + n;
   TreeLds t;
   size_t off = 0;
@@ -202,6 +206,7 @@ struct SnapT {
   __device__ __forceinline__ I32* ps(int k) const { return base + k * side + 2 * h; }
   __device__ __forceinline__ I32* flow(int k) const { return base + k * side + 2 * h + w; }
 };
+
 __device__ __forceinline__ int32_t pack_ps(int pre, int size) { return (int32_t)((uint32_t)(uint16_t)pre | ((uint32_t)size << 16)); }
 __device__ __forceinline__ int ps_pre(int32_t v) { return (int)((uint32_t)v & 0xffffu); }
 __device__ __forceinline__ int ps_size(int32_t v) { return (int)((uint32_t)v >> 16); }
@@ -210,7 +215,7 @@ __device__ __forceinline__ int ps_size(int32_t v) { return (int)((uint32_t)v >> 
 typedef SnapT<int32_t, int16_t> Snap;
 typedef SnapT<FLOCK_LDS int32_t, FLOCK_LDS int16_t> SnapL;
 template <class SN>
-__device__ inline SN carve_snap(int32_t* aux, int V) {
+__device__ __forceinline__ SN carve_snap(int32_t* aux, int V) {
   SN s;
   s.base = (decltype(s.base))aux;
   s.h = (V + 1) / 2 + 4;
@@ -240,7 +245,7 @@ __device__ __forceinline__ int32_t cost_at(const Ctx& C, int i, int j) { return 
 // order) and their latency overlaps tile k's LDS reads and stores.
 // ---------------------------------------------------------------------------
 template <int G>
-__device__ void transpose(const Ctx& C, int32_t* tile) {
+__device__ __forceinline__ void transpose(const Ctx& C, int32_t* tile) {
   const int rk = grank<G>();
   const int tx = rk % 64, ty = rk / 64;
   constexpr int R = G / 64;                // rows of a tile per pass of the group
@@ -294,6 +299,16 @@ __device__ void transpose(const Ctx& C, int32_t* tile) {
   load_chunk(0);
   unit(0);
   for (int q = 1; q < units; ++q) unit(q);
+}
+
+// Padding cells of every row (in the library's own copy of the matrix) price positive in
+// the sweeps, see kPadCost.
+template <int G>
+__device__ __forceinline__ void write_padding(const Ctx& C) {
+  const int padw = C.ld - C.n;
+  FLOCK_GLOBAL int32_t* cw = (FLOCK_GLOBAL int32_t*)C.cost;
+  if (padw > 0)
+    for (int e = grank<G>(); e < C.m * padw; e += G) cw[(uint32_t)((e / padw) * C.ld + C.n + e % padw)] = kPadCost;
 }
 
 // ---------------------------------------------------------------------------
@@ -417,7 +432,7 @@ __device__ __forceinline__ void wave_line_track(gcint* data, int len, const uint
 typedef const FLOCK_GLOBAL int16_t gcshort;
 
 template <int G>
-__device__ void line_book(const Ctx& C, int L, uint32_t* keys, FLOCK_GLOBAL int16_t* books) {
+__device__ __forceinline__ void line_book(const Ctx& C, int L, uint32_t* keys, FLOCK_GLOBAL int16_t* books) {
   const int m = C.m, n = C.n, tid = grank<G>();
   const bool row = L < m;
   gcint* data = row ? C.cost + (uint32_t)(L * C.ld) : C.costT + (uint32_t)((L - m) * C.ldT);
@@ -492,7 +507,7 @@ __host__ __device__ inline size_t vogel_trk_bytes(int m, int n) { return align16
 constexpr int kRegLines = 4;       // lines per rank of the work-queue engines
 constexpr int kRegLinesWide = 8;   // lines per rank of the large-instance set-up kernel
 template <int G, class TRK, int KL>
-__device__ void vogel_run(const Ctx& C, gcint* supply, gcint* demand, char* base, TRK* trk, Shared& S, gint* brow,
+__device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* demand, char* base, TRK* trk, Shared& S, gint* brow,
                           gint* bcol, gint* bflow, gcshort* books) {
   const int m = C.m, n = C.n, V = C.V, tid = grank<G>();
   const int lane = tid % kWave, wave = tid / kWave;
@@ -823,7 +838,7 @@ __device__ void vogel_run(const Ctx& C, gcint* supply, gcint* demand, char* base
 // large-instance set-up kernel, which has registers to spare), for m+n up to
 // kRegLinesWide * G, with the tracked keys in LDS or in global scratch.
 template <int G, bool kWide = false>
-__device__ void vogel(const Ctx& C, gcint* supply, gcint* demand, char* base, size_t avail, Shared& S, gint* brow,
+__device__ __forceinline__ void vogel(const Ctx& C, gcint* supply, gcint* demand, char* base, size_t avail, Shared& S, gint* brow,
                       gint* bcol, gint* bflow, int32_t* scratch, gcshort* books = nullptr, char* gstate = nullptr) {
   const size_t need = vogel_lds_bytes(C.m, C.n);
   const size_t needR = vogel_reg_lds_bytes(C.m, C.n);
@@ -859,7 +874,7 @@ __device__ void vogel(const Ctx& C, gcint* supply, gcint* demand, char* base, si
 // North-west corner rule (IBFS_nwc.cu:3-34; a tie moves to the next row, :17-23, except
 // on the last row).  Sequential, m+n-1 steps.
 template <int G>
-__device__ inline void nwc(const Ctx& C, gcint* supply, gcint* demand, gint* brow, gint* bcol, gint* bflow) {
+__device__ __forceinline__ void nwc(const Ctx& C, gcint* supply, gcint* demand, gint* brow, gint* bcol, gint* bflow) {
   if (grank<G>() != 0) return;
   int i = 0, j = 0;
   int64_t rs = supply[0], rd = demand[0];
@@ -887,7 +902,7 @@ __device__ __forceinline__ void set_dual(const TreeLds& t, int m, int x, int32_t
 // Returns false if the cells do not form a spanning tree.
 // ---------------------------------------------------------------------------
 template <int G>
-__device__ bool build_tree(const Ctx& C, gcint* brow, gcint* bcol, gcint* bflow, const TreeLds& t, int32_t* scr,
+__device__ __forceinline__ bool build_tree(const Ctx& C, gcint* brow, gcint* bcol, gcint* bflow, const TreeLds& t, int32_t* scr,
                            Shared& S) {
   const int m = C.m, V = C.V, tid = grank<G>();
   int32_t* start = scr;                    // V+1
@@ -1078,7 +1093,7 @@ struct SweepChunks { static constexpr bool value = SweepSlots<G>::value * G * 4 
 
 // shape: sweep_shape<G> of the whole row (used unless SweepChunks)
 template <int G, int K>
-__device__ uint64_t sweep_argmin(const Ctx& C, const TreeLds& t, Shared& S, const SweepShape& shape, CandSet<K>& mine) {
+__device__ __forceinline__ uint64_t sweep_argmin(const Ctx& C, const TreeLds& t, Shared& S, const SweepShape& shape, CandSet<K>& mine) {
   constexpr int kSlots = SweepSlots<G>::value;
   static_assert(K == 1 || K == kSlots, "one candidate per rank or one per slot");
   constexpr bool kChunks = SweepChunks<G>::value;
@@ -1241,21 +1256,22 @@ __device__ __forceinline__ uint64_t reprice(const Ctx& C, const TreeLds& t, cons
 
 // ---------------------------------------------------------------------------
 // One tile of a full sweep (the large-instance path's sweep grid): vectors [tile*vpt,
-// (tile+1)*vpt) of the padded matrix against the duals in global memory (u then v).
-// Writes the tile's argmin key (r, row-major index) to keys[tile] and, per wavefront,
-// its best cell (row, col, cost) to cands[3*(tile*W + wave)] (row -1: none).
+// (tile+1)*vpt) of the padded matrix against the duals of the saved tree (global memory).
+// Writes the tile's argmin key (r, cell) to keys[tile] and, per 16-lane row of its
+// wavefronts, the best cell (row, col, cost) to cands (row -1: none).
 // Everything comes from kernel arguments, so a rank issues its cost vectors, their row
-// duals, their four column duals and the phase word together (one round trip); as in
-// sweep_argmin, a vector is compared by its least reduced cost and the winning cell is
-// recovered once at the end.  When the phase word is not 1 (instance done) nothing is
-// written.
+// duals, their column duals (one aligned vector: the saved tree pads them like the rows)
+// and the phase word together (one round trip); as in sweep_argmin, a vector is compared
+// by its least reduced cost and the winning cell is recovered once at the end.  When the
+// phase word is not 1 (instance done) nothing is written.
 // ---------------------------------------------------------------------------
 // candidates a 256-thread sweep tile writes: one per 16-lane row of each wavefront
 constexpr int kTileCands = 16;
 struct MinU64Row { __device__ __forceinline__ uint64_t operator()(uint64_t a, uint64_t b) const { return b < a ? b : a; } };
 struct SweepArgs {
   const int32_t* cost;   // m x ld, padded rows
-  const int32_t* dual;   // m + n: u then v
+  const int32_t* du;     // the saved tree's duals
+  const int32_t* dv;     // 16-byte aligned, padded to ld with zeros
   const int32_t* phase;  // instance phase word
   uint64_t* keys;
   int32_t* cands;
@@ -1264,13 +1280,14 @@ struct SweepArgs {
 };
 
 template <int G>
-__device__ void sweep_tile(const SweepArgs& A, uint32_t tile, Shared& S) {
+__device__ __forceinline__ void sweep_tile(const SweepArgs& A, uint32_t tile, Shared& S) {
   const int tid = grank<G>(), lane = tid % kWave, wave = tid / kWave;
   static_assert(G / kWave * 4 == kTileCands, "a tile's candidates: four rows per wavefront");
   constexpr int U = 4;  // vectors in flight per rank
   gcint* cost = gl(A.cost);
-  gcint* dual = gl(A.dual);
-  const int m = A.m, n = A.n, nLast = A.n - 1;
+  gcint* du = gl(A.du);
+  gcint* dv = gl(A.dv);
+  const int m = A.m;
   const uint32_t vpr = (uint32_t)A.ld >> 2;
   const uint32_t nvec = (uint32_t)m * vpr;
   // q / vpr as (q * magic) >> 40 with magic = floor(2^40 / vpr) + 1: the error term is
@@ -1284,33 +1301,25 @@ __device__ void sweep_tile(const SweepArgs& A, uint32_t tile, Shared& S) {
   int32_t bestR = kBig;
   uint32_t bestQ = 0xffffffffu;
   for (uint32_t q0 = v0 + (uint32_t)tid; q0 < v1; q0 += U * G) {
-    i32x4 cv[U];
-    int32_t uu[U], vv[U][4];
-    uint32_t c4[U];
+    i32x4 cv[U], vv[U];
+    int32_t uu[U];
 #pragma unroll
     for (int k = 0; k < U; ++k) {
       const uint32_t q = q0 + (uint32_t)k * G;
-      const uint32_t qq = q < v1 ? q : v0;  // out-of-range slots re-read the tile's first vector
+      const uint32_t qq = q < v1 ? q : q0;  // slots past the tile repeat the rank's first vector
       const uint32_t r = (uint32_t)(((uint64_t)qq * magic) >> 40);
-      c4[k] = qq - r * vpr;
-      cv[k] = *(const FLOCK_GLOBAL i32x4*)(cost + (r * ld + 4 * c4[k]));
-      uu[k] = dual[r];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int j = 4 * (int)c4[k] + e;
-        vv[k][e] = dual[m + (j < nLast ? j : nLast)];
-      }
+      const uint32_t c4 = 4 * (qq - r * vpr);
+      cv[k] = *(const FLOCK_GLOBAL i32x4*)(cost + (r * ld + c4));
+      uu[k] = du[r];
+      vv[k] = *(const FLOCK_GLOBAL i32x4*)(dv + c4);
     }
 #pragma unroll
     for (int k = 0; k < U; ++k) {
       const uint32_t q = q0 + (uint32_t)k * G;
-      const int lim = q < v1 ? n - 4 * (int)c4[k] : 0;  // cells past the row end or the tile never win
-      const int32_t r0 = lim > 0 ? cv[k].x - uu[k] - vv[k][0] : kBig;
-      const int32_t r1 = lim > 1 ? cv[k].y - uu[k] - vv[k][1] : kBig;
-      const int32_t r2 = lim > 2 ? cv[k].z - uu[k] - vv[k][2] : kBig;
-      const int32_t r3 = lim > 3 ? cv[k].w - uu[k] - vv[k][3] : kBig;
-      const int32_t mn = imin(imin(r0, r1), imin(r2, r3));
-      const bool better = mn < bestR;
+      // padding cells price above every real cell of their vector (see sweep_argmin)
+      const int32_t mn =
+          imin(imin(cv[k].x - vv[k].x, cv[k].y - vv[k].y), imin(cv[k].z - vv[k].z, cv[k].w - vv[k].w)) - uu[k];
+      const bool better = mn < bestR;  // a repeated vector never is
       bestR = better ? mn : bestR;
       bestQ = better ? q : bestQ;
     }
@@ -1320,18 +1329,13 @@ __device__ void sweep_tile(const SweepArgs& A, uint32_t tile, Shared& S) {
   const bool none = bestQ == 0xffffffffu;
   const uint32_t qb = none ? v0 : bestQ;
   const uint32_t rb = (uint32_t)(((uint64_t)qb * magic) >> 40);
-  const uint32_t cb = qb - rb * vpr;
-  const i32x4 c = *(const FLOCK_GLOBAL i32x4*)(cost + (rb * ld + 4 * cb));
-  const int32_t ub = dual[rb];
-  const int32_t cc[4] = {c.x, c.y, c.z, c.w};
-  int e = 3;
-#pragma unroll
-  for (int j = 3; j >= 0; --j) {
-    const int col = 4 * (int)cb + j;
-    e = (col < n && cc[j] - ub - dual[m + (col < nLast ? col : nLast)] == bestR) ? j : e;
-  }
-  const int32_t ce = e == 0 ? cc[0] : e == 1 ? cc[1] : e == 2 ? cc[2] : cc[3];
-  const uint32_t colb = 4 * cb + (uint32_t)e;
+  const uint32_t cb = 4 * (qb - rb * vpr);
+  const i32x4 c = *(const FLOCK_GLOBAL i32x4*)(cost + (rb * ld + cb));
+  const int32_t ub = du[rb];
+  const i32x4 vb = *(const FLOCK_GLOBAL i32x4*)(dv + cb);
+  const int e = c.x - vb.x - ub == bestR ? 0 : c.y - vb.y - ub == bestR ? 1 : c.z - vb.z - ub == bestR ? 2 : 3;
+  const int32_t ce = e == 0 ? c.x : e == 1 ? c.y : e == 2 ? c.z : c.w;
+  const uint32_t colb = cb + (uint32_t)e;
   const uint64_t key = none ? kNoKey : pack_vi(bestR, cell_id(rb, colb));
   // one candidate per 16-lane row of each wavefront (kTileCands per tile): the row's
   // least key by DPP row shifts lands in the row's lane 15
@@ -1382,7 +1386,7 @@ __device__ void sweep_tile(const SweepArgs& A, uint32_t tile, Shared& S) {
 // four (the graph path's round kernel and the work-queue kernels below 1024 threads; the
 // 1024-thread work-queue kernel keeps kR, as it would spill more in its other phases).
 template <int G, int kR, class SN, bool kWideWin = false>
-__device__ void pivot_pass(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej, int32_t r) {
+__device__ __forceinline__ void pivot_pass(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej, int32_t r) {
   const int m = C.m, V = C.V, tid = grank<G>();
   const uint64_t t0 = now_ticks();
   const int I = ei, J = m + ej;
@@ -1696,9 +1700,9 @@ __device__ __forceinline__ void pivot(const Ctx& C, const TreeLds& t, const SN& 
 // `claim` needs V words (the pivot's snapshot region, free between pivots).  Returns
 // the pivots made; stops at the iteration budget.
 // ---------------------------------------------------------------------------
-template <int G>
-__device__ __attribute__((noinline)) int multi_pivot(const Ctx& C, const TreeLds& t, const Snap& sn, uint32_t* claim, Shared& S,
-                           const Cand& cand, int64_t iter, int64_t maxIt, int rounds) {
+template <int G, class SN>
+__device__ __forceinline__ int multi_pivot(const Ctx& C, const TreeLds& t, const SN& sn, uint32_t* claim,
+                                           Shared& S, const Cand& cand, int64_t iter, int64_t maxIt, int rounds) {
   const int m = C.m, V = C.V, tid = grank<G>();
   constexpr uint32_t kRange = (1u << 22) - 1;
   const int I = cand.row, J = m + cand.col;
@@ -1745,46 +1749,52 @@ __device__ __attribute__((noinline)) int multi_pivot(const Ctx& C, const TreeLds
 }
 
 // ---------------------------------------------------------------------------
-// Save / restore the tree between scheduling steps (server mode).
-// state layout (int32): parent, depth, pre, size, slot, flow, dual  (7 x V)
-// ---------------------------------------------------------------------------
-// Pivot set-up after the tree is built or loaded: vat (vertex at each pre-order
-// position) and the cycle-depth minima.
+// Pivot set-up after the tree is built or loaded: the cycle-depth minima, and (tree_index)
+// vat, the vertex at each pre-order position.
 template <int G>
-__device__ void tree_index(const Ctx& C, const TreeLds& t, Shared& S) {
-  for (int x = grank<G>(); x < C.V; x += G) t.vat[t.pre(x)] = (int16_t)x;
+__device__ __forceinline__ void pivot_init(Shared& S) {
   if (grank<G>() == 0) { S.dlo[0] = 0x7fffffff; S.dlo[1] = 0x7fffffff; S.dsel = 0; }
+}
+template <int G>
+__device__ __forceinline__ void tree_index(const Ctx& C, const TreeLds& t, Shared& S) {
+  for (int x = grank<G>(); x < C.V; x += G) t.vat[t.pre(x)] = (int16_t)x;
+  pivot_init<G>(S);
   gsync<G>();
 }
 
-template <int G>
-__device__ void save_state(const Ctx& C, const TreeLds& t, gint* st) {
-  const int V = C.V;
-  for (int x = grank<G>(); x < V; x += G) {
-    st[x] = t.parent[x]; st[V + x] = t.depth[x]; st[2 * V + x] = t.pre(x); st[3 * V + x] = t.size(x);
-    st[4 * V + x] = t.slot[x]; st[5 * V + x] = t.flow[x]; st[6 * V + x] = dual_of(t, C.m, x);
-  }
-}
-// Duals only, at the state's dual array (6V..7V), for the sweep grid (tree in global).
-template <int G>
-__device__ void save_duals(const Ctx& C, const TreeLds& t, gint* st) {
-  const int V = C.V;
-  for (int x = grank<G>(); x < V; x += G) st[6 * V + x] = dual_of(t, C.m, x);
+// The saved tree (server slices, graph-path rounds) is the LDS tree region as it is,
+// copied in 16-byte vectors: 20 bytes per vertex and no conversion.  (Seven int32 arrays
+// took 28 bytes, a scalar load and a 16-bit store per field and vertex, and a pass to
+// rebuild vat.)  A state buffer also holds Vogel's line state when that does not fit LDS.
+__host__ __device__ inline size_t state_bytes(int m, int n) {
+  const size_t a = tree_lds_bytes(m, n), b = vogel_lds_bytes(m, n);
+  return a > b ? a : b;
 }
 template <int G>
-__device__ void load_state(const Ctx& C, const TreeLds& t, gcint* st) {
-  const int V = C.V;
-  for (int x = grank<G>(); x < V; x += G) {
-    t.parent[x] = (int16_t)st[x]; t.depth[x] = (int16_t)st[V + x]; t.pre(x) = (int16_t)st[2 * V + x];
-    t.size(x) = (int16_t)st[3 * V + x]; t.slot[x] = (int16_t)st[4 * V + x]; t.flow[x] = st[5 * V + x];
-    set_dual(t, C.m, x, st[6 * V + x]);
+__device__ __forceinline__ void save_state(const char* tree, size_t bytes, gint* st) {
+  const int nv = (int)(bytes / 16);
+  FLOCK_GLOBAL i32x4* o = (FLOCK_GLOBAL i32x4*)st;
+  for (int k = grank<G>(); k < nv; k += G) o[k] = ((const FLOCK_LDS i32x4*)tree)[k];
+}
+// (the caller's next barrier publishes the tree)
+template <int G>
+__device__ __forceinline__ void load_state(char* tree, size_t bytes, gcint* st) {
+  const int nv = (int)(bytes / 16), tid = grank<G>();
+  const FLOCK_GLOBAL i32x4* in = (const FLOCK_GLOBAL i32x4*)st;
+  constexpr int U = 4;  // loads in flight
+  for (int k0 = tid; k0 < nv; k0 += U * G) {
+    i32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = in[k0 + u * G < nv ? k0 + u * G : k0];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k0 + u * G < nv) ((FLOCK_LDS i32x4*)tree)[k0 + u * G] = v[u];
   }
-  gsync<G>();
 }
 
 // Final outputs: basis by slot, duals, objective, count of positive flows.
 template <int G>
-__device__ void write_outputs(const Ctx& C, const TreeLds& t, DevInstance& D, Shared& S) {
+__device__ __forceinline__ void write_outputs(const Ctx& C, const TreeLds& t, DevInstance& D, Shared& S) {
   const int m = C.m, V = C.V;
   gint* dual = gl(uniform_ptr(D.dual));
   gint* brow = gl(uniform_ptr(D.basis_row));
@@ -1816,7 +1826,7 @@ __device__ void write_outputs(const Ctx& C, const TreeLds& t, DevInstance& D, Sh
 // the candidate set alive through Dantzig's sweeps).
 enum { kRuleDantzig = 0, kRuleCandidates = 1, kRuleMulti = 2 };
 template <int G, int kRule>
-__device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes, const EngineParams& P) {
+__device__ __forceinline__ void solve_instance(DevInstance& D, char* region, size_t region_bytes, const EngineParams& P) {
   if (D.phase == 2) return;
   Shared& S = *(Shared*)region;
   char* smem = region + shared_bytes();
@@ -1832,22 +1842,21 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
   const int m = C.m, n = C.n, V = C.V;
   const TreeLds t = carve_tree(smem, m, n);
   const size_t treeBytes = tree_lds_bytes(m, n);
-  int32_t* aux = (treeBytes + 4 * aux_ints(m, n) <= avail) ? (int32_t*)(smem + treeBytes)
-                                                          : uniform_ptr(D.scratch);
   const bool auxLds = treeBytes + 4 * aux_ints(m, n) <= avail;
-  const Snap sn = carve_snap<Snap>(aux, V);
-  const SnapL snL = carve_snap<SnapL>(aux, V);
   // 256- and 512-thread engines keep the pivot's snapshot in LDS only (one pivot code
   // path, fewer live registers); the host gives them only instances whose tree and
   // snapshot fit their LDS
   constexpr bool kMulti = kRule == kRuleMulti, kCands = kRule == kRuleCandidates;
-  constexpr bool kSnapLdsOnly = (G == 256 || G == 512) && !kMulti;
+  constexpr bool kSnapLdsOnly = G == 256 || G == 512;
   if constexpr (kSnapLdsOnly) {
     if (!auxLds) {
       if (grank<G>() == 0) { D.status = 6; D.phase = 2; D.iterations = 0; }
       return;
     }
   }
+  int32_t* aux = kSnapLdsOnly || auxLds ? (int32_t*)(smem + treeBytes) : uniform_ptr(D.scratch);
+  const Snap sn = carve_snap<Snap>(aux, V);
+  const SnapL snL = carve_snap<SnapL>(aux, V);
   const bool fresh = D.phase == 0;
   int32_t mode = fresh ? 0 : uniform(D.mode);  // switch rule: 1 once multi-pivoting stopped
   const bool lead = grank<G>() == 0;
@@ -1862,18 +1871,14 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
     // Vogel and the tree build cannot stop at a slice deadline: count this group as busy
     // meanwhile (relaxed device-scope counter; it only decides when pivoting groups stop)
     if (P.busy && lead) __hip_atomic_fetch_add(P.busy, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (C.ld > n) {  // padding cells of every row price positive in the sweep (kPadCost)
-      const int padw = C.ld - n;
-      FLOCK_GLOBAL int32_t* cw = (FLOCK_GLOBAL int32_t*)C.cost;  // the library's own copy
-      for (int e = grank<G>(); e < m * padw; e += G) cw[(uint32_t)((e / padw) * C.ld + n + e % padw)] = kPadCost;
-    }
+    write_padding<G>(C);
     if (P.initial == 1) {
       nwc<G>(C, supply, demand, brow, bcol, bflow);
     } else {
       transpose<G>(C, (int32_t*)smem);
       __threadfence_block();
       gsync<G>();
-      vogel<G>(C, supply, demand, smem, avail, S, brow, bcol, bflow, uniform_ptr(D.scratch));
+      vogel<G, G == 512>(C, supply, demand, smem, avail, S, brow, bcol, bflow, uniform_ptr(D.scratch));
     }
     __threadfence_block();
     gsync<G>();
@@ -1891,10 +1896,16 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
       return;
     }
   } else {
-    load_state<G>(C, t, gl(uniform_ptr(D.state)));
+    load_state<G>(smem, treeBytes, gl(uniform_ptr(D.state)));
   }
-  for (int j = n + grank<G>(); j < C.ld; j += G) t.dv[j] = 0;  // padding duals (published below)
-  tree_index<G>(C, t, S);
+  // padding duals, 0 in a saved tree already (published below)
+  if (fresh) {
+    for (int j = n + grank<G>(); j < C.ld; j += G) t.dv[j] = 0;
+    tree_index<G>(C, t, S);
+  } else {
+    pivot_init<G>(S);
+    gsync<G>();
+  }
   // pivots still allowed (this call counts in 32 bits; D.iterations holds the earlier ones)
   const int64_t iter0 = fresh ? 0 : D.iterations;
   const int64_t maxIt = P.max_iterations > 0 ? P.max_iterations : 50LL * V + 100000;
@@ -1938,8 +1949,11 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
         // the switch rule makes one claim round per sweep and leaves multi-pivoting for
         // good once a round pivots fewer than 10 times (switch_model_parallel.cu:182-184)
         const bool sw = P.pricing == 4;
-        const int made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cands.get(0), done, budget,
-                                        sw ? 1 : P.minor_limit);
+        int made;
+        if constexpr (kSnapLdsOnly)
+          made = multi_pivot<G>(C, t, snL, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit);
+        else
+          made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit);
         if (S.status != 0) { status = S.status; finished = true; break; }
         done = uniform(done + made);
         if (sw && made < 10) mode = 1;
@@ -1955,7 +1969,7 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
   if (finished) {
     write_outputs<G>(C, t, D, S);
   } else {
-    save_state<G>(C, t, gl(uniform_ptr(D.state)));
+    save_state<G>(smem, treeBytes, gl(uniform_ptr(D.state)));
   }
   if (lead) {
     // a fresh instance's counters start at zero (the launch's reset cleared them)
@@ -1982,7 +1996,7 @@ __device__ void solve_instance(DevInstance& D, char* region, size_t region_bytes
 // D.phase is 1 while the loop runs and 2 when done; later kernels return at once.
 // ---------------------------------------------------------------------------
 template <int G>
-__device__ void large_setup(DevInstance& D, char* region, size_t region_bytes, const EngineParams& P,
+__device__ __forceinline__ void large_setup(DevInstance& D, char* region, size_t region_bytes, const EngineParams& P,
                             gcshort* books) {
   Shared& S = *(Shared*)region;
   char* smem = region + shared_bytes();
@@ -2027,12 +2041,11 @@ __device__ void large_setup(DevInstance& D, char* region, size_t region_bytes, c
   if (ok) ok = build_tree<G>(C, brow, bcol, bflow, t, aux, S);
   { const uint64_t t2 = now_ticks(); if (lead) S.tk[1] += (int64_t)(t2 - tp); tp = t2; }
   if (ok) {
-    if (treeGlobal) {  // the tree stays where it is; the sweep grid reads the duals
-      tree_index<G>(C, t, S);
-      save_duals<G>(C, t, gl(uniform_ptr(D.state)));
-    } else {
-      save_state<G>(C, t, gl(uniform_ptr(D.state)));
-    }
+    write_padding<G>(C);
+    for (int j = C.n + grank<G>(); j < C.ld; j += G) t.dv[j] = 0;  // padding duals
+    tree_index<G>(C, t, S);
+    // a tree in global memory stays where it is; the sweep grid reads its duals there
+    if (!treeGlobal) save_state<G>(smem, treeBytes, gl(uniform_ptr(D.state)));
   }
   if (lead) {
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
@@ -2042,36 +2055,40 @@ __device__ void large_setup(DevInstance& D, char* region, size_t region_bytes, c
   }
 }
 
-template <int G, bool kMulti>
-__device__ void large_round(DevInstance& D, char* region, size_t region_bytes, const EngineParams& P,
-                            const uint64_t* keys, const int32_t* cands, int nblocks) {
-  if (D.phase != 1) return;
+// geo: the instance's sizes and buffers (a copy in the kernel's arguments, so that its first
+// loads do not wait for the descriptor's); D: the descriptor in memory.
+// kTreeGlobal: the tree lives in the state buffer (see large_setup).  With the choice made
+// at run time every access to the tree was a flat one: at 1000x1000 a pivot's cycle pass
+// took 1.9 us instead of 1.2.
+template <int G, int kRule, bool kTreeGlobal>
+__device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& geo, char* region, size_t region_bytes,
+                            const EngineParams& P, const uint64_t* keys, const int32_t* cands, int nblocks) {
+  constexpr bool kMulti = kRule == kRuleMulti, kCands = kRule == kRuleCandidates;
   Shared& S = *(Shared*)region;
   char* smem = region + shared_bytes();
   const size_t avail = region_bytes - shared_bytes();
   Ctx C;
-  C.cost = gl(uniform_ptr(D.cost)); C.costT = gl(uniform_ptr(D.costT));
-  C.m = uniform(D.m); C.n = uniform(D.n); C.V = C.m + C.n; C.ld = uniform(D.ld); C.ldT = uniform(D.ldT);
-  const int n = C.n, tid = grank<G>();
-  const bool treeGlobal = P.tree_global != 0;  // see large_setup
-  const TreeLds t = carve_tree(treeGlobal ? (char*)uniform_ptr(D.state) : smem, C.m, n);
-  const size_t treeBytes = tree_lds_bytes(C.m, n);
-  const bool auxLds = !treeGlobal && treeBytes + 4 * aux_ints(C.m, C.n) <= avail;
-  int32_t* aux = auxLds ? (int32_t*)(smem + treeBytes) : uniform_ptr(D.scratch);
+  C.cost = gl(geo.cost); C.costT = gl(geo.costT);
+  C.m = geo.m; C.n = geo.n; C.V = C.m + C.n; C.ld = geo.ld; C.ldT = geo.ldT;
+  const int tid = grank<G>();
+  const TreeLds t = carve_tree(kTreeGlobal ? (char*)geo.state : smem, C.m, C.n);
+  const size_t treeBytes = tree_lds_bytes(C.m, C.n);
+  const bool auxLds = !kTreeGlobal && treeBytes + 4 * aux_ints(C.m, C.n) <= avail;
+  int32_t* aux = auxLds ? (int32_t*)(smem + treeBytes) : geo.scratch;
   const Snap sn = carve_snap<Snap>(aux, C.V);
   const SnapL snL = carve_snap<SnapL>(aux, C.V);
   const bool lead = tid == 0;
+  // the phase is tested after the tree's loads are under way: a finished instance's rounds
+  // load it for nothing, the others save a memory round trip
+  const int32_t phase = D.phase;
+  if constexpr (!kTreeGlobal) load_state<G>(smem, treeBytes, gl((const int32_t*)geo.state));
+  if (phase != 1) return;
   if (lead) {
     S.status = 0;
     for (int k = 0; k < 6; ++k) S.tk[k] = D.ticks[k];
   }
-  if (treeGlobal) {  // the tree (vat included) persists in global memory between rounds
-    if (tid == 0) { S.dlo[0] = 0x7fffffff; S.dlo[1] = 0x7fffffff; S.dsel = 0; }
-    gsync<G>();
-  } else {
-    load_state<G>(C, t, gl(uniform_ptr(D.state)));
-    tree_index<G>(C, t, S);
-  }
+  pivot_init<G>(S);
+  gsync<G>();
   uint64_t key = kNoKey;
   for (int b = tid; b < nblocks; b += G) { const uint64_t k = keys[b]; key = k < key ? k : key; }
   key = group_min_u64<G>(key, S);
@@ -2084,7 +2101,7 @@ __device__ void large_round(DevInstance& D, char* region, size_t region_bytes, c
   cs.clear();
   Cand cand;
   cand.row = -1; cand.col = 0; cand.cost = 0;
-  if (P.pricing >= 1) {
+  if constexpr (kRule != kRuleDantzig) {
     uint64_t bestk[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) bestk[k] = kNoKey;
@@ -2107,7 +2124,7 @@ __device__ void large_round(DevInstance& D, char* region, size_t region_bytes, c
   // multi-pivot rules: rank 0 holds the sweep's argmin cell, so every round pivots at
   // least once whatever tiles the ranks' candidates came from (the grid can have more
   // tiles than a rank per wavefront candidate)
-  if ((P.pricing == 2 || P.pricing == 4) && tid == 0 && key != kNoKey && key_val(key) < 0) {
+  if (kMulti && tid == 0 && key != kNoKey && key_val(key) < 0) {
     cand.row = cell_row(key);
     cand.col = cell_col(key);
     cand.cost = cost_at(C, cand.row, cand.col);
@@ -2140,7 +2157,7 @@ __device__ void large_round(DevInstance& D, char* region, size_t region_bytes, c
       else pivot<G, true>(C, t, sn, S, ei, ej, key_val(key));
       if (S.status != 0) { status = S.status; finished = true; break; }
       ++iter;
-      if (P.pricing != 1 || ++minor >= P.minor_limit) break;  // Dantzig: one pivot per sweep
+      if (!kCands || ++minor >= P.minor_limit) break;  // Dantzig: one pivot per sweep
       const uint64_t tp = now_ticks();
       key = group_min1_u64<G, 0>(reprice_set(C, t, cs), S);
       if (lead) S.tk[3] += (int64_t)(now_ticks() - tp);
@@ -2149,11 +2166,9 @@ __device__ void large_round(DevInstance& D, char* region, size_t region_bytes, c
   }
   if (finished) {
     write_outputs<G>(C, t, D, S);
-  } else if (treeGlobal) {
-    gsync<G>();  // the last pivot's tree writes before the duals are read back
-    save_duals<G>(C, t, gl(uniform_ptr(D.state)));
-  } else {
-    save_state<G>(C, t, gl(uniform_ptr(D.state)));
+  } else if constexpr (!kTreeGlobal) {
+    gsync<G>();  // the last pivot's vat writes
+    save_state<G>(smem, treeBytes, gl(geo.state));
   }
   if (lead) {
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
@@ -2164,11 +2179,14 @@ __device__ void large_round(DevInstance& D, char* region, size_t region_bytes, c
   }
 }
 
-// Arguments of the sweep grid for instance D (duals at its state's dual array).
-__host__ __device__ inline SweepArgs sweep_args(const DevInstance& D, int V, uint64_t* keys, int32_t* cands,
-                                                uint32_t vpt, const int32_t* phase) {
+// Arguments of the sweep grid for instance D (duals of the tree in its state buffer).
+__host__ __device__ inline SweepArgs sweep_args(const DevInstance& D, uint64_t* keys, int32_t* cands, uint32_t vpt,
+                                                const int32_t* phase) {
   SweepArgs A;
-  A.cost = D.cost; A.dual = D.state + 6 * (size_t)V; A.phase = phase; A.keys = keys; A.cands = cands;
+  const size_t rows = align16(4 * (size_t)((D.m + 3) & ~3)), cols = align16(4 * (size_t)((D.n + 3) & ~3));
+  const char* end = (const char*)D.state + tree_lds_bytes(D.m, D.n);  // u and v are the last arrays
+  A.cost = D.cost; A.du = (const int32_t*)(end - cols - rows); A.dv = (const int32_t*)(end - cols);
+  A.phase = phase; A.keys = keys; A.cands = cands;
   A.m = D.m; A.n = D.n; A.ld = D.ld; A.vpt = vpt;
   return A;
 }
@@ -2180,7 +2198,7 @@ __host__ __device__ inline SweepArgs sweep_args(const DevInstance& D, int V, uin
 // deadline no instance is started after it.
 // ---------------------------------------------------------------------------
 template <int T, int G, int kRule>
-__device__ void queue_worker(DevInstance* insts, const int32_t* order, int32_t count, int32_t* head,
+__device__ __forceinline__ void queue_worker(DevInstance* insts, const int32_t* order, int32_t count, int32_t* head,
                              const EngineParams& P, char* smem) {
   const size_t region_bytes = (size_t)P.lds_bytes;
   char* region = smem + (size_t)(threadIdx.x / G) * region_bytes;

@@ -14,7 +14,7 @@
 #include <vector>
 
 #include "../../include/flock_amd.h"
-#include "engine.h"
+#include "kernels.h"
 #include "runtime_internal.h"
 
 using namespace flock;
@@ -22,66 +22,8 @@ using namespace flock;
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-// Persistent work-queue kernel (body: queue_worker in engine.h).  The workgroup-per-
-// instance configurations of up to 512 threads are held to 168 VGPRs, i.e. three waves
-// per SIMD; the few values that spill are stored at kernel entry and reloaded once per
-// instance, outside the pivot loop.
-template <int T, int G, int R>
-struct QueueWaves { static constexpr int value = (G == T && T <= 512 && R != kRuleMulti) ? 3 : 1; };
-template <int T, int G, int R>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(QueueWaves<T, G, R>::value))) void k_solve_queue(DevInstance* insts, const int32_t* order, int32_t count,
-                                                   int32_t* head, EngineParams P) {
-  extern __shared__ __align__(16) char smem[];
-  queue_worker<T, G, R>(insts, order, count, head, P, smem);
-}
-
-// Large-instance path (bodies in engine.h): setup and rounds run on one workgroup of
-// T = 512 or 1024 threads, the sweep on a grid of 256-thread workgroups, one matrix tile
-// each.
-template <int T>
-__global__ __launch_bounds__(T) void k_large_setup(DevInstance* insts, const int16_t* books, EngineParams P) {
-  extern __shared__ __align__(16) char smem[];
-  large_setup<T>(insts[0], smem, (size_t)P.lds_bytes, P, gl(books));
-}
-// Transpose of the cost matrix, one 64x64 tile per workgroup staged through LDS.
-__global__ __launch_bounds__(256) void k_large_transpose(const DevInstance* insts) {
-  __shared__ int32_t tile[64 * 65];
-  const DevInstance& D = insts[0];
-  const int m = D.m, n = D.n, ld = D.ld, ldT = D.ldT;
-  const int32_t* cost = D.cost;
-  int32_t* costT = D.costT;
-  const int bi = (int)blockIdx.y * 64, bj = (int)blockIdx.x * 64;
-  const int tx = (int)threadIdx.x % 64, ty = (int)threadIdx.x / 64;
-  for (int r = ty; r < 64; r += 4) {
-    const int i = bi + r, j = bj + tx;
-    tile[r * 65 + tx] = (i < m && j < n) ? cost[(size_t)i * ld + j] : 0;
-  }
-  __syncthreads();
-  for (int r = ty; r < 64; r += 4) {
-    const int j = bj + r, i = bi + tx;
-    if (j < n && i < m) costT[(size_t)j * ldT + i] = tile[tx * 65 + r];
-  }
-}
-// Vogel books: one workgroup sorts one line (rows, then columns).
-__global__ __launch_bounds__(256) void k_large_books(const DevInstance* insts, int16_t* books) {
-  __shared__ uint32_t keys[16384];  // a line of up to 16384 entries (m+n <= 16383)
-  const DevInstance& D = insts[0];
-  Ctx C;
-  C.cost = gl(uniform_ptr(D.cost)); C.costT = gl(uniform_ptr(D.costT));
-  C.m = uniform(D.m); C.n = uniform(D.n); C.V = C.m + C.n; C.ld = uniform(D.ld); C.ldT = uniform(D.ldT);
-  line_book<256>(C, (int)blockIdx.x, keys, gl(books));
-}
-template <int T, bool M>
-__global__ __launch_bounds__(T) void k_large_round(DevInstance* insts, const uint64_t* keys, const int32_t* cands,
-                                                   int32_t nblocks, EngineParams P) {
-  extern __shared__ __align__(16) char smem[];
-  large_round<T, M>(insts[0], smem, (size_t)P.lds_bytes, P, keys, cands, nblocks);
-}
-__global__ __launch_bounds__(256) void k_large_sweep(SweepArgs A) {
-  __shared__ Shared S;
-  sweep_tile<256>(A, blockIdx.x, S);
-}
-
+// The work-queue kernels and the large-instance path's kernels are compiled in their own
+// files (queue_*.hip, large.hip); kernels.h declares them.
 // The launch-to-completion floor of a grid: the same grid as the sweep, no work.
 __global__ __launch_bounds__(256) void k_empty_grid() {}
 
@@ -196,13 +138,11 @@ struct KernelCfg {
   int threads;  // workgroup size
   int group;    // threads per instance (64 = one wavefront per instance)
   int max_v;    // largest m+n the configuration accepts
-  const void* fn[3];  // by pricing rule: Dantzig, candidate list, multi-pivot
+  const void* const* fn;  // by pricing rule: Dantzig, candidate list, multi-pivot
 };
 
 static const KernelCfg kCfgs[] = {
-#define FLOCK_CFG(T, G, MAXV)                                                                                   \
-  {T, G, MAXV, {(const void*)k_solve_queue<T, G, kRuleDantzig>, (const void*)k_solve_queue<T, G, kRuleCandidates>, \
-                (const void*)k_solve_queue<T, G, kRuleMulti>}}
+#define FLOCK_CFG(T, G, MAXV) {T, G, MAXV, queue_kernels_##T##_##G}
     FLOCK_CFG(256, 64, 2048),
     FLOCK_CFG(128, 64, 2048),
     FLOCK_CFG(64, 64, 2048),
@@ -215,7 +155,11 @@ constexpr int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
 
 // size-class policy (tuned on MI355X; see autotune): instances with m+n up to
 // g_wave_max_v get one wavefront each, packed g_wave_pack per workgroup; larger ones
-// get a whole workgroup of 256 threads up to g_wg256_max_v, else 1024 threads.
+// get a whole workgroup of 256 threads up to g_wg256_max_v, else 512 threads while the tree
+// and the pivot's snapshot fit LDS (m+n up to about 3600), else 1024.  A workgroup of 1024
+// loses at every size that 512 can take: its barriers cost 144 cycles instead of 48 and
+// four waves share each SIMD (61x1203 dantzig 8.4 against 6.2 ms, 100x2400 candidates 15.7
+// against 13.3 ms, 1800x1700 candidates 100 against 92 ms).
 static int g_wave_max_v = 0;
 static int g_wave_pack = 4;
 static int g_wg256_max_v = 2000;
@@ -228,10 +172,22 @@ static int g_prio_permille = 0;
 static int g_sweep_vectors = 4;
 static int g_large_threads = 512;  // large-instance setup / round workgroup (512 or 1024)
 static int g_large_minor_limit = 64;  // large-instance path's candidate minor limit (0: g_minor_limit)
+// launches of at most one instance per compute unit: 256 threads up to the first, 512 up to
+// the second (where they fit LDS), else 1024
 static int g_few_256_max_v = 256;
-static int g_few_512_max_v = 1000;
-// plain solves of matrices with at least this many cells take the graph path
+static int g_few_512_max_v = kMaxVertices;
+// plain solves of matrices with at least this many cells take the graph path; with
+// candidate pricing, where a sweep serves tens of pivots, at least kCandGraphFactor times
+// as many if the 512-thread engine can take them (device ms, engine against graph path:
+// dantzig 420x430 15.3 / 15.1, 500x500 18.9 / 16.3; candidates 800x800 17.8 / 19.8, 1000x1000
+// 28.4 / 28.0, 1300x1300 49.4 / 46.5, 1800x1700 92 / 72)
 static int g_graph_min_cells = 250000;
+constexpr int kCandGraphFactor = 4;
+
+// the kernels' pricing rule (the switch rule starts with multi-pivot rounds)
+static int rule_of(const EngineParams& P) {
+  return (P.pricing == 2 || P.pricing == 4) ? kRuleMulti : P.pricing == 1 ? kRuleCandidates : kRuleDantzig;
+}
 
 int num_cfgs() { return kNumCfgs; }
 
@@ -281,7 +237,7 @@ static int pick_cfg_raw(int m, int n, const flock_options* opt, int64_t count) {
   if (threads == 512) return 4;
   if (threads == 1024) return 5;
   if (count <= g_cus) return V <= g_few_256_max_v ? 3 : (V <= g_few_512_max_v ? 4 : 5);
-  return V <= g_wg256_max_v ? 3 : 5;
+  return V <= g_wg256_max_v ? 3 : 4;
 }
 
 size_t cfg_group_bytes(int cfg, int m, int n, bool* aux_in_lds) {
@@ -298,7 +254,7 @@ int launch_queue_on(int cfg, DevInstance* d_insts, const int32_t* d_order, int32
   const int gpw = K.threads / K.group;
   const size_t lds = group_bytes * gpw;
   if (lds > g_lds_max) return set_error(FLOCK_E_TOO_LARGE, "LDS need %zu exceeds %zu", lds, g_lds_max);
-  const void* fn = K.fn[(P.pricing == 2 || P.pricing == 4) ? kRuleMulti : P.pricing == 1 ? kRuleCandidates : kRuleDantzig];
+  const void* fn = K.fn[rule_of(P)];
   if (lds > 65536) HIP_TRY(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   int occ = 0;
   HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, K.threads, lds));
@@ -365,7 +321,7 @@ int Batch::layout(int32_t count, const flock_instance* inst, bool with_state) {
     o.bflow = off; off += al(4 * (size_t)V);
     o.dual = off; off += al(4 * (size_t)V);
     o.scratch = off; off += al(4 * aux_ints(m, nn));
-    o.state = with_state ? off : 0; if (with_state) off += al(4 * 7 * (size_t)V);
+    o.state = with_state ? off : 0; if (with_state) off += al(state_bytes(m, nn));
     o.books = with_state ? off : 0; if (with_state) off += al(4 * (size_t)m * nn);
   }
   bytes = off;
@@ -574,7 +530,14 @@ struct LargeRunner {
     return FLOCK_OK;
   }
 
-  int graph(DevInstance* d_insts, int nblocks, const SweepArgs& A, const EngineParams& P, size_t lds, int threads) {
+  // the round kernel of a workgroup size, pricing rule and tree placement (a tree in global
+  // memory always has 1024 threads)
+  static const void* round_fn(int threads, int rule, bool tree_global) {
+    return (threads == 512 ? round_kernels_512 : tree_global ? round_kernels_1024_global : round_kernels_1024)[rule];
+  }
+
+  int graph(DevInstance* d_insts, const DevInstance& geo, int nblocks, const SweepArgs& A, const EngineParams& P, size_t lds,
+            int threads) {
     if (exec && g_insts == d_insts && g_nblocks == nblocks && g_threads == threads &&
         std::memcmp(&g_A, &A, sizeof A) == 0 && std::memcmp(&g_P, &P, sizeof P) == 0)
       return FLOCK_OK;
@@ -583,13 +546,11 @@ struct LargeRunner {
     HIP_TRY(hipStreamBeginCapture(g_stream, hipStreamCaptureModeThreadLocal));
     for (int k = 0; k < kRoundsPerGraph; ++k) {
       hipLaunchKernelGGL(k_large_sweep, dim3(nblocks), dim3(256), 0, g_stream, A);
-      const bool multi = P.pricing == 2 || P.pricing == 4;
-      const void* fn = threads == 512 ? (multi ? (const void*)k_large_round<512, true> : (const void*)k_large_round<512, false>)
-                                      : (multi ? (const void*)k_large_round<1024, true> : (const void*)k_large_round<1024, false>);
+      const void* fn = round_fn(threads, rule_of(P), P.tree_global != 0);
       const uint64_t* kp = keys;
       const int32_t* cp = cands;
       int32_t nb = nblocks;
-      void* args[] = {(void*)&d_insts, (void*)&kp, (void*)&cp, (void*)&nb, (void*)&P};
+      void* args[] = {(void*)&d_insts, (void*)&geo, (void*)&kp, (void*)&cp, (void*)&nb, (void*)&P};
       (void)hipLaunchKernel(fn, dim3(1), dim3(threads), args, lds, g_stream);
     }
     const hipError_t ce = hipStreamEndCapture(g_stream, &gr);
@@ -629,11 +590,10 @@ struct LargeRunner {
       P.tree_global = 1;
     }
     const int threads = (g_large_threads == 512 && !P.tree_global && o.m + o.n <= kLargeSmallMaxV) ? 512 : 1024;
-    const void* fsetup = threads == 512 ? (const void*)k_large_setup<512> : (const void*)k_large_setup<1024>;
+    const void* const fsetup = threads == 512 ? setup_kernel_512 : setup_kernel_1024;
     if (lds > 65536) {
-      const void* fns[] = {(const void*)k_large_round<512, false>, (const void*)k_large_round<512, true>,
-                           (const void*)k_large_round<1024, false>, (const void*)k_large_round<1024, true>};
-      for (const void* f : fns) HIP_TRY(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      HIP_TRY(hipFuncSetAttribute(round_fn(threads, rule_of(P), P.tree_global != 0),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     }
     // the set-up kernel runs alone: it takes the LDS that Vogel's register mode needs for
     // its line state and tracked keys when that is more than the rounds' and still fits
@@ -664,8 +624,8 @@ struct LargeRunner {
       void* args[] = {(void*)&di, (void*)&books, (void*)&Ps};
       HIP_TRY(hipLaunchKernel(fsetup, dim3(1), dim3(threads), args, slds, g_stream));
     }
-    SweepArgs A = sweep_args(b.hdesc[0], o.m + o.n, keys, cands, vpt, &b.d_insts[0].phase);
-    if ((st = graph(b.d_insts, nblocks, A, P, lds, threads))) return st;
+    SweepArgs A = sweep_args(b.hdesc[0], keys, cands, vpt, &b.d_insts[0].phase);
+    if ((st = graph(b.d_insts, b.hdesc[0], nblocks, A, P, lds, threads))) return st;
     // every round pivots or finishes, so maxIt + 1 rounds always suffice
     const int64_t maxIt = P.max_iterations > 0 ? P.max_iterations : 50LL * (o.m + o.n) + 100000;
     const int64_t maxGraphs = (maxIt + 1) / kRoundsPerGraph + 3;
@@ -698,7 +658,14 @@ LargeRunner* large_runner() {
   return r;
 }
 
-int graph_min_cells() { return g_graph_min_cells; }
+// whether a plain solve takes the graph path
+bool use_graph_path(const flock_instance* in, const flock_options* opt) {
+  if (in->m + in->n > kMaxVertices) return true;
+  if (g_graph_min_cells <= 0 || (opt && opt->threads != 0)) return false;
+  const bool cand = opt && (opt->pricing == FLOCK_PRICE_CANDIDATES || opt->pricing == FLOCK_PRICE_AUTO);
+  const int64_t factor = cand && snap_fits_lds(in->m, in->n) ? kCandGraphFactor : 1;
+  return (int64_t)in->m * in->n >= factor * g_graph_min_cells;
+}
 
 // ---------------------------------------------------------------------------
 // Plain solve of one instance on the per-instance engine, with the fewest host-device
@@ -846,9 +813,7 @@ int flock_solve(const flock_instance* inst, const flock_options* opt, flock_resu
   flock::Batch& b = *bp;
   // large matrices: graph of sweep-grid and pivot-round kernels (needs the state buffer);
   // instances whose tree cannot live in one workgroup's LDS always take it
-  const int gmin = flock::graph_min_cells();
-  const bool large = (inst->m + inst->n > flock::kMaxVertices) ||
-                     (gmin > 0 && (!opt || opt->threads == 0) && (int64_t)inst->m * inst->n >= gmin);
+  const bool large = flock::use_graph_path(inst, opt);
   if (!large) {  // per-instance engine: one copy in, one launch, one copy out
     static thread_local flock::PlainArena* pa = new flock::PlainArena();
     st = pa->solve(inst, opt, res);
@@ -1073,7 +1038,9 @@ int flock_autotune_large(const flock_instance* inst, const flock_options* opt, f
   bool have_ref = false;
   double bms = 1e300;
   // one measurement: warm-up + timed solve; the objective must equal the first one's
-  auto measure = [&](const flock_tuning& t, double* ms) -> int {
+  auto measure = [&](flock_tuning t, double* ms) -> int {
+    // the path is measured wherever graph_min_cells sends any pricing rule to it
+    if (t.graph_min_cells > 0) t.graph_min_cells = std::max(1, t.graph_min_cells / kCandGraphFactor);
     int e = flock_tuning_set(&t);
     if (e) return e;
     flock_result r;
@@ -1131,7 +1098,7 @@ int flock_measure_sweep(const flock_instance* inst, int32_t reps, double* sweep_
   // the sweep kernel reads the duals from the saved tree state and runs while phase == 1
   b.hdesc[0].phase = 1;
   const flock::Batch::Offs& o = b.offs[0];
-  HIP_TRY(hipMemsetAsync((char*)b.base + o.state, 0, 4 * 7 * (size_t)(o.m + o.n), flock::lib_stream()));
+  HIP_TRY(hipMemsetAsync((char*)b.base + o.state, 0, state_bytes(o.m, o.n), flock::lib_stream()));
   if ((st = b.upload(inst))) return st;
   uint32_t vpt;
   int nblocks;
@@ -1141,7 +1108,7 @@ int flock_measure_sweep(const flock_instance* inst, int32_t reps, double* sweep_
   HIP_TRY(hipEventCreate(&e0));
   HIP_TRY(hipEventCreate(&e1));
   hipStream_t sm = flock::lib_stream();
-  const SweepArgs A = sweep_args(b.hdesc[0], o.m + o.n, lr->keys, lr->cands, vpt, &b.d_insts[0].phase);
+  const SweepArgs A = sweep_args(b.hdesc[0], lr->keys, lr->cands, vpt, &b.d_insts[0].phase);
   auto timed = [&](bool sweep, double* out) -> int {
     for (int w = 0; w < 3; ++w) {  // warm-up
       if (sweep) hipLaunchKernelGGL(k_large_sweep, dim3(nblocks), dim3(256), 0, sm, A);

@@ -40,7 +40,7 @@ int launch_reset(DevInstance* d_insts, int32_t count, int32_t* d_heads, int32_t 
                  uint64_t* d_t0 = nullptr);
 EngineParams make_params(const flock_options* opt);
 int noalloc_setup();  // noalloc.hip: per-device set-up of flock_solve_noalloc
-int graph_min_cells();
+bool use_graph_path(const flock_instance* in, const flock_options* opt);
 struct LargeRunner;
 LargeRunner* large_runner();
 

@@ -92,7 +92,7 @@ size_t request_bytes(int m, int n, int* ld, int* ldT) {
   *ld = (n + 3) & ~3;
   *ldT = (m + 3) & ~3;
   return al(4 * (size_t)m * *ld) + al(4 * (size_t)n * *ldT) + al(4 * (size_t)m) + al(4 * (size_t)n) +
-         4 * al(4 * (size_t)V) + al(4 * aux_ints(m, n)) + al(4 * 7 * (size_t)V);
+         4 * al(4 * (size_t)V) + al(4 * aux_ints(m, n)) + al(state_bytes(m, n));
 }
 
 constexpr size_t kStagingBytes = (size_t)256 << 20;

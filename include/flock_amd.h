@@ -192,7 +192,8 @@ void flock_server_destroy(flock_server* s);
 /* ---- size-class policy (which engine configuration solves an instance) ----------
  * Instances with m+n <= wave_max_v get one 64-lane wavefront each, wave_pack (1, 2 or
  * 4) per workgroup; larger ones get a 256-thread workgroup up to wg256_max_v, else a
- * 1024-thread workgroup.  flock_autotune() measures candidates on a sample and installs
+ * 512-thread workgroup while their basis tree fits its LDS (m+n up to about 3600), else
+ * 1024 threads.  flock_autotune() measures candidates on a sample and installs
  * the fastest; flock_tuning_set/get read and write the policy directly. */
 typedef struct flock_tuning {
   int32_t wave_max_v;
@@ -207,8 +208,9 @@ typedef struct flock_tuning {
   /* must be 0 (team sweeps, where idle workgroups helped sweep one large matrix, are
    * not part of this library; large matrices take the graph path below) */
   int32_t team_min_cells;
-  /* plain solves of matrices with at least this many cells run as a graph of sweep-grid
-   * and pivot-round kernels (0: never) */
+  /* plain solves of matrices with at least this many cells (four times as many with
+   * candidate pricing, for m+n up to about 3600) run as a graph of sweep-grid and
+   * pivot-round kernels (0: never) */
   int32_t graph_min_cells;
   /* per mille (0..1000) of each launch's instances, largest first, whose workgroups run at
    * raised wave priority, so that co-resident workgroups do not slow the instances that
@@ -227,7 +229,7 @@ int flock_tuning_get(flock_tuning* t);
 int flock_tuning_set(const flock_tuning* t);
 /* Autotuner: uploads the `count` sample instances once, then measures candidate
  * policies on them (one warm-up and one timed batch launch each, coordinate descent
- * over the minor-iteration limit, the 256- vs 1024-thread threshold, instances per
+ * over the minor-iteration limit, the 256-thread threshold, instances per
  * workgroup (a wavefront per instance, 1, 2 or 4 per workgroup, for the smallest
  * instances) and the raised-priority share), checks that every candidate returns the
  * same objectives, installs the fastest and returns it in *out with its batch time in
@@ -235,8 +237,8 @@ int flock_tuning_set(const flock_tuning* t);
 int flock_autotune(int32_t count, const flock_instance* inst, const flock_options* opt, flock_tuning* out,
                    double* best_ms);
 
-/* Autotuner of the large-instance path: solves `inst` (which must take the graph path:
- * at least graph_min_cells cells, or m+n > 8000) with each sweep tile shape (1, 2, 4, 8
+/* Autotuner of the large-instance path: solves `inst` (at least graph_min_cells cells, or
+ * m+n > 8000) on the graph path with each sweep tile shape (1, 2, 4, 8
  * vectors per thread), then at the best shape with the other set-up / round workgroup
  * size (512 or 1024 threads), then (candidate pricing) with the path's minor limit at
  * 32, 64 and 128, two solves each, checks that the objectives agree, installs the

@@ -312,7 +312,7 @@ extern "C" int emu_solve(int m, int n, const int32_t* cost, const int32_t* suppl
   int32_t* bf = exact<int32_t>(V - 1);
   int32_t* du = exact<int32_t>(V);
   int32_t* scr = exact<int32_t>(aux_ints(m, n));
-  int32_t* st = exact<int32_t>(7 * (size_t)V);
+  int32_t* st = exact<int32_t>(state_bytes(m, n) / 4);
   DevInstance D;
   std::memset(&D, 0, sizeof D);
   D.cost = c; D.costT = cT; D.supply = s; D.demand = d; D.m = m; D.n = n; D.ld = ld; D.ldT = ldT;
@@ -375,7 +375,7 @@ extern "C" int emu_large(int m, int n, const int32_t* cost, const int32_t* suppl
   int32_t* d = exact<int32_t>(n); std::memcpy(d, demand, 4 * (size_t)n);
   D.supply = s; D.demand = d; D.m = m; D.n = n; D.ld = ld; D.ldT = ldT;
   D.basis_row = exact<int32_t>(V - 1); D.basis_col = exact<int32_t>(V - 1); D.basis_flow = exact<int32_t>(V - 1);
-  D.dual = exact<int32_t>(V); D.scratch = exact<int32_t>(aux_ints(m, n)); D.state = exact<int32_t>(7 * (size_t)V);
+  D.dual = exact<int32_t>(V); D.scratch = exact<int32_t>(aux_ints(m, n)); D.state = exact<int32_t>(state_bytes(m, n) / 4);
   EngineParams P;
   std::memset(&P, 0, sizeof P);
   P.pricing = pricing; P.minor_limit = 64;
@@ -407,11 +407,16 @@ extern "C" int emu_large(int m, int n, const int32_t* cost, const int32_t* suppl
   run_lanes<256>([&] { large_setup<256>(D, region, region_bytes, P, gl((const int16_t*)books)); });
   int rounds = 0;
   while (!setup_only && D.phase == 1 && rounds < 1000000) {
-    const SweepArgs A = sweep_args(D, V, keys, cands, vpt, &D.phase);
+    const SweepArgs A = sweep_args(D, keys, cands, vpt, &D.phase);
     for (int b = 0; b < nblocks; ++b) run_lanes<256>([&, b] { sweep_tile<256>(A, (uint32_t)b, *S); });
     run_lanes<256>([&] {
-      if (pricing == 2 || pricing == 4) large_round<256, true>(D, region, region_bytes, P, keys, cands, nblocks);
-      else large_round<256, false>(D, region, region_bytes, P, keys, cands, nblocks);
+      auto round = [&](auto rule) {
+        if (tree_global) large_round<256, decltype(rule)::value, true>(D, D, region, region_bytes, P, keys, cands, nblocks);
+        else large_round<256, decltype(rule)::value, false>(D, D, region, region_bytes, P, keys, cands, nblocks);
+      };
+      if (pricing == 2 || pricing == 4) round(std::integral_constant<int, kRuleMulti>{});
+      else if (pricing == 1) round(std::integral_constant<int, kRuleCandidates>{});
+      else round(std::integral_constant<int, kRuleDantzig>{});
     });
     ++rounds;
   }
