@@ -206,11 +206,15 @@ def options(pricing: str = "dantzig", initial: str = "vogel", max_iterations: in
     return o
 
 
+def _address(a: np.ndarray) -> int:
+    return a.__array_interface__["data"][0]
+
+
 def _as_c(inst):
     cost = np.ascontiguousarray(inst.cost, dtype=np.int32)
     supply = np.ascontiguousarray(inst.supply, dtype=np.int32)
     demand = np.ascontiguousarray(inst.demand, dtype=np.int32)
-    ci = _Instance(cost.shape[0], cost.shape[1], cost.ctypes.data, supply.ctypes.data, demand.ctypes.data)
+    ci = _Instance(cost.shape[0], cost.shape[1], _address(cost), _address(supply), _address(demand))
     return ci, (cost, supply, demand)
 
 
@@ -249,6 +253,30 @@ def _result_buffers(m: int, n: int):
     r.u = bufs["u"].ctypes.data
     r.v = bufs["v"].ctypes.data
     return r, bufs
+
+
+def _batch_buffers(insts, res):
+    """Result arrays of a whole batch: one allocation per field, each instance's arrays
+    slices of it (six allocations per instance otherwise).  Sets the pointers in `res`."""
+    ms = [inst.m for inst in insts]
+    ns = [inst.n for inst in insts]
+    slots = sum(ms) + sum(ns) - len(insts)
+    fields = {k: np.zeros(slots, np.int32) for k in ("rows", "cols", "flows")}
+    u, v, fl = np.zeros(sum(ms), np.int32), np.zeros(sum(ns), np.int32), np.zeros((slots, 3), np.int32)
+    at = {k: _address(a) for k, a in dict(fields, u=u, v=v, fl=fl).items()}
+    bufs, s, i, j = [], 0, 0, 0
+    for r, m, n in zip(res, ms, ns):
+        e = s + m + n - 1
+        bufs.append(dict(rows=fields["rows"][s:e], cols=fields["cols"][s:e], flows=fields["flows"][s:e],
+                         u=u[i:i + m], v=v[j:j + n], fl=fl[s:e]))
+        r.flows = at["fl"] + 12 * s
+        r.basis_row = at["rows"] + 4 * s
+        r.basis_col = at["cols"] + 4 * s
+        r.basis_flow = at["flows"] + 4 * s
+        r.u = at["u"] + 4 * i
+        r.v = at["v"] + 4 * j
+        s, i, j = e, i + m, j + n
+    return bufs
 
 
 def _solution(r: _Result, b) -> Solution:
@@ -309,14 +337,7 @@ class Batch:
     def results(self, full: bool = True) -> list[Solution]:
         n = len(self.insts)
         res = (_Result * n)()
-        bufs = []
-        for k, inst in enumerate(self.insts):
-            if full:
-                r, b = _result_buffers(inst.m, inst.n)
-            else:
-                r, b = _Result(), None
-            res[k] = r
-            bufs.append(b)
+        bufs = _batch_buffers(self.insts, res) if full else None
         st = lib().flock_batch_results(self._h, res)
         if st:
             raise FlockError(st, last_error())

@@ -307,22 +307,34 @@ int Batch::layout(int32_t count, const flock_instance* inst, bool with_state) {
   off += al(sizeof(int32_t) * (size_t)count);  // order
   off += al(sizeof(int32_t) * kMaxClasses);    // queue heads
   off += al(sizeof(uint64_t));                 // device clock at the batch launch
+  // outputs of all instances first, so that they come back in one copy; then each
+  // instance's inputs (cost, supply, demand adjacent, so that they go over together) and
+  // its device-only buffers
+  out_off = off;
   for (int k = 0; k < count; ++k) {
-    const int m = inst[k].m, nn = inst[k].n, V = m + nn;
+    const size_t V = (size_t)inst[k].m + inst[k].n;
+    Offs& o = offs[k];
+    o.brow = off; off += al(4 * V);
+    o.bcol = off; off += al(4 * V);
+    o.bflow = off; off += al(4 * V);
+    o.dual = off; off += al(4 * V);
+  }
+  out_bytes = off - out_off;
+  for (int k = 0; k < count; ++k) {
+    const int m = inst[k].m, nn = inst[k].n;
     const int ld = (nn + 3) & ~3, ldT = (m + 3) & ~3;
     Offs& o = offs[k];
     o.m = m; o.n = nn; o.ld = ld; o.ldT = ldT;
     o.cost = off; off += al(4 * (size_t)m * ld);
-    o.costT = off; off += al(4 * (size_t)nn * ldT);
     o.supply = off; off += al(4 * (size_t)m);
     o.demand = off; off += al(4 * (size_t)nn);
-    o.brow = off; off += al(4 * (size_t)V);
-    o.bcol = off; off += al(4 * (size_t)V);
-    o.bflow = off; off += al(4 * (size_t)V);
-    o.dual = off; off += al(4 * (size_t)V);
-    o.scratch = off; off += al(4 * aux_ints(m, nn));
-    o.state = with_state ? off : 0; if (with_state) off += al(state_bytes(m, nn));
-    o.books = with_state ? off : 0; if (with_state) off += al(4 * (size_t)m * nn);
+  }
+  for (int k = 0; k < count; ++k) {
+    Offs& o = offs[k];
+    o.costT = off; off += al(4 * (size_t)o.n * o.ldT);
+    o.scratch = off; off += al(4 * aux_ints(o.m, o.n));
+    o.state = with_state ? off : 0; if (with_state) off += al(state_bytes(o.m, o.n));
+    o.books = with_state ? off : 0; if (with_state) off += al(4 * (size_t)o.m * o.n);
   }
   bytes = off;
   return FLOCK_OK;
@@ -360,20 +372,47 @@ int Batch::alloc() {
 }
 
 int Batch::upload(const flock_instance* inst, char* pinned, size_t pinned_cap) {
-  for (int k = 0; k < n; ++k) {
-    const Offs& o = offs[k];
-    char* b = (char*)base;
-    const size_t rows = 4 * (size_t)o.m * o.ld;
-    if (pinned && n == 1 && rows <= pinned_cap) {  // padded rows staged in pinned memory: one fast copy
-      for (int i = 0; i < o.m; ++i)
-        std::memcpy(pinned + 4 * (size_t)i * o.ld, inst[k].cost + (size_t)i * o.n, 4 * (size_t)o.n);
-      HIP_TRY(hipMemcpyAsync(b + o.cost, pinned, rows, hipMemcpyHostToDevice, g_stream));
-    } else {
-      HIP_TRY(hipMemcpy2DAsync(b + o.cost, 4 * (size_t)o.ld, inst[k].cost, 4 * (size_t)o.n, 4 * (size_t)o.n, o.m,
-                               hipMemcpyHostToDevice, g_stream));
+  char* b = (char*)base;
+  if (pinned && n == 1 && 4 * (size_t)offs[0].m * offs[0].ld <= pinned_cap) {
+    // padded rows staged in pinned memory: one fast copy
+    const Offs& o = offs[0];
+    for (int i = 0; i < o.m; ++i)
+      std::memcpy(pinned + 4 * (size_t)i * o.ld, inst[0].cost + (size_t)i * o.n, 4 * (size_t)o.n);
+    HIP_TRY(hipMemcpyAsync(b + o.cost, pinned, 4 * (size_t)o.m * o.ld, hipMemcpyHostToDevice, g_stream));
+    HIP_TRY(hipMemcpyAsync(b + o.supply, inst[0].supply, 4 * (size_t)o.m, hipMemcpyHostToDevice, g_stream));
+    HIP_TRY(hipMemcpyAsync(b + o.demand, inst[0].demand, 4 * (size_t)o.n, hipMemcpyHostToDevice, g_stream));
+  } else {
+    // The instances' inputs are contiguous on the device: they are packed on the host in
+    // pieces of up to kUploadPiece bytes (or one larger instance), one copy each.  (Three
+    // copies an instance: 512 instances of up to 96x96 took 224 ms from host arrays to
+    // solutions, most of it in copies of a few hundred bytes; 4.7 ms with one copy each
+    // way.)
+    constexpr size_t kUploadPiece = (size_t)8 << 20;
+    std::vector<char> piece;
+    for (int k0 = 0; k0 < n;) {
+      const size_t begin = offs[k0].cost;
+      int k1 = k0;
+      size_t end = begin;
+      while (k1 < n) {
+        const size_t e = offs[k1].demand + al(4 * (size_t)offs[k1].n);
+        if (k1 > k0 && e - begin > kUploadPiece) break;
+        end = e; ++k1;
+      }
+      if (piece.size() < end - begin) piece.resize(end - begin);
+      for (int k = k0; k < k1; ++k) {
+        const Offs& o = offs[k];
+        char* c = piece.data() + (o.cost - begin);
+        if (o.ld == o.n) std::memcpy(c, inst[k].cost, 4 * (size_t)o.m * o.n);
+        else
+          for (int i = 0; i < o.m; ++i)
+            std::memcpy(c + 4 * (size_t)i * o.ld, inst[k].cost + (size_t)i * o.n, 4 * (size_t)o.n);
+        std::memcpy(piece.data() + (o.supply - begin), inst[k].supply, 4 * (size_t)o.m);
+        std::memcpy(piece.data() + (o.demand - begin), inst[k].demand, 4 * (size_t)o.n);
+      }
+      HIP_TRY(hipMemcpyAsync(b + begin, piece.data(), end - begin, hipMemcpyHostToDevice, g_stream));
+      HIP_TRY(hipStreamSynchronize(g_stream));  // the piece is packed again
+      k0 = k1;
     }
-    HIP_TRY(hipMemcpyAsync(b + o.supply, inst[k].supply, 4 * (size_t)o.m, hipMemcpyHostToDevice, g_stream));
-    HIP_TRY(hipMemcpyAsync(b + o.demand, inst[k].demand, 4 * (size_t)o.n, hipMemcpyHostToDevice, g_stream));
   }
   HIP_TRY(hipMemcpyAsync(d_insts, hdesc.data(), sizeof(DevInstance) * (size_t)n, hipMemcpyHostToDevice, g_stream));
   // Work order: largest estimated work first (pivots ~ m+n, each sweeping m*n cells).
@@ -442,7 +481,14 @@ int Batch::download_desc() {
   return FLOCK_OK;
 }
 
-int Batch::fill_result(int k, flock_result* r) {
+int Batch::download_outputs() {
+  h_out.resize(out_bytes);
+  HIP_TRY(hipMemcpyAsync(h_out.data(), (const char*)base + out_off, out_bytes, hipMemcpyDeviceToHost, g_stream));
+  HIP_TRY(hipStreamSynchronize(g_stream));
+  return FLOCK_OK;
+}
+
+void Batch::fill_result(int k, flock_result* r) {
   const DevInstance& D = hdesc[k];
   const Offs& o = offs[k];
   const int V = o.m + o.n;
@@ -450,39 +496,26 @@ int Batch::fill_result(int k, flock_result* r) {
   r->iterations = D.iterations;
   r->status = D.status;
   r->sweeps = D.sweeps;
-  for (int k = 0; k < 6; ++k) r->phase_us[k] = (double)D.ticks[k] / g_ticks_per_us;
+  for (int q = 0; q < 6; ++q) r->phase_us[q] = (double)D.ticks[q] / g_ticks_per_us;
   r->start_us = (double)(int64_t)(D.t_start - h_t0) / g_ticks_per_us;
   r->done_us = (double)(int64_t)(D.t_done - h_t0) / g_ticks_per_us;
-  r->n_flows = 0;
-  char* b = (char*)base;
-  std::vector<int32_t> br, bc, bf;
-  const bool need_basis = r->flows || r->basis_row || r->basis_col || r->basis_flow;
-  if (need_basis) {
-    br.resize(V - 1); bc.resize(V - 1); bf.resize(V - 1);
-    if (V > 1) {
-      HIP_TRY(hipMemcpyAsync(br.data(), b + o.brow, 4 * (size_t)(V - 1), hipMemcpyDeviceToHost, g_stream));
-      HIP_TRY(hipMemcpyAsync(bc.data(), b + o.bcol, 4 * (size_t)(V - 1), hipMemcpyDeviceToHost, g_stream));
-      HIP_TRY(hipMemcpyAsync(bf.data(), b + o.bflow, 4 * (size_t)(V - 1), hipMemcpyDeviceToHost, g_stream));
-    }
+  r->n_flows = D.n_flows;
+  if (!wants_arrays(*r)) return;
+  auto at = [&](size_t off) { return (const int32_t*)(h_out.data() + (off - out_off)); };
+  const int32_t *br = at(o.brow), *bc = at(o.bcol), *bf = at(o.bflow), *du = at(o.dual);
+  if (r->u) std::memcpy(r->u, du, 4 * (size_t)o.m);
+  if (r->v) std::memcpy(r->v, du + o.m, 4 * (size_t)o.n);
+  if (r->basis_row) std::memcpy(r->basis_row, br, 4 * (size_t)(V - 1));
+  if (r->basis_col) std::memcpy(r->basis_col, bc, 4 * (size_t)(V - 1));
+  if (r->basis_flow) std::memcpy(r->basis_flow, bf, 4 * (size_t)(V - 1));
+  if (!(r->flows || r->basis_row || r->basis_col || r->basis_flow)) return;
+  int nf = 0;
+  for (int s = 0; s < V - 1; ++s) {
+    if (bf[s] == 0) continue;
+    if (r->flows) r->flows[nf] = flock_flow{br[s], bc[s], bf[s]};
+    ++nf;
   }
-  if (r->u) HIP_TRY(hipMemcpyAsync(r->u, b + o.dual, 4 * (size_t)o.m, hipMemcpyDeviceToHost, g_stream));
-  if (r->v) HIP_TRY(hipMemcpyAsync(r->v, b + o.dual + 4 * (size_t)o.m, 4 * (size_t)o.n, hipMemcpyDeviceToHost, g_stream));
-  HIP_TRY(hipStreamSynchronize(g_stream));
-  if (need_basis) {
-    if (r->basis_row) std::memcpy(r->basis_row, br.data(), 4 * (size_t)(V - 1));
-    if (r->basis_col) std::memcpy(r->basis_col, bc.data(), 4 * (size_t)(V - 1));
-    if (r->basis_flow) std::memcpy(r->basis_flow, bf.data(), 4 * (size_t)(V - 1));
-    int nf = 0;
-    for (int s = 0; s < V - 1; ++s) {
-      if (bf[s] == 0) continue;
-      if (r->flows) r->flows[nf] = flock_flow{br[s], bc[s], bf[s]};
-      ++nf;
-    }
-    r->n_flows = nf;
-  } else {
-    r->n_flows = D.n_flows;
-  }
-  return FLOCK_OK;
+  r->n_flows = nf;
 }
 
 Batch::~Batch() {
@@ -841,12 +874,14 @@ int flock_solve(const flock_instance* inst, const flock_options* opt, flock_resu
   st = flock::large_runner()->run(b, P);
   if (st) { res->status = st; return st; }
   HIP_TRY(hipEventRecord(e1, flock::lib_stream()));
-  if ((st = b.download_desc())) { res->status = st; return st; }
+  if ((st = b.download_desc()) || (flock::Batch::wants_arrays(*res) && (st = b.download_outputs()))) {
+    res->status = st;
+    return st;
+  }
   float ms = 0;
   HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
-  st = b.fill_result(0, res);
+  b.fill_result(0, res);
   res->solve_ms = ms;
-  if (st) { res->status = st; return st; }
   return res->status;
 }
 
@@ -894,11 +929,11 @@ int flock_batch_results(flock_batch* bb, flock_result* res) {
   flock::Batch* b = reinterpret_cast<flock::Batch*>(bb);
   if (!b || !res) return flock::set_error(FLOCK_E_INVALID, "null batch/result");
   int st = b->download_desc();
+  bool arrays = false;
+  for (int k = 0; k < b->n; ++k) arrays = arrays || flock::Batch::wants_arrays(res[k]);
+  if (!st && arrays) st = b->download_outputs();
   if (st) return st;
-  for (int k = 0; k < b->n; ++k) {
-    st = b->fill_result(k, &res[k]);
-    if (st) return st;
-  }
+  for (int k = 0; k < b->n; ++k) b->fill_result(k, &res[k]);
   return FLOCK_OK;
 }
 

@@ -68,6 +68,8 @@ struct Batch {
   std::vector<Class> classes;
   std::vector<int32_t> sorted_order;
   std::vector<int32_t> class_order;
+  size_t out_off = 0, out_bytes = 0;  // every instance's basis and duals, contiguous
+  std::vector<char> h_out;            // their host copy (download_outputs)
   int64_t planned_for = -1;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0;
@@ -80,7 +82,12 @@ struct Batch {
   int plan(const flock_options* opt);
   int run(const EngineParams& P, int grid_cap);
   int download_desc();
-  int fill_result(int k, flock_result* r);
+  int download_outputs();
+  // needs download_desc(), and download_outputs() where the result asks for arrays
+  void fill_result(int k, flock_result* r);
+  static bool wants_arrays(const flock_result& r) {
+    return r.flows || r.basis_row || r.basis_col || r.basis_flow || r.u || r.v;
+  }
   ~Batch();
 };
 

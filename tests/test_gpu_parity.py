@@ -212,6 +212,28 @@ def test_sweep_block_edges_exact(threads):
         assert c.objective == o.objective and certify(inst, c)[0] == 0
 
 
+@pytest.mark.parametrize("sizes", [[(1, 1)], [(1, 2), (3, 5), (2, 1)], [(17, 33), (1500, 1500), (5, 6), (64, 63)],
+                                   [(600, 701)] * 7 + [(9, 250)]])
+def test_batch_packed_copies(sizes):
+    """A batch's packed upload (pieces of 8 MiB, one instance larger than a piece, a piece
+    that ends between instances, padded and unpadded rows) and its one download: every
+    result certified, its arrays the instance's own, objectives equal to plain solves."""
+    rng = np.random.default_rng(len(sizes))
+    insts = [_rand(rng, m, n, cmax=900) for m, n in sizes]
+    say("packed batch", sizes)
+    b = F.Batch(insts)
+    b.run(pricing="candidates")
+    full, short = b.results(), b.results(full=False)
+    b.close()
+    for inst, s, q in zip(insts, full, short):
+        p = F.solve(inst, pricing="candidates")
+        assert s.status == 0 and s.objective == q.objective == p.objective
+        assert s.iterations == q.iterations and s.n_flows == q.n_flows == len(s.flow_list)
+        assert certify(inst, s) == (0, s.objective)
+        pos = s.flows != 0
+        assert np.array_equal(s.flow_list, np.stack([s.rows[pos], s.cols[pos], s.flows[pos]], axis=1))
+
+
 def test_batch_mixed_configurations():
     """One batch mixing wavefront and workgroup classes, candidates pricing."""
     rng = np.random.default_rng(8)
