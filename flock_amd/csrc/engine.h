@@ -69,8 +69,7 @@ struct Shared {
   int32_t cnt2;       // Vogel: column refresh list counter (cnt: rows)
   int32_t lastx;      // Vogel: the line covered by the previous step
   int32_t dlo[2];     // pivot: least depth of a cycle vertex (atomicMin), by pivot parity
-  int32_t dsel;       // pivot: parity slot of dlo used by the next pivot
-  int32_t pad_[5];
+  int32_t pad_[6];
   uint64_t red1[3][16];  // one-barrier reductions (group_min1 / group_max1), by buffer
 };
 
@@ -1037,32 +1036,34 @@ struct SweepSlots { static constexpr int value = G == kWave ? 4 : 8; };
 template <int G>
 struct CandsPerRank { static constexpr int value = G == kWave ? 4 : 8; };
 
-// Cell (row, col) as one word whose order is row-major order (m+n <= 16383)
-__device__ __forceinline__ uint32_t cell_id(uint32_t row, uint32_t col) { return (row << 16) | col; }
-__device__ __forceinline__ int cell_row(uint64_t key) { return (int)((uint32_t)key >> 16); }
-__device__ __forceinline__ int cell_col(uint64_t key) { return (int)((uint32_t)key & 0xffffu); }
+// Cell (row, col) as one word whose order is row-major order (m+n <= 16383); the halves are
+// the byte offsets of the row's and the column's dual.
+__device__ __forceinline__ uint32_t cell_id(uint32_t row, uint32_t col) { return (row << 18) | (col << 2); }
+__device__ __forceinline__ int cell_row(uint64_t key) { return (int)((uint32_t)key >> 18); }
+__device__ __forceinline__ int cell_col(uint64_t key) { return (int)(((uint32_t)key & 0xffffu) >> 2); }
 
 struct Cand {
   int32_t row, col, cost;
 };
-// K candidate cells of one rank: row << 16 | col (-1: none) and cost
+// K candidate cells of one rank: cell id and cost (an empty slot is cell 0 at the padding
+// cost, which never prices negative: u_0 = 0 and every dual is below 2^30)
 template <int K>
 struct CandSet {
-  int32_t rc[K];
+  uint32_t id[K];
   int32_t cost[K];
   __device__ __forceinline__ void clear() {
 #pragma unroll
-    for (int k = 0; k < K; ++k) { rc[k] = -1; cost[k] = 0; }
+    for (int k = 0; k < K; ++k) { id[k] = 0; cost[k] = kPadCost; }
   }
   __device__ __forceinline__ Cand get(int k) const {
     Cand c;
-    c.row = rc[k] < 0 ? -1 : (rc[k] >> 16);
-    c.col = rc[k] < 0 ? 0 : (rc[k] & 0xffff);
+    c.row = cell_row(id[k]);
+    c.col = cell_col(id[k]);
     c.cost = cost[k];
     return c;
   }
   __device__ __forceinline__ void set(int k, const Cand& c) {
-    rc[k] = c.row < 0 ? -1 : ((c.row << 16) | c.col);
+    id[k] = cell_id((uint32_t)c.row, (uint32_t)c.col);
     cost[k] = c.cost;
   }
 };
@@ -1201,14 +1202,14 @@ __device__ __forceinline__ uint64_t sweep_argmin(const Ctx& C, const TreeLds& t,
       r = better ? bestR[s] : r;
       id = better ? is : id;
     }
-    const uint32_t br = id >> 16, bc = id & 0xffffu;
+    const uint32_t br = (uint32_t)cell_row(id), bc = (uint32_t)cell_col(id);
     const i32x4 c = *(const FLOCK_GLOBAL i32x4*)((gcbyte*)C.cost + 4 * (br * ld + bc));
     const int32_t u = t.du[br];
     const i32x4 vv = *(const i32x4*)(t.dv + bc);
     const int e = c.x - vv.x - u == r ? 0 : c.y - vv.y - u == r ? 1 : c.z - vv.z - u == r ? 2 : 3;
-    mine.rc[0] = (int32_t)(id + (uint32_t)e);
+    mine.id[0] = id + 4 * (uint32_t)e;
     mine.cost[0] = e == 0 ? c.x : e == 1 ? c.y : e == 2 ? c.z : c.w;
-    key = pack_vi(r, id + (uint32_t)e);
+    key = pack_vi(r, id + 4 * (uint32_t)e);
   } else {
     // each slot's first cell at its minimum (its vector reloaded; the K loads together)
     i32x4 cv[K];
@@ -1221,7 +1222,7 @@ __device__ __forceinline__ uint64_t sweep_argmin(const Ctx& C, const TreeLds& t,
       const i32x4 c = cv[k];
       const int e = c.x - vv.x - u == bestR[k] ? 0 : c.y - vv.y - u == bestR[k] ? 1 : c.z - vv.z - u == bestR[k] ? 2 : 3;
       const uint32_t id = cell_id(bestRow[k], col[k] + (uint32_t)e);
-      mine.rc[k] = (int32_t)id;
+      mine.id[k] = id;
       mine.cost[k] = e == 0 ? c.x : e == 1 ? c.y : e == 2 ? c.z : c.w;
       const uint64_t kk = pack_vi(bestR[k], id);
       key = kk < key ? kk : key;
@@ -1230,21 +1231,22 @@ __device__ __forceinline__ uint64_t sweep_argmin(const Ctx& C, const TreeLds& t,
   return group_min1_u64<G, 2>(key, S);
 }
 
-// Re-price a rank's candidates with the current duals (costs kept in registers): their
-// least (r, row-major index) key.
+// Re-price a rank's candidates with the current duals (costs kept in registers): the key of
+// the least reduced cost (of equal ones the rank's first).
 template <int K>
-__device__ __forceinline__ uint64_t reprice_set(const Ctx& C, const TreeLds& t, const CandSet<K>& cs) {
-  uint64_t key = kNoKey;
+__device__ __forceinline__ uint64_t reprice_set(const TreeLds& t, const CandSet<K>& cs) {
+  int32_t best = kBig;
+  uint32_t id = 0;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int32_t rc = cs.rc[k];
-    const int row = rc < 0 ? 0 : (rc >> 16), col = rc < 0 ? 0 : (rc & 0xffff);
-    const int32_t r = cs.cost[k] - t.du[row] - t.dv[col];
-    // an empty slot ORs in all ones (kNoKey) instead of branching
-    const uint64_t kk = pack_vi(r, (uint32_t)rc) | (rc < 0 ? kNoKey : 0ull);
-    key = kk < key ? kk : key;
+    const int32_t u = *(const int32_t*)((const char*)t.du + (cs.id[k] >> 16));
+    const int32_t v = *(const int32_t*)((const char*)t.dv + (cs.id[k] & 0xffffu));
+    const int32_t r = cs.cost[k] - u - v;
+    const bool better = r < best;
+    best = better ? r : best;
+    id = better ? cs.id[k] : id;
   }
-  return key;
+  return pack_vi(best, id);
 }
 
 // Re-price a candidate with the current duals (cost kept in a register).
@@ -1381,22 +1383,34 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs& A, uint32_t tile, Sh
 //     minus P[1]).  The entering arc takes the leaving arc's slot (PIVOT_uv.cu:248-261);
 //     duals in the subtree shift by -/+ r so that the entering arc becomes tight.
 // ---------------------------------------------------------------------------
+template <int N>
+struct IntC { static constexpr int value = N; };
+
+// Phase timers: reading the clock takes 80 cycles and drains the LDS queue, and a pivot has
+// four readings, so every eighth pivot is timed and counted eight times.
+constexpr int kTimedEvery = 8;
+__device__ __forceinline__ bool timed_pivot(int count) { return count % kTimedEvery == 0; }
+
 // kR: vertices each rank handles per pass, their LDS loads issued together.
 // kWideWin: the re-root's windowed form takes twice the slots per rank where kR is below
 // four (the graph path's round kernel and the work-queue kernels below 1024 threads; the
 // 1024-thread work-queue kernel keeps kR, as it would spill more in its other phases).
 template <int G, int kR, class SN, bool kWideWin = false>
-__device__ __forceinline__ void pivot_pass(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej, int32_t r) {
+__device__ __forceinline__ bool pivot_pass(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej, int32_t r,
+                                           int count) {
   const int m = C.m, V = C.V, tid = grank<G>();
-  const uint64_t t0 = now_ticks();
+  const bool timed = timed_pivot(count);
+  uint64_t t0 = 0;
+  if (timed) t0 = now_ticks();
   const int I = ei, J = m + ej;
   // every scalar the in-place pass needs is read here or taken from the snapshot: once
   // the group minimum is known, ranks go straight on to rewrite their own vertices
   const int preI = t.pre(I), preJ = t.pre(J), depI = t.depth[I], depJ = t.depth[J];
-  const int sel = S.dsel;
+  const int sel = count & 1;
   // ---- A: leaving arc, and every cycle vertex snapshotted by side and depth (the least
   // cycle depth, one below the apex, goes to S.dlo[sel])
   uint64_t best = kNoKey;
+  int dlo = 0x7fffffff;
   // with several vertices per rank, every LDS load of a pass is issued before the first
   // use (no per-vertex branch waits on a load), so one wait covers all kR vertices
   for (int x0 = tid; x0 < V; x0 += kR * G) {
@@ -1424,7 +1438,7 @@ __device__ __forceinline__ void pivot_pass(const Ctx& C, const TreeLds& t, const
         const int sd = aI ? 0 : 1;
         sn.vert(sd)[d] = (int16_t)x; sn.ps(sd)[d] = pack_ps(px[u], sx[u]);
         sn.slot(sd)[d] = (int16_t)slx[u]; sn.flow(sd)[d] = fx[u];
-        atomicMin(&S.dlo[sel], d);
+        dlo = d < dlo ? d : dlo;
         const uint32_t lowbits =
             aI ? ((1u << 31) | ((uint32_t)d << 16) | (uint32_t)x) : (((32767u - (uint32_t)d) << 16) | (uint32_t)x);
         const uint64_t k = aI == (x < m) ? (((uint64_t)(uint32_t)fx[u] << 32) | lowbits) : kNoKey;
@@ -1432,19 +1446,23 @@ __device__ __forceinline__ void pivot_pass(const Ctx& C, const TreeLds& t, const
       }
     }
   }
-  best = group_min1_u64<G, 1>(best, S);  // its barrier also publishes the snapshot
-  if (best == kNoKey) {  // no blocking arc: the tree is corrupt; report instead of pivoting
-    if (tid == 0) S.status = 2;
-    gsync<G>();
-    return;
+  if (dlo != 0x7fffffff) {
+    int z = 0;  // opaque: known to be uniform, the address would get a loop over the lanes
+    asm volatile("" : "+v"(z));
+    atomicMin(&S.dlo[sel + z], dlo);
   }
+  best = group_min1_u64<G, 1>(best, S);  // its barrier also publishes the snapshot
+  if (best == kNoKey) return false;  // no blocking arc: the tree is corrupt (the same in every rank)
   const int a = (int)(best & 0xffffu);
   const int32_t theta = (int32_t)(best >> 32);
   const bool sideI = (best >> 31) & 1u;
   const int dA = sideI ? (int)((best >> 16) & 0x7fffu) : 32767 - (int)((best >> 16) & 0x7fffu);
   const int o = sideI ? J : I;
-  const uint64_t t1 = now_ticks();
-  if (tid == 0) S.tk[4] += (int64_t)(t1 - t0);
+  uint64_t t1 = 0;
+  if (timed) {
+    t1 = now_ticks();
+    if (tid == 0) S.tk[4] += kTimedEvery * (int64_t)(t1 - t0);
+  }
   // the chain P[0] = a .. P[k] = q on q's side: snapshot entries dA .. dA + k
   const int qs = sideI ? 0 : 1;
   const int32_t psA = sn.ps(qs)[dA];
@@ -1491,57 +1509,69 @@ __device__ __forceinline__ void pivot_pass(const Ctx& C, const TreeLds& t, const
     // instead of being hoisted to the kernel start and kept in scratch
     int tidr = tid;
     asm volatile("" : "+v"(tidr));
-    int xs[kRW], np[kRW], lo[kRW];
+    int xs[kRW], np[kRW];  // vertex (complemented: none) and new position of each slot
 #pragma unroll
-    for (int u = 0; u < kRW; ++u) {
-      const int w = tidr + u * G;
-      const int p = (w < s ? A : outBase) + w;
-      const bool valid = w < wsize;
-      // slots past the window read position 0, the root, and keep it complemented: the
-      // root is never in the window (it has no parent arc), so no rank rewrites its
-      // depth or dual in this pass; vat itself is rewritten only after the barrier below
-      const int x = t.vat[valid ? p : 0];
-      xs[u] = valid ? x : ~x;
-      lo[u] = 0;
-    }
-    // every slot searches (a slot outside the subtree keeps lo = 0): skipping slots by a
-    // uniform test costs more than the searches it saves
-    for (int len = len0; len > 1;) {
-      const int half = len >> 1;
-      int32_t v[kRW];
+    for (int u = 0; u < kRW; ++u) { xs[u] = -1; np[u] = 0; }
+    // NS slots of this wavefront: a wavefront takes only the slots that reach the window
+    // (half of them on average; four slots' work for every window was a fifth of a pivot's
+    // instructions)
+    auto slots = [&](auto ns) {
+      constexpr int NS = decltype(ns)::value;
+      int lo[NS];
 #pragma unroll
-      for (int u = 0; u < kRW; ++u) v[u] = cPS[lo[u] + half];
-#pragma unroll
-      for (int u = 0; u < kRW; ++u) {
-        const int p = A + tidr + u * G;
-        const bool anc = (uint32_t)(p - ps_pre(v[u])) < (uint32_t)ps_size(v[u]);
-        lo[u] = anc ? lo[u] + half : lo[u];
+      for (int u = 0; u < NS; ++u) {
+        const int w = tidr + u * G;
+        const int p = (w < s ? A : outBase) + w;
+        const bool valid = w < wsize;
+        // slots past the window read position 0, the root, and keep it complemented: the
+        // root is never in the window (it has no parent arc), so no rank rewrites its
+        // depth or dual in this pass; vat itself is rewritten only after the barrier below
+        const int x = t.vat[valid ? p : 0];
+        xs[u] = valid ? x : ~x;
+        lo[u] = 0;
       }
-      len -= half;
-    }
+      // every slot searches (a slot outside the subtree keeps lo = 0)
+      for (int len = len0; len > 1;) {
+        const int half = len >> 1;
+        int32_t v[NS];
 #pragma unroll
-    for (int u = 0; u < kRW; ++u) {
-      const int w = tidr + u * G;
-      const bool inSub = w < s;
-      const int p = (inSub ? A : outBase) + w;
-      const int tt = lo[u];
-      const int x = xs[u] < 0 ? ~xs[u] : xs[u];
-      const int dx = t.depth[x], di = x < m ? x : x + dvIdx;
-      const int32_t du = t.du[di];
-      // P[tt] \ P[tt+1] follows P[tt+1]'s interval; for tt = k (P[k] = q) entry t1 = k
-      // gives p >= p1, so the same formula leaves q's interval in place
-      const int t1 = tt < k ? tt + 1 : k;
-      const int32_t v0 = cPS[tt], v1 = cPS[t1];
-      const int p1 = ps_pre(v1), sz1 = ps_size(v1);
-      const int nrel = p - ps_pre(v0) + (p < p1 ? sz1 : 0);
-      np[u] = inSub ? newStart + nrel : p + shift;
-      const int ndep = inSub ? depBase + dx - 2 * tt : dx;
-      const int32_t ndual = du + (inSub ? (x < m ? dRow : dCol) : 0);
-      if (xs[u] >= 0) {
-        t.pre(x) = (int16_t)np[u]; t.depth[x] = (int16_t)ndep;
-        t.du[di] = ndual;
+        for (int u = 0; u < NS; ++u) v[u] = cPS[lo[u] + half];
+#pragma unroll
+        for (int u = 0; u < NS; ++u) {
+          const int p = A + tidr + u * G;
+          const bool anc = (uint16_t)(p - v[u]) < (uint16_t)((uint32_t)v[u] >> 16);  // p - pre < size
+          lo[u] = anc ? lo[u] + half : lo[u];
+        }
+        len -= half;
       }
-    }
+#pragma unroll
+      for (int u = 0; u < NS; ++u) {
+        const int w = tidr + u * G;
+        const bool inSub = w < s;
+        const int p = (inSub ? A : outBase) + w;
+        const int tt = lo[u];
+        const int x = xs[u] < 0 ? ~xs[u] : xs[u];
+        const int dx = t.depth[x], di = x < m ? x : x + dvIdx;
+        const int32_t du = t.du[di];
+        // P[tt] \ P[tt+1] follows P[tt+1]'s interval; for tt = k (P[k] = q) entry t1 = k
+        // gives p >= p1, so the same formula leaves q's interval in place
+        const int t1 = tt < k ? tt + 1 : k;
+        const int32_t v0 = cPS[tt], v1 = cPS[t1];
+        const int p1 = ps_pre(v1), sz1 = ps_size(v1);
+        const int nrel = p - ps_pre(v0) + (p < p1 ? sz1 : 0);
+        np[u] = inSub ? newStart + nrel : p + shift;
+        const int ndep = inSub ? depBase + dx - 2 * tt : dx;
+        const int32_t ndual = du + (inSub ? (x < m ? dRow : dCol) : 0);
+        if (xs[u] >= 0) {
+          t.pre(x) = (int16_t)np[u]; t.depth[x] = (int16_t)ndep;
+          t.du[di] = ndual;
+        }
+      }
+    };
+    const int reach = wsize - uniform(tid & ~(kWave - 1));  // window slots from this wavefront's first on
+    if (kRW > 2 && reach > 2 * G) slots(IntC<(kRW > 2 ? kRW : 2)>{});
+    else if (reach > G) slots(IntC<2>{});
+    else if (reach > 0) slots(IntC<1>{});
     // cycle vertices: sizes on the paths to o and a, flows +-theta, the chain's arcs
     for (int i = tid; i < nc; i += G) {
       const int sd = i < n0 ? 0 : 1;
@@ -1574,9 +1604,9 @@ __device__ __forceinline__ void pivot_pass(const Ctx& C, const TreeLds& t, const
 #pragma unroll
     for (int u = 0; u < kRW; ++u)
       if (xs[u] >= 0) t.vat[np[u]] = (int16_t)xs[u];
-    if (tid == 0) { S.dlo[sel ^ 1] = 0x7fffffff; S.dsel = sel ^ 1; }
-    if (tid == 0) S.tk[5] += (int64_t)(now_ticks() - t1);
-    return;
+    if (tid == 0) S.dlo[sel ^ 1] = 0x7fffffff;
+    if (timed && tid == 0) S.tk[5] += kTimedEvery * (int64_t)(now_ticks() - t1);
+    return true;
   }
   for (int x0 = tid; x0 < V; x0 += kR * G) {
     int px[kR], sx[kR], dx[kR], lo[kR];
@@ -1669,19 +1699,22 @@ __device__ __forceinline__ void pivot_pass(const Ctx& C, const TreeLds& t, const
       }
     }
   }
-  if (tid == 0) { S.dlo[sel ^ 1] = 0x7fffffff; S.dsel = sel ^ 1; }
+  if (tid == 0) S.dlo[sel ^ 1] = 0x7fffffff;
   gsync<G>();
-  if (tid == 0) S.tk[5] += (int64_t)(now_ticks() - t1);
+  if (timed && tid == 0) S.tk[5] += kTimedEvery * (int64_t)(now_ticks() - t1);
+  return true;
 }
 
+// count: a running count of pivots, its parity alternating from one pivot to the next.  Returns false, in every rank,
+// when the tree is corrupt.
 template <int G, bool kWideWin = false, class SN>
-__device__ __forceinline__ void pivot(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej,
-                                      int32_t r) {
+__device__ __forceinline__ bool pivot(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej,
+                                      int32_t r, int count) {
   // 1024-thread groups take two vertices per rank and pass at most (their registers are
   // capped at 128)
   constexpr int kRBig = G >= 1024 ? 2 : 4;
-  if (C.V > 2 * G) pivot_pass<G, kRBig, SN, kWideWin>(C, t, sn, S, ei, ej, r);
-  else pivot_pass<G, 1, SN, kWideWin>(C, t, sn, S, ei, ej, r);
+  if (C.V > 2 * G) return pivot_pass<G, kRBig, SN, kWideWin>(C, t, sn, S, ei, ej, r, count);
+  return pivot_pass<G, 1, SN, kWideWin>(C, t, sn, S, ei, ej, r, count);
 }
 
 // ---------------------------------------------------------------------------
@@ -1696,13 +1729,14 @@ __device__ __forceinline__ void pivot(const Ctx& C, const TreeLds& t, const SN& 
 // Accepted cycles share no arc, so pivoting them one after another leaves every other
 // accepted cycle, its reduced cost and its theta unchanged; they pivot best first.  The
 // best candidate always wins.  Rounds repeat on the same candidates (re-priced) up to
-// minor_limit times or until none prices negative; then the caller sweeps again.
+// minor_limit times or until none prices negative; then the caller sweeps again.  iter: the
+// pivots made before, maxIt: the budget.
 // `claim` needs V words (the pivot's snapshot region, free between pivots).  Returns
-// the pivots made; stops at the iteration budget.
+// the pivots made (-1: the tree is corrupt); stops at the iteration budget.
 // ---------------------------------------------------------------------------
 template <int G, class SN>
 __device__ __forceinline__ int multi_pivot(const Ctx& C, const TreeLds& t, const SN& sn, uint32_t* claim,
-                                           Shared& S, const Cand& cand, int64_t iter, int64_t maxIt, int rounds) {
+                                           Shared& S, const Cand& cand, int iter, int maxIt, int rounds) {
   const int m = C.m, V = C.V, tid = grank<G>();
   constexpr uint32_t kRange = (1u << 22) - 1;
   const int I = cand.row, J = m + cand.col;
@@ -1739,8 +1773,7 @@ __device__ __forceinline__ int multi_pivot(const Ctx& C, const TreeLds& t, const
       const uint64_t k = group_min_u64<G>(accepted ? reprice(C, t, cand) : kNoKey, S);
       if (k == kNoKey || key_val(k) >= 0) break;
       if (accepted && key_idx(k) == mine) { accepted = false; spent = true; }
-      pivot<G>(C, t, sn, S, cell_row(k), cell_col(k), key_val(k));
-      if (S.status != 0) return done;
+      if (!pivot<G>(C, t, sn, S, cell_row(k), cell_col(k), key_val(k), iter + done)) return -1;
       ++done; ++inRound;
     }
     if (inRound == 0) break;  // nothing prices negative any more (uniform)
@@ -1753,7 +1786,7 @@ __device__ __forceinline__ int multi_pivot(const Ctx& C, const TreeLds& t, const
 // vat, the vertex at each pre-order position.
 template <int G>
 __device__ __forceinline__ void pivot_init(Shared& S) {
-  if (grank<G>() == 0) { S.dlo[0] = 0x7fffffff; S.dlo[1] = 0x7fffffff; S.dsel = 0; }
+  if (grank<G>() == 0) { S.dlo[0] = 0x7fffffff; S.dlo[1] = 0x7fffffff; }
 }
 template <int G>
 __device__ __forceinline__ void tree_index(const Ctx& C, const TreeLds& t, Shared& S) {
@@ -1921,15 +1954,19 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
   bool haveList = false;
   for (;;) {
     uint64_t key;
-    tp = now_ticks();
     if (kCands && haveList && minor < P.minor_limit) {
-      key = group_min1_u64<G, 0>(reprice_set(C, t, cands), S);
-      if (lead) S.tk[3] += (int64_t)(now_ticks() - tp);
-      if (key == kNoKey || key_val(key) >= 0) { haveList = false; continue; }
+      const bool timed = timed_pivot(done);
+      if (timed) tp = now_ticks();
+      key = group_min1_u64<G, 0>(reprice_set(t, cands), S);
+      if (timed && lead) S.tk[3] += kTimedEvery * (int64_t)(now_ticks() - tp);
+      if (key_val(key) >= 0) { haveList = false; continue; }
       ++minor;
     } else {
+      // (candidate sweeps are few and all timed)
+      const bool timed = kCands || timed_pivot(done);
+      if (timed) tp = now_ticks();
       key = sweep_argmin<G, K>(C, t, S, shape, cands);
-      if (lead) S.tk[2] += (int64_t)(now_ticks() - tp);
+      if (timed && lead) S.tk[2] += (kCands ? 1 : kTimedEvery) * (int64_t)(now_ticks() - tp);
       ++sweeps;
       haveList = kCands;
       minor = 0;
@@ -1937,7 +1974,9 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
     }
     if (done >= budget) { status = 1; finished = true; break; }
     if (P.step_pivots > 0 && done >= P.step_pivots) break;
-    if (P.deadline && done > 0) {  // one decision for the whole group; >= 1 pivot per call
+    // one decision for the whole group, every fourth pivot (the clock, a barrier and, past
+    // the deadline, a read of the launch's counter); >= 1 pivot per call
+    if (P.deadline && done % 4 == 1) {
       if (lead)
         S.stop = now_ticks() >= P.deadline &&
                  (!P.busy || __hip_atomic_load(P.busy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0);
@@ -1954,16 +1993,17 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
           made = multi_pivot<G>(C, t, snL, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit);
         else
           made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit);
-        if (S.status != 0) { status = S.status; finished = true; break; }
+        if (made < 0) { status = 2; finished = true; break; }
         done = uniform(done + made);
         if (sw && made < 10) mode = 1;
         continue;
       }
     }
     const int ei = cell_row(key), ej = cell_col(key);
-    if (kSnapLdsOnly || auxLds) pivot<G, (G < 1024)>(C, t, snL, S, ei, ej, key_val(key));
-    else pivot<G, (G < 1024)>(C, t, sn, S, ei, ej, key_val(key));
-    if (S.status != 0) { status = S.status; finished = true; break; }
+    bool ok;
+    if (kSnapLdsOnly || auxLds) ok = pivot<G, (G < 1024)>(C, t, snL, S, ei, ej, key_val(key), done);
+    else ok = pivot<G, (G < 1024)>(C, t, sn, S, ei, ej, key_val(key), done);
+    if (!ok) { status = 2; finished = true; break; }
     ++done;
   }
   if (finished) {
@@ -2141,10 +2181,12 @@ __device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& g
       if (iter >= maxIt) { status = 1; finished = true; }
       else {
         const bool sw = P.pricing == 4;
-        const int done = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cand, iter, maxIt, sw ? 1 : P.minor_limit);
-        iter += done;
-        if (S.status != 0) { status = S.status; finished = true; }
-        if (sw && done < 10) mode = 1;
+        const int made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cand, 0,
+                                        maxIt - iter < 0x7fffffff ? (int)(maxIt - iter) : 0x7fffffff,
+                                        sw ? 1 : P.minor_limit);
+        if (made < 0) { status = 2; finished = true; }
+        else iter += made;
+        if (sw && made < 10) mode = 1;
       }
     }
   }
@@ -2153,15 +2195,18 @@ __device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& g
     for (;;) {
       if (iter >= maxIt) { status = 1; finished = true; break; }
       const int ei = cell_row(key), ej = cell_col(key);
-      if (auxLds) pivot<G, true>(C, t, snL, S, ei, ej, key_val(key));
-      else pivot<G, true>(C, t, sn, S, ei, ej, key_val(key));
-      if (S.status != 0) { status = S.status; finished = true; break; }
+      bool ok;
+      if (auxLds) ok = pivot<G, true>(C, t, snL, S, ei, ej, key_val(key), (int)iter);
+      else ok = pivot<G, true>(C, t, sn, S, ei, ej, key_val(key), (int)iter);
+      if (!ok) { status = 2; finished = true; break; }
       ++iter;
       if (!kCands || ++minor >= P.minor_limit) break;  // Dantzig: one pivot per sweep
-      const uint64_t tp = now_ticks();
-      key = group_min1_u64<G, 0>(reprice_set(C, t, cs), S);
-      if (lead) S.tk[3] += (int64_t)(now_ticks() - tp);
-      if (key == kNoKey || key_val(key) >= 0) break;  // list exhausted: next full sweep
+      const bool timed = timed_pivot((int)iter);
+      uint64_t tp = 0;
+      if (timed) tp = now_ticks();
+      key = group_min1_u64<G, 0>(reprice_set(t, cs), S);
+      if (timed && lead) S.tk[3] += kTimedEvery * (int64_t)(now_ticks() - tp);
+      if (key_val(key) >= 0) break;  // list exhausted: next full sweep
     }
   }
   if (finished) {

@@ -102,7 +102,8 @@ typedef struct flock_result {
   /* device time per phase in microseconds, measured inside the solving workgroup:
    * [0] transpose + Vogel, [1] tree build + duals, [2] full reduced-cost sweeps,
    * [3] candidate re-pricing, [4] pivot cycle discovery + leaving arc,
-   * [5] pivot flow update + subtree re-rooting (incremental duals) */
+   * [5] pivot flow update + subtree re-rooting (incremental duals).  [3] to [5], and [2]
+   * where every pivot has its sweep, are sampled: every eighth pivot, counted eight times */
   double phase_us[6];
   /* batches: device-clock microseconds from the start of the batch launch until this
    * instance's solve started / finished (its latency inside the batch) */
