@@ -187,6 +187,26 @@ __device__ __forceinline__ int64_t wave_sum_i64(int64_t x) {
   return (int64_t)wave_reduce_u64((uint64_t)x, 0ull, AddU64{});
 }
 
+// Halfword-wise unsigned minimum.
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t min_u16x2(uint32_t a, uint32_t b) {
+  u16x2 x, y;
+  __builtin_memcpy(&x, &a, 4);
+  __builtin_memcpy(&y, &b, 4);
+  const u16x2 r = __builtin_elementwise_min(x, y);
+  uint32_t o;
+  __builtin_memcpy(&o, &r, 4);
+  return o;
+}
+// LDS words that one rank stores while others load them and drop the value (plain ds_read
+// and ds_write; the memory model asks for atomics there).
+__device__ __forceinline__ int32_t lds_load(const int32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void lds_store(int32_t* p, int32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 // Workgroup reductions.  `red` is an LDS array of at least T/64 + 1 entries.  The
 // result slot is written only after a barrier that every wave passes after reading the
 // previous result, so back-to-back calls on the same `red` are safe.

@@ -66,10 +66,9 @@ struct Shared {
   int32_t idx;
   int32_t stop;       // deadline reached (rank 0 decides, the group follows)
   int32_t pad0_[2];
-  int32_t cnt2;       // Vogel: column refresh list counter (cnt: rows)
-  int32_t lastx;      // Vogel: the line covered by the previous step
+  int32_t cnt2;       // Vogel, register mode: list count of the odd steps (cnt: the even ones)
   int32_t dlo[2];     // pivot: least depth of a cycle vertex (atomicMin), by pivot parity
-  int32_t pad_[6];
+  int32_t pad_[7];
   uint64_t red1[3][16];  // one-barrier reductions (group_min1 / group_max1), by buffer
 };
 
@@ -95,6 +94,12 @@ template <int G, int kBuf>
 __device__ __forceinline__ uint64_t group_max1_u64(uint64_t x, Shared& S) {
   if constexpr (G == kWave) return wave_max_u64(x);
   else return block_max1_u64<G>(x, S.red1[kBuf]);
+}
+// The same max on buffer 0 or 2 in turn, for a loop with no other barrier.
+template <int G>
+__device__ __forceinline__ uint64_t group_max_alt(uint64_t x, Shared& S, int odd) {
+  if constexpr (G == kWave) return wave_max_u64(x);
+  else return block_max1_u64<G>(x, S.red1[2 * odd]);
 }
 template <int G>
 __device__ __forceinline__ int64_t group_sum_i64(int64_t x, Shared& S) {
@@ -364,7 +369,6 @@ template <class TRK>
 __device__ __forceinline__ void wave_line_track(gcint* data, int len, const uint8_t* crossCov, int lane, int b,
                                                 TRK* out, uint8_t* nt, uint32_t& k1, uint32_t& k2) {
   uint32_t l[kTrack] = {~0u, ~0u, ~0u, ~0u};
-  uint32_t cnt = 0;
   constexpr int U = 4;
   if (len <= U * kWave) {  // short line: one scalar load per lane and slot
 #pragma unroll
@@ -373,7 +377,6 @@ __device__ __forceinline__ void wave_line_track(gcint* data, int len, const uint
       const int32_t c = data[j < len ? j : 0];
       const bool live = j < len && !crossCov[j < len ? j : 0];
       track_insert(live ? (((uint32_t)c << b) | (uint32_t)j) : ~0u, l);  // ~0u inserts nothing
-      cnt += live ? 1u : 0u;
     }
   }
   const int nvec = len > U * kWave ? (len + 3) >> 2 : 0;
@@ -397,11 +400,9 @@ __device__ __forceinline__ void wave_line_track(gcint* data, int len, const uint
         const int j = j0 + e;
         const bool live = j < len && ((f[u] >> (8 * e)) & 0xffu) == 0;
         track_insert(live ? (((uint32_t)cc[e] << b) | (uint32_t)j) : ~0u, l);
-        cnt += live ? 1u : 0u;
       }
     }
   }
-  const uint32_t total = wave_sum_u32(cnt);
   // the kTrack smallest of the wave: every lane holds its own kTrack smallest, so
   // kTrack rounds of (wave min, the owner pops it) find them in order (keys are unique)
   uint32_t got[kTrack];
@@ -411,10 +412,12 @@ __device__ __forceinline__ void wave_line_track(gcint* data, int len, const uint
     got[e] = mn;
     if (l[0] == mn && mn != ~0u) { l[0] = l[1]; l[1] = l[2]; l[2] = l[3]; l[3] = ~0u; }
   }
+  const bool more = __ballot(l[0] != ~0u) != 0;  // a further uncovered cell in some lane
   if (lane == 0) {
+    int found = 0;
 #pragma unroll
-    for (int e = 0; e < kTrack; ++e) out[e] = got[e];
-    *nt = (uint8_t)((total < (uint32_t)kTrack ? total : (uint32_t)kTrack) | (total <= (uint32_t)kTrack ? kTrackFull : 0));
+    for (int e = 0; e < kTrack; ++e) { out[e] = got[e]; found += got[e] != ~0u ? 1 : 0; }
+    *nt = (uint8_t)(found | (more ? 0 : kTrackFull));
   }
   k1 = got[0]; k2 = got[1];
 }
@@ -492,169 +495,175 @@ __device__ __forceinline__ void wave_book_track(gcshort* book, gcint* data, int 
   k2 = wave_min_u32(r1);
 }
 
+// Minimum over the lanes of each 16-lane row, in the row's lane 15.
+__device__ __forceinline__ uint32_t row_min_u32(uint32_t x) {
+  MaxU32 op;
+  x = ~x;
+  x = op(x, dpp_u32<0x111, 0xf>(0u, x));
+  x = op(x, dpp_u32<0x112, 0xf>(0u, x));
+  x = op(x, dpp_u32<0x114, 0xf>(0u, x));
+  x = op(x, dpp_u32<0x118, 0xf>(0u, x));
+  return ~x;
+}
+
+// Book read of four lines by one wavefront, a 16-lane row each: as wave_book_track, 16
+// entries per ballot.  line: the row's line (its row's lanes agree), active: whether the row
+// has one.  k1/k2 are valid in the row's lane 15.
+template <class TRK>
+__device__ __forceinline__ void row_book_track(gcshort* book, gcint* data, int len, int16_t* pos, const uint8_t* crossCov,
+                                               int lane, int b, bool active, TRK* out, uint8_t* nt, uint32_t& k1,
+                                               uint32_t& k2) {
+  const int shift = lane & ~15, sl = lane & 15;
+  int at = *pos, found = 0, first = -1;
+  uint32_t r0 = ~0u, r1 = ~0u;
+  for (;;) {
+    const bool on = active && at < len && found <= kTrack;
+    if (__ballot(on) == 0) break;
+    const int q = at + sl;
+    const bool in = on && q < len;
+    const int idx = in ? book[q] : 0;
+    const int32_t cst = data[idx];
+    const bool live = in && !crossCov[idx];
+    const uint32_t mask = (uint32_t)(__ballot(live) >> shift) & 0xffffu;
+    if (on && first < 0 && mask) first = at + __ffsll((unsigned long long)mask) - 1;
+    if (live) {
+      const int rank = found + __popcll((unsigned long long)(mask & ((1u << sl) - 1u)));
+      const uint32_t key = ((uint32_t)cst << b) | (uint32_t)idx;
+      if (rank < kTrack) out[rank] = key;
+      if (rank == 0) r0 = key;
+      if (rank == 1) r1 = key;
+    }
+    if (on) { found += __popcll((unsigned long long)mask); at += 16; }
+  }
+  if (active && sl == 0) {
+    *pos = (int16_t)(first >= 0 ? first : len);
+    *nt = (uint8_t)((found < kTrack ? found : kTrack) | (found <= kTrack ? kTrackFull : 0));
+  }
+  k1 = row_min_u32(r0);
+  k2 = row_min_u32(r1);
+}
+
 // Vogel's LDS state (aliases the tree and aux regions): cover flags, residuals,
 // penalties, the scan list, per-line tracked count/flag and book position; the tracked
 // keys (kTrack per line, 16 bytes) follow in LDS when they fit, else they live in the
 // instance's global scratch.
 __host__ __device__ inline size_t vogel_trk_bytes(int m, int n) { return align16(16 * (size_t)(m + n)); }
 
-// KL > 0 (register mode): each rank keeps its (at most KL) lines' tracked keys, counts,
-// dirty flags and argmax keys in registers, so a step touches LDS only for the few lines
-// whose tracked keys met the line covered last (dirty lines) and for scans; the tracked
-// keys in `trk` are read only after the first pass and after scans, so they may live in
-// global memory.  KL = 0: every step walks every line's state in LDS.
-constexpr int kRegLines = 4;       // lines per rank of the work-queue engines
-constexpr int kRegLinesWide = 8;   // lines per rank of the large-instance set-up kernel
-template <int G, class TRK, int KL>
-__device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* demand, char* base, TRK* trk, Shared& S, gint* brow,
+// Vogel's line state in LDS (or global memory), carved from `base`.  kPen: the scan mode's
+// penalties (the register mode's live in its ranks' registers).
+struct VogelState {
+  uint8_t *covR, *covC;  // cover flags
+  int32_t* res;          // residual supplies, then demands
+  int32_t* pen;
+  int16_t* list;         // lines to scan
+  uint8_t* nt;           // tracked count and full flag of a line
+  int16_t* bpos;         // book read positions
+};
+template <bool kPen>
+__device__ __forceinline__ VogelState vogel_state(const Ctx& C, char* base) {
+  const int m = C.m, n = C.n, V = C.V;
+  VogelState st;
+  size_t off = 0;
+  st.covR = (uint8_t*)(base + off); off += align16((size_t)((m + 3) & ~3));
+  st.covC = (uint8_t*)(base + off); off += align16((size_t)((n + 3) & ~3));
+  st.res = (int32_t*)(base + off); off += align16(4 * (size_t)V);
+  st.pen = kPen ? (int32_t*)(base + off) : nullptr;
+  if (kPen) off += align16(4 * (size_t)V);
+  st.list = (int16_t*)(base + off); off += align16(2 * (size_t)V);
+  st.nt = (uint8_t*)(base + off); off += align16((size_t)V);
+  st.bpos = (int16_t*)(base + off);
+  return st;
+}
+
+// First pass without books: the kTrack smallest keys of every line, one rank per line,
+// read from the opposite-major copy (row L is column L of the transpose), so the lanes of
+// a wavefront read consecutive addresses and each rank keeps its own top keys with no
+// cross-lane reduction.  Every cell is uncovered at step 0.
+template <int G, class TRK>
+__device__ __forceinline__ void vogel_first_pass(const Ctx& C, TRK* trk, uint8_t* nt, int bRow, int bCol) {
+  const int m = C.m, n = C.n, V = C.V, tid = grank<G>();
+  constexpr int U = 16;  // loads in flight per rank
+  for (int L = tid; L < V; L += G) {
+    const bool row = L < m;
+    gcint* lbase = row ? (gcint*)C.costT + L : C.cost + (L - m);
+    const uint32_t stride = (uint32_t)(row ? C.ldT : C.ld);
+    const int len = row ? n : m;
+    const int b = row ? bRow : bCol;
+    uint32_t l[kTrack] = {~0u, ~0u, ~0u, ~0u};
+    for (int k0 = 0; k0 < len; k0 += U) {
+      int32_t c[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u < len ? k0 + u : len - 1;
+        c[u] = lbase[(uint32_t)k * stride];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u;
+        track_insert(k < len ? (((uint32_t)c[u] << b) | (uint32_t)k) : ~0u, l);  // ~0u inserts nothing
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kTrack; ++e) trk[4 * L + e] = l[e];
+    nt[L] = (uint8_t)((len < kTrack ? len : kTrack) | (len <= kTrack ? kTrackFull : 0));
+  }
+}
+
+// The first minimum uncovered cell of line Lc, by the whole group, as (cost, cross index);
+// kNoKey when every cross line is covered.
+template <int G>
+__device__ __forceinline__ uint64_t vogel_search(const Ctx& C, int Lc, const VogelState& st, Shared& S, gcshort* books) {
+  const int m = C.m, n = C.n, tid = grank<G>();
+  const uint8_t* cross = Lc < m ? st.covC : st.covR;
+  gcint* data = Lc < m ? C.cost + (uint32_t)(Lc * C.ld) : C.costT + (uint32_t)((Lc - m) * C.ldT);
+  const int len = Lc < m ? n : m;
+  uint64_t mk = kNoKey;
+  if (books) {  // first uncovered book entry from the line's read position on
+    gcshort* book = books + (Lc < m ? (size_t)Lc * n : (size_t)m * n + (size_t)(Lc - m) * m);
+    for (int at = st.bpos[Lc]; at < len; at += G) {
+      const int q = at + tid;
+      uint64_t f = kNoKey;
+      if (q < len) { const int j = book[q]; if (!cross[j]) f = (uint64_t)q; }
+      f = group_min_u64<G>(f, S);
+      if (f != kNoKey) { const int j = book[(int)f]; mk = pack_vi(data[j], (uint32_t)j); break; }
+    }
+  } else {
+    for (int j = tid; j < len; j += G)
+      if (!cross[j]) { const uint64_t k = pack_vi(data[j], (uint32_t)j); mk = k < mk ? k : mk; }
+    mk = group_min_u64<G>(mk, S);
+  }
+  return mk;
+}
+
+// Scan mode: every step walks every line's state (instances with more lines than the
+// register mode takes, and line state in global memory).
+template <int G, class TRK>
+__device__ __forceinline__ void vogel_scan(const Ctx& C, gcint* supply, gcint* demand, char* base, TRK* trk, Shared& S, gint* brow,
                           gint* bcol, gint* bflow, gcshort* books) {
   const int m = C.m, n = C.n, V = C.V, tid = grank<G>();
   const int lane = tid % kWave, wave = tid / kWave;
   constexpr int W = G / kWave;
-  constexpr bool kReg = KL > 0;
-  constexpr int kRL = KL > 0 ? KL : 1;  // register slots (one unused slot when KL = 0)
-  size_t off = 0;
-  uint8_t* covR = (uint8_t*)(base + off); off += align16((size_t)((m + 3) & ~3));
-  uint8_t* covC = (uint8_t*)(base + off); off += align16((size_t)((n + 3) & ~3));
-  int32_t* res = (int32_t*)(base + off); off += align16(4 * (size_t)V);
-  // penalties are kept in LDS by the scan mode only (the register mode's are in the keys)
-  int32_t* pen = kReg ? nullptr : (int32_t*)(base + off);
-  if (!kReg) off += align16(4 * (size_t)V);
-  int16_t* list = (int16_t*)(base + off); off += align16(2 * (size_t)V);
-  uint8_t* nt = (uint8_t*)(base + off); off += align16((size_t)V);
-  int16_t* bpos = (int16_t*)(base + off);  // book read positions
+  const VogelState st = vogel_state<true>(C, base);
+  uint8_t *covR = st.covR, *covC = st.covC, *nt = st.nt;
+  int32_t *res = st.res, *pen = st.pen;
+  int16_t *list = st.list, *bpos = st.bpos;
   const int bRow = index_bits(n), bCol = index_bits(m);  // rows track column indices and vice versa
 
   for (int L = tid; L < V; L += G) {
     res[L] = L < m ? supply[L] : demand[L - m];
-    if constexpr (!kReg) pen[L] = 0;
+    pen[L] = 0;
     nt[L] = 0; bpos[L] = 0;  // with books nothing is tracked: every line is read at step 0
     if (L < m) covR[L] = 0; else covC[L - m] = 0;
   }
-  if (!books) {
-    // First pass without books: the kTrack smallest keys of every line, one rank per
-    // line, read from the opposite-major copy (row L is column L of the transpose), so
-    // the lanes of a wavefront read consecutive addresses and each rank keeps its own
-    // top keys with no cross-lane reduction.  Every cell is uncovered at step 0.
-    constexpr int U = 16;  // loads in flight per rank
-    for (int L = tid; L < V; L += G) {
-      const bool row = L < m;
-      gcint* lbase = row ? (gcint*)C.costT + L : C.cost + (L - m);
-      const uint32_t stride = (uint32_t)(row ? C.ldT : C.ld);
-      const int len = row ? n : m;
-      const int b = row ? bRow : bCol;
-      uint32_t l[kTrack] = {~0u, ~0u, ~0u, ~0u};
-      for (int k0 = 0; k0 < len; k0 += U) {
-        int32_t c[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int k = k0 + u < len ? k0 + u : len - 1;
-          c[u] = lbase[(uint32_t)k * stride];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int k = k0 + u;
-          track_insert(k < len ? (((uint32_t)c[u] << b) | (uint32_t)k) : ~0u, l);  // ~0u inserts nothing
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < kTrack; ++e) trk[4 * L + e] = l[e];
-      nt[L] = (uint8_t)((len < kTrack ? len : kTrack) | (len <= kTrack ? kTrackFull : 0));
-    }
-  }
-  if (tid == 0) { S.pend_row = 1; S.pend_col = 1; S.cnt = 0; S.lastx = -1; }
+  if (!books) vogel_first_pass<G>(C, trk, nt, bRow, bCol);
+  if (tid == 0) { S.pend_row = 1; S.pend_col = 1; S.cnt = 0; }
   int covCols = 0;  // columns covered so far (only rank 0 eliminates, so only its copy counts)
-  // register state of this rank's lines L = tid + u*G (kReg): tracked keys, argmax key,
-  // and one word of flags -- tracked count (bits 0-2), full (3), dirty (4), covered (5),
-  // listed for a scan (6)
-  constexpr uint32_t fFull = 8, fDirty = 16, fCov = 32, fNeed = 64;
-  uint32_t rk[kRL][4];
-  uint32_t rf[kRL];
-  uint64_t rkey[kRL];
-  if constexpr (kReg) {
-#pragma unroll
-    for (int u = 0; u < kRL; ++u) {
-      const int L = tid + u * G;
-      rk[u][0] = rk[u][1] = rk[u][2] = rk[u][3] = ~0u;
-      rf[u] = fDirty | (L >= V ? fCov : 0u);
-      rkey[u] = (uint64_t)(uint32_t)L << 18;
-      if (!books && L < V) {  // the first pass tracked this rank's line: clean, with its key
-        const u32x4 tk = *(const u32x4*)(trk + 4 * L);
-        const uint8_t ntl = nt[L];
-        const int cnt = ntl & 0x7f;
-        const int b = L < m ? bRow : bCol;
-        rk[u][0] = tk.x; rk[u][1] = tk.y; rk[u][2] = tk.z; rk[u][3] = tk.w;
-        rf[u] = (uint32_t)cnt | ((ntl & kTrackFull) ? fFull : 0u);
-        const uint32_t k1 = cnt > 0 ? tk.x : ~0u, k2 = cnt > 1 ? tk.y : ~0u;
-        rkey[u] = ((uint64_t)(uint32_t)(key_penalty(k1, k2, b) + 1) << 32) | ((uint64_t)(uint32_t)L << 18) |
-                  (k1 != ~0u ? ((1u << 17) | (k1 & ((1u << b) - 1u))) : 0u);
-      }
-    }
-  }
   gsync<G>();
 
   for (int step = 0; step < V - 1; ++step) {
     const bool pendR = S.pend_row != 0, pendC = S.pend_col != 0;
     uint64_t best = 0;
-    if constexpr (kReg) {
-      // the line covered by the previous step: its own rank marks it, ranks whose lines
-      // tracked it mark those dirty and move their first uncovered cell on if it was it
-      const int X = S.lastx;
-      const bool xRow = X >= 0 && X < m;
-      const uint32_t xIdx = X < 0 ? 0xffffu : (uint32_t)(xRow ? X : X - m);
-      // the rank index, opaque to the compiler here, so line numbers and the values
-      // derived from them are recomputed each step instead of being kept (spilled)
-      // across the whole Vogel loop
-      int tidr = tid;
-      asm volatile("" : "+v"(tidr));
-      const int wave0 = uniform(tid & ~(kWave - 1));  // this wavefront's first rank
-#pragma unroll
-      for (int u = 0; u < kRL; ++u) {
-        if (wave0 + u * G >= V) continue;  // uniform: the wavefront has no line in slot u
-        const int L = tidr + u * G;
-        const bool row = L < m;
-        const int b = row ? bRow : bCol;
-        const uint32_t mask = (1u << b) - 1u;
-        const bool isX = L == X;
-        rf[u] |= isX ? fCov : 0u;
-        rkey[u] = isX ? ((uint64_t)(uint32_t)L << 18) : rkey[u];  // penalty -1
-        const bool live = (rf[u] & fCov) == 0;
-        const int cnt = (int)(rf[u] & 7u);
-        bool hit = false;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) hit = hit | ((e < cnt) & ((rk[u][e] & mask) == xIdx));
-        hit = hit & live & (X >= 0) & (row != xRow);
-        rf[u] |= hit ? fDirty : 0u;
-        const bool refreshL = live & ((rf[u] & fDirty) != 0) & (row ? pendR : pendC);
-        const bool jcHit = hit & (((uint32_t)rkey[u] & 0x3ffffu) == ((1u << 17) | xIdx));
-        if (refreshL | jcHit) {  // few lines per step: walk the tracked keys against the flags
-          const uint8_t* cross = row ? covC : covR;
-          bool unc[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) unc[e] = (e < cnt) & (cross[e < cnt ? (rk[u][e] & mask) : 0] == 0);
-          const uint32_t* kk = rk[u];
-          const uint32_t k1 = unc[0] ? kk[0] : unc[1] ? kk[1] : unc[2] ? kk[2] : unc[3] ? kk[3] : ~0u;
-          const uint32_t a3 = unc[3] ? kk[3] : ~0u;
-          const uint32_t a2 = unc[2] ? kk[2] : a3;
-          const uint32_t a1 = unc[1] ? kk[1] : a2;
-          const uint32_t k2 = unc[0] ? a1 : unc[1] ? a2 : unc[2] ? a3 : ~0u;
-          const uint32_t jbits = k1 == ~0u ? 0u : ((1u << 17) | (k1 & mask));
-          if (refreshL) {
-            if ((k2 != ~0u) | ((rf[u] & fFull) != 0)) {
-              rkey[u] = ((uint64_t)(uint32_t)(key_penalty(k1, k2, b) + 1) << 32) | ((uint64_t)(uint32_t)L << 18) | jbits;
-              rf[u] &= ~fDirty;
-            } else {
-              rf[u] |= fNeed;
-              list[atomicAdd(&S.cnt, 1)] = (int16_t)L;
-            }
-          } else {  // penalty stays (stale kind); the first uncovered cell moves on
-            rkey[u] = (rkey[u] & ~0x3ffffull) | jbits;
-          }
-        }
-        best = ((rf[u] & fNeed) == 0 && L < V && rkey[u] > best) ? rkey[u] : best;
-      }
-    } else {
-      constexpr bool refresh = true;
+    {
       // kVB lines per rank at a time, every LDS load of a batch issued before first use
       constexpr int kVB = 4;
       for (int L0 = tid; L0 < V; L0 += kVB * G) {
@@ -701,7 +710,7 @@ __device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* de
           const uint32_t a2 = unc[2] ? kk[2] : a3;
           const uint32_t a1 = unc[1] ? kk[1] : a2;
           const uint32_t k2 = unc[0] ? a1 : unc[1] ? a2 : unc[2] ? a3 : ~0u;
-          const bool refreshL = refresh & !cov[u] & (row ? pendR : pendC);
+          const bool refreshL = !cov[u] & (row ? pendR : pendC);
           const bool resolved = (k2 != ~0u) | ((ntv[u] & kTrackFull) != 0);
           const bool need = refreshL & !resolved;
           const int32_t p = refreshL ? (resolved ? key_penalty(k1, k2, b) : 0) : pv[u];
@@ -738,9 +747,7 @@ __device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* de
         else
           wave_line_track(data, len, cross, lane, b, trk + 4 * L, &nt[L], k1, k2);
         const int32_t p = key_penalty(k1, k2, b);
-        if constexpr (!kReg) {
-          if (lane == 0) pen[L] = p;
-        }
+        if (lane == 0) pen[L] = p;
         const uint64_t k = ((uint64_t)(uint32_t)(p + 1) << 32) | ((uint64_t)(uint32_t)L << 18) |
                            (k1 != ~0u ? ((1u << 17) | (k1 & ((1u << b) - 1u))) : 0u);
         wbest = k > wbest ? k : wbest;
@@ -750,25 +757,6 @@ __device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* de
 #pragma unroll
       for (int w = 0; w < W; ++w) best = S.red1[1][w] > best ? S.red1[1][w] : best;
       if (tid == 0) S.cnt = 0;  // read above, before the barrier; next used after this step's last one
-      if constexpr (kReg) {  // scanned lines: fresh tracked keys (all uncovered) back to registers
-        int tidr = tid;  // opaque, as in the refresh above
-        asm volatile("" : "+v"(tidr));
-#pragma unroll
-        for (int u = 0; u < kRL; ++u) {
-          if ((rf[u] & fNeed) == 0) continue;
-          const int L = tidr + u * G;
-          const bool row = L < m;
-          const int b = row ? bRow : bCol;
-          const u32x4 tk = *(const u32x4*)(trk + 4 * L);
-          const uint8_t ntl = nt[L];
-          rk[u][0] = tk.x; rk[u][1] = tk.y; rk[u][2] = tk.z; rk[u][3] = tk.w;
-          const int cnt = ntl & 0x7f;
-          rf[u] = (uint32_t)cnt | ((ntl & kTrackFull) ? fFull : 0u);  // clean, not covered, not listed
-          const uint32_t k1 = cnt > 0 ? tk.x : ~0u, k2 = cnt > 1 ? tk.y : ~0u;
-          rkey[u] = ((uint64_t)(uint32_t)(key_penalty(k1, k2, b) + 1) << 32) | ((uint64_t)(uint32_t)L << 18) |
-                    (k1 != ~0u ? ((1u << 17) | (k1 & ((1u << b) - 1u))) : 0u);
-        }
-      }
     }
   decided:
     const int Lc = (int)((best >> 18) & 0x3fffu);
@@ -776,24 +764,7 @@ __device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* de
     if ((best >> 17) & 1u) {
       jc = (int)(best & 0x1ffffu);  // the line's first uncovered tracked key: its first minimum
     } else {  // nothing uncovered is tracked: search the line itself
-      const uint8_t* cross = Lc < m ? covC : covR;
-      gcint* data = Lc < m ? C.cost + (uint32_t)(Lc * C.ld) : C.costT + (uint32_t)((Lc - m) * C.ldT);
-      const int len = Lc < m ? n : m;
-      uint64_t mk = kNoKey;
-      if (books) {  // first uncovered book entry from the line's read position on
-        gcshort* book = books + (Lc < m ? (size_t)Lc * n : (size_t)m * n + (size_t)(Lc - m) * m);
-        for (int at = bpos[Lc]; at < len; at += G) {
-          const int q = at + tid;
-          uint64_t f = kNoKey;
-          if (q < len) { const int j = book[q]; if (!cross[j]) f = (uint64_t)q; }
-          f = group_min_u64<G>(f, S);
-          if (f != kNoKey) { const int j = book[(int)f]; mk = pack_vi(data[j], (uint32_t)j); break; }
-        }
-      } else {
-        for (int j = tid; j < len; j += G)
-          if (!cross[j]) { const uint64_t k = pack_vi(data[j], (uint32_t)j); mk = k < mk ? k : mk; }
-        mk = group_min_u64<G>(mk, S);
-      }
+      const uint64_t mk = vogel_search<G>(C, Lc, st, S, books);
       if (mk == kNoKey) {  // no uncovered cross line: cannot happen for a balanced instance
         if (tid == 0) S.status = 4;
         gsync<G>();
@@ -812,18 +783,235 @@ __device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* de
       int32_t f;
       if (coverRow) {
         f = rs; res[m + q] = rd - rs; res[r] = 0; covR[r] = 1;
-        if constexpr (!kReg) pen[r] = -1;
+        pen[r] = -1;
       } else {
         f = rd; res[r] = rs - rd; res[m + q] = 0; covC[q] = 1;
-        if constexpr (!kReg) pen[m + q] = -1;
+        pen[m + q] = -1;
         ++covCols;
       }
       S.pend_row = coverRow ? 1 : 0;
       S.pend_col = coverRow ? 0 : 1;
-      S.lastx = coverRow ? r : m + q;
       brow[step] = r; bcol[step] = q; bflow[step] = f;
     }
     gsync<G>();
+  }
+}
+
+// Register mode: each rank keeps its (at most KL) lines' tracked keys, their cross lines
+// and the lines' penalties in registers.  A step compares the line covered last with the
+// tracked cross lines (packed 16-bit vertex numbers); a line that tracked it drops that
+// key, so the first two keys left are always its smallest uncovered ones and no cover flag
+// is read outside scans.  Its penalty is refreshed when its kind is pending (the stale
+// rule) and, with fewer than two keys left of a longer line, the line is listed for a scan.
+// Every rank follows the elimination itself from the two residuals, so a step has one
+// barrier, the argmax's: rank 0 writes a step's residuals back in the next step, after
+// that barrier, and meanwhile every rank takes those two from its registers; two buffers
+// alternate under the argmax.
+// Bound: the chain of a step (two wavefront minima, barrier, residuals) and its vector
+// instructions, about 20 a line slot.  The former step (cover flags re-read for every
+// touched line, rank 0 eliminating between two barriers, 320 vector instructions at four
+// slots) took 2.0 us at 500x480 on 256 threads and 2.4 us at 1000x1000 on 512; this one
+// takes 1.5 and 1.6 us, and 3.6 instead of 5.9 us at 4000x2000 on 1024.
+constexpr int kRegLines = 4;       // lines per rank of the work-queue engines
+constexpr int kRegLinesWide = 8;   // where m+n needs them, on 512 threads (and the set-up on 1024)
+template <int G, class TRK, int KL>
+__device__ __forceinline__ void vogel_reg(const Ctx& C, gcint* supply, gcint* demand, char* base, TRK* trk, Shared& S,
+                                          gint* brow, gint* bcol, gint* bflow, gcshort* books) {
+  const int m = C.m, n = C.n, V = C.V, tid = grank<G>();
+  const int lane = tid % kWave, wave = tid / kWave;
+  constexpr int W = G / kWave;
+  const VogelState st = vogel_state<false>(C, base);
+  const int bRow = index_bits(n), bCol = index_bits(m);  // rows track column indices and vice versa
+  for (int L = tid; L < V; L += G) {
+    st.res[L] = L < m ? supply[L] : demand[L - m];
+    st.nt[L] = 0; st.bpos[L] = 0;  // with books nothing is tracked: every line is read at step 0
+    if (L < m) st.covR[L] = 0; else st.covC[L - m] = 0;
+  }
+  if (!books) vogel_first_pass<G>(C, trk, st.nt, bRow, bCol);
+  if (tid == 0) { S.cnt = 0; S.cnt2 = 0; }
+  // per line L = tid + u*G: tracked keys (~0u: none), their cross vertices (0xffff: none),
+  // penalty + 1 (0: covered, listed or past V), flags: dirty row / dirty column, all
+  // uncovered cells tracked
+  constexpr uint32_t fFull = 4;
+  uint32_t l[KL][4], id01[KL], id23[KL], pen1[KL], fl[KL];
+  auto penalty1 = [&](uint32_t k1, uint32_t k2, int b) { return (uint32_t)key_penalty(k1, k2, b) + 1u; };
+  // a freshly tracked line (all keys uncovered, clean)
+  auto load_line = [&](int u, int L) {
+    const u32x4 tk = *(const u32x4*)(trk + 4 * L);
+    const uint32_t ntl = st.nt[L];
+    const int cnt = (int)(ntl & 0x7fu);
+    const bool row = L < m;
+    const int b = row ? bRow : bCol;
+    const uint32_t mask = (1u << b) - 1u, base0 = row ? (uint32_t)m : 0u;  // first cross vertex
+    l[u][0] = cnt > 0 ? tk.x : ~0u; l[u][1] = cnt > 1 ? tk.y : ~0u;
+    l[u][2] = cnt > 2 ? tk.z : ~0u; l[u][3] = cnt > 3 ? tk.w : ~0u;
+    uint32_t id[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) id[e] = e < cnt ? (l[u][e] & mask) + base0 : 0xffffu;
+    id01[u] = id[0] | (id[1] << 16); id23[u] = id[2] | (id[3] << 16);
+    fl[u] = (ntl & kTrackFull) ? fFull : 0u;
+    pen1[u] = penalty1(l[u][0], l[u][1], b);
+  };
+#pragma unroll
+  for (int u = 0; u < KL; ++u) {
+    const int L = tid + u * G;
+    l[u][0] = l[u][1] = l[u][2] = l[u][3] = ~0u;
+    id01[u] = id23[u] = ~0u;
+    pen1[u] = 0;
+    fl[u] = L >= V ? 0u : L < m ? 1u : 2u;
+    if (!books && L < V) load_line(u, L);
+  }
+  // the line covered last, the pending kinds (1 rows, 2 columns) and the last step's cell
+  // with its new residuals: the same in every rank
+  int X = 0xfffe, pr = -1, pq = -1, covCols = 0;
+  uint32_t pend = 3;
+  int32_t prs = 0, prd = 0;
+  gsync<G>();
+
+  for (int step = 0; step < V - 1; ++step) {
+    // the rank index, opaque to the compiler here, so line numbers are recomputed each step
+    // instead of being kept (spilled) across the whole loop
+    int tidr = tid;
+    asm volatile("" : "+v"(tidr));
+    const int wave0 = uniform(tid & ~(kWave - 1));  // this wavefront's first rank
+    const uint32_t xx = (uint32_t)X | ((uint32_t)X << 16);
+    // a rank may list lines of the next step before another has read this step's count
+    int32_t* listed = step & 1 ? &S.cnt2 : &S.cnt;
+    uint32_t bpen = 0, bkey = ~0u;
+    int bL = tidr;
+#pragma unroll
+    for (int u = 0; u < KL; ++u) {
+      if (wave0 + u * G >= V) continue;  // uniform: the wavefront has no line in slot u
+      const int L = tidr + u * G;
+      const uint32_t d01 = id01[u] ^ xx, d23 = id23[u] ^ xx;
+      const uint32_t d = min_u16x2(d01, d23);
+      const bool hit = ((d - 0x00010001u) & ~d & 0x80008000u) != 0;  // a zero half: X is tracked
+      if (hit | (L == X) | ((fl[u] & pend) != 0)) {  // few lines per step
+        if (L == X) {
+          pen1[u] = 0; id01[u] = id23[u] = ~0u; fl[u] = 0;
+        } else {
+          const bool row = L < m;
+          if (hit) {  // drop that key
+            const bool h0 = (d01 & 0xffffu) == 0, h1 = h0 | (d01 < 0x10000u), h2 = h1 | ((d23 & 0xffffu) == 0);
+            l[u][0] = h0 ? l[u][1] : l[u][0];
+            l[u][1] = h1 ? l[u][2] : l[u][1];
+            l[u][2] = h2 ? l[u][3] : l[u][2];
+            l[u][3] = ~0u;
+            const uint32_t i1 = id01[u] >> 16, i2 = id23[u] & 0xffffu, i3 = id23[u] >> 16;
+            const uint32_t j0 = h0 ? i1 : (id01[u] & 0xffffu);
+            id01[u] = j0 | ((h1 ? i2 : i1) << 16);
+            id23[u] = (h2 ? i3 : i2) | 0xffff0000u;
+            fl[u] |= row ? 1u : 2u;
+          }
+          if (fl[u] & pend) {
+            if ((l[u][1] != ~0u) | ((fl[u] & fFull) != 0)) {
+              pen1[u] = penalty1(l[u][0], l[u][1], row ? bRow : bCol);
+            } else {
+              pen1[u] = 0;
+              st.list[atomicAdd(listed, 1)] = (int16_t)L;
+              fl[u] |= 8u;  // listed
+            }
+            fl[u] &= ~3u;
+          }
+        }
+      }
+      const bool better = pen1[u] >= bpen;  // the last maximum
+      bpen = better ? pen1[u] : bpen;
+      bkey = better ? l[u][0] : bkey;
+      bL = better ? L : bL;
+    }
+    auto argmax_key = [&](uint32_t p1, int L, uint32_t k1) {
+      const uint32_t mask = (1u << (L < m ? bRow : bCol)) - 1u;
+      return ((uint64_t)p1 << 32) | ((uint64_t)(uint32_t)L << 18) | (k1 != ~0u ? ((1u << 17) | (k1 & mask)) : 0u);
+    };
+    uint64_t best = group_max_alt<G>(argmax_key(bpen, bL, bkey), S, step & 1);
+    // lines to scan (the count was published by the atomics before the max's barrier);
+    // uniform: every rank reads the same count
+    const int cnt = uniform(*listed);
+    if (cnt != 0) {
+      // one wavefront per listed line; each wavefront's max key of its lines is combined
+      // with the max above through buffer 1 (idle outside pivots)
+      uint64_t wbest = 0;
+      if (books && cnt > W) {
+        // more lines than wavefronts: four at a time (equal costs let one covered column
+        // list hundreds of rows; 4000x2000 with costs 1..8 scans 55 lines a step)
+        for (int e0 = 4 * wave; e0 < cnt; e0 += 4 * W) {
+          const int e = e0 + (lane >> 4);
+          const bool active = e < cnt;
+          const int L = st.list[active ? e : e0];
+          const bool row = L < m;
+          const int b = row ? bRow : bCol;
+          uint32_t k1, k2;
+          row_book_track(books + (row ? (size_t)L * n : (size_t)m * n + (size_t)(L - m) * m),
+                         row ? C.cost + (uint32_t)(L * C.ld) : (gcint*)(C.costT + (uint32_t)((L - m) * C.ldT)),
+                         row ? n : m, &st.bpos[L], row ? st.covC : st.covR, lane, b, active, trk + 4 * L, &st.nt[L],
+                         k1, k2);
+          const uint64_t k = argmax_key(penalty1(k1, k2, b), L, k1);
+          if (active && (lane & 15) == 15) wbest = k > wbest ? k : wbest;
+        }
+        wbest = wave_max_u64(wbest);
+      } else
+      for (int e = wave; e < cnt; e += W) {
+        const int L = st.list[e];
+        if (L < 0 || L >= V) continue;  // guard: list entries are lines
+        const bool row = L < m;
+        gcint* data = row ? C.cost + (uint32_t)(L * C.ld) : C.costT + (uint32_t)((L - m) * C.ldT);
+        const int len = row ? n : m;
+        const int b = row ? bRow : bCol;
+        const uint8_t* cross = row ? st.covC : st.covR;
+        uint32_t k1, k2;
+        if (books)
+          wave_book_track(books + (row ? (size_t)L * n : (size_t)m * n + (size_t)(L - m) * m), data, len, &st.bpos[L],
+                          cross, lane, b, trk + 4 * L, &st.nt[L], k1, k2);
+        else
+          wave_line_track(data, len, cross, lane, b, trk + 4 * L, &st.nt[L], k1, k2);
+        const uint64_t k = argmax_key(penalty1(k1, k2, b), L, k1);
+        wbest = k > wbest ? k : wbest;
+      }
+      if (lane == 0) S.red1[1][wave] = wbest;
+      gsync<G>();
+#pragma unroll
+      for (int w = 0; w < W; ++w) best = S.red1[1][w] > best ? S.red1[1][w] : best;
+      if (tid == 0) *listed = 0;  // read by every rank before the barrier
+      int tids = tid;  // opaque, as above
+      asm volatile("" : "+v"(tids));
+#pragma unroll
+      for (int u = 0; u < KL; ++u)
+        if (fl[u] & 8u) load_line(u, tids + u * G);
+      // no barrier closes the scan: the list, the tracked keys and buffer 1 are written
+      // again only after the next step's argmax barrier, this count two steps on
+    }
+    const int Lc = (int)((best >> 18) & 0x3fffu);
+    int jc;
+    if ((best >> 17) & 1u) {
+      jc = (int)(best & 0x1ffffu);  // the line's first uncovered tracked key: its first minimum
+    } else {  // nothing uncovered is tracked: search the line itself
+      const uint64_t mk = vogel_search<G>(C, Lc, st, S, books);
+      if (mk == kNoKey) {  // no uncovered cross line: cannot happen for a balanced instance
+        if (tid == 0) S.status = 4;
+        gsync<G>();
+        return;
+      }
+      jc = (int)key_idx(mk);
+      // every rank has read the cover flags for the search before rank 0 changes them
+      gsync<G>();
+    }
+    const int r = Lc < m ? Lc : jc, q = Lc < m ? jc : Lc - m;
+    const int32_t lr = lds_load(&st.res[r]), lq = lds_load(&st.res[m + q]);
+    const int32_t rs = r == pr ? prs : lr, rd = q == pq ? prd : lq;
+    bool coverRow = rd > rs;
+    coverRow = coverRow | (covCols == n - 1);
+    if (tid == 0) {
+      if (pr >= 0) { lds_store(&st.res[pr], prs); lds_store(&st.res[m + pq], prd); }
+      if (coverRow) st.covR[r] = 1; else st.covC[q] = 1;  // next read by a scan, after a barrier
+      brow[step] = r; bcol[step] = q; bflow[step] = coverRow ? rs : rd;
+    }
+    pr = r; pq = q;
+    prs = coverRow ? 0 : rs - rd;
+    prd = coverRow ? rd - rs : 0;
+    X = coverRow ? r : m + q;
+    pend = coverRow ? 1u : 2u;
+    covCols += coverRow ? 0 : 1;
   }
 }
 
@@ -833,9 +1021,8 @@ __device__ __forceinline__ void vogel_run(const Ctx& C, gcint* supply, gcint* de
 // gstate: global memory of at least vogel_lds_bytes for the line state when even that
 // does not fit the `avail` LDS bytes at `base` (large-instance path with the tree in
 // global memory); null otherwise.
-// kWide: also instantiate the register mode with kRegLinesWide lines per rank (the
-// large-instance set-up kernel, which has registers to spare), for m+n up to
-// kRegLinesWide * G, with the tracked keys in LDS or in global scratch.
+// kWide: also instantiate the register mode with kRegLinesWide lines per rank, with the
+// tracked keys in LDS or in global scratch.
 template <int G, bool kWide = false>
 __device__ __forceinline__ void vogel(const Ctx& C, gcint* supply, gcint* demand, char* base, size_t avail, Shared& S, gint* brow,
                       gint* bcol, gint* bflow, int32_t* scratch, gcshort* books = nullptr, char* gstate = nullptr) {
@@ -849,21 +1036,21 @@ __device__ __forceinline__ void vogel(const Ctx& C, gcint* supply, gcint* demand
   if ((regLines || regWide) && needR + trkBytes <= avail) {  // register mode, tracked keys in LDS
     LdsTrk* trk = (LdsTrk*)(base + needR);
     if (regLines) {
-      vogel_run<G, LdsTrk, kRegLines>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
+      vogel_reg<G, LdsTrk, kRegLines>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
     } else {
-      if constexpr (kWide) vogel_run<G, LdsTrk, kRegLinesWide>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
+      if constexpr (kWide) vogel_reg<G, LdsTrk, kRegLinesWide>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
     }
   } else if (!regLines && !regWide && need + trkBytes <= avail) {  // scan mode, tracked keys in LDS
-    vogel_run<G, LdsTrk, 0>(C, supply, demand, base, (LdsTrk*)(base + need), S, brow, bcol, bflow, books);
+    vogel_scan<G, LdsTrk>(C, supply, demand, base, (LdsTrk*)(base + need), S, brow, bcol, bflow, books);
   } else if (need <= avail) {
     GlTrk* trk = (GlTrk*)scratch;
-    if (kWide && C.V <= kRegLinesWide * G) {
-      if constexpr (kWide) vogel_run<G, GlTrk, kRegLinesWide>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
+    if (regWide) {
+      if constexpr (kWide) vogel_reg<G, GlTrk, kRegLinesWide>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
     } else {
-      vogel_run<G, GlTrk, 0>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
+      vogel_scan<G, GlTrk>(C, supply, demand, base, trk, S, brow, bcol, bflow, books);
     }
   } else if (gstate) {
-    vogel_run<G, GlTrk, 0>(C, supply, demand, gstate, (GlTrk*)scratch, S, brow, bcol, bflow, books);
+    vogel_scan<G, GlTrk>(C, supply, demand, gstate, (GlTrk*)scratch, S, brow, bcol, bflow, books);
   } else {  // the host sizes LDS so that this cannot happen; report instead of overrunning it
     if (grank<G>() == 0) S.status = 6;
     gsync<G>();

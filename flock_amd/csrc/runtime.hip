@@ -623,7 +623,11 @@ struct LargeRunner {
       P.tree_global = 1;
     }
     const int threads = (g_large_threads == 512 && !P.tree_global && o.m + o.n <= kLargeSmallMaxV) ? 512 : 1024;
-    const void* const fsetup = threads == 512 ? setup_kernel_512 : setup_kernel_1024;
+    // the set-up takes 512 threads while its Vogel holds at most 8 lines a rank (1700x1500:
+    // 6.5 ms of Vogel against 7.2 on 1024 threads), else 1024, whose wavefronts scan twice
+    // the lines at a time (4000x2000 with equal supplies: 27 against 33 ms)
+    const int sthreads = !P.tree_global && o.m + o.n <= kRegLinesWide * 512 ? 512 : 1024;
+    const void* const fsetup = sthreads == 512 ? setup_kernel_512 : setup_kernel_1024;
     if (lds > 65536) {
       HIP_TRY(hipFuncSetAttribute(round_fn(threads, rule_of(P), P.tree_global != 0),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -655,7 +659,7 @@ struct LargeRunner {
       EngineParams Ps = P;
       Ps.lds_bytes = (int32_t)slds;
       void* args[] = {(void*)&di, (void*)&books, (void*)&Ps};
-      HIP_TRY(hipLaunchKernel(fsetup, dim3(1), dim3(threads), args, slds, g_stream));
+      HIP_TRY(hipLaunchKernel(fsetup, dim3(1), dim3(sthreads), args, slds, g_stream));
     }
     SweepArgs A = sweep_args(b.hdesc[0], keys, cands, vpt, &b.d_insts[0].phase);
     if ((st = graph(b.d_insts, b.hdesc[0], nblocks, A, P, lds, threads))) return st;

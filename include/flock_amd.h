@@ -220,7 +220,7 @@ typedef struct flock_tuning {
   /* large-instance path (graph of sweep grid and pivot rounds): the sweep tile's shape, in
    * 16-byte cost vectors per thread of a 256-thread tile (1..64; default 4) */
   int32_t sweep_vectors;
-  /* large-instance path: threads of the set-up and pivot-round workgroup, 512 or 1024
+  /* large-instance path: threads of the pivot-round workgroup, 512 or 1024
    * (512 applies to instances with m+n <= 2048 whose basis tree fits LDS) */
   int32_t large_threads;
   /* large-instance path: candidate pricing's minor iterations per full sweep (0: minor_limit) */

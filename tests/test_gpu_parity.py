@@ -234,6 +234,28 @@ def test_batch_packed_copies(sizes):
         assert np.array_equal(s.flow_list, np.stack([s.rows[pos], s.cols[pos], s.flows[pos]], axis=1))
 
 
+# Vogel's register mode: m+n at the edges of 4 and 8 lines per rank, with few distinct costs
+# (one covered line lists many others) and with many
+VOGEL_EDGES = [(64, 100, 156), (64, 100, 157), (256, 23, 1000), (256, 24, 1000), (256, 1000, 25), (512, 48, 2000),
+               (512, 49, 2000), (512, 96, 4000), (512, 97, 4000), (0, 170, 1878), (0, 130, 3966), (0, 130, 3967)]
+
+
+@pytest.mark.parametrize("threads,m,n", VOGEL_EDGES)
+@pytest.mark.parametrize("cmax", [3, 20000])
+def test_vogel_line_slots_exact(threads, m, n, cmax):
+    """The initial basis, slot by slot (after one Dantzig pivot on both sides), equals the
+    oracle's: integers, no tolerance."""
+    rng = np.random.default_rng(m + n + cmax)
+    inst = _rand(rng, m, n, cmax=cmax, smax=900, zeros=cmax == 3)
+    say("vogel edge", threads, m, n, cmax)
+    s = F.solve(inst, pricing="dantzig", threads=threads, max_iterations=1)
+    o = oracle.solve(inst.cost, inst.supply, inst.demand, max_iterations=1)
+    assert s.iterations == o.iterations
+    assert np.array_equal(s.rows, o.rows) and np.array_equal(s.cols, o.cols)
+    assert np.array_equal(s.flows.astype(np.int64), o.flows)
+    assert np.array_equal(s.u.astype(np.int64), o.u) and np.array_equal(s.v.astype(np.int64), o.v)
+
+
 def test_batch_mixed_configurations():
     """One batch mixing wavefront and workgroup classes, candidates pricing."""
     rng = np.random.default_rng(8)
