@@ -60,12 +60,11 @@ struct Shared {
   int64_t tk[6];      // phase tick counters (rank 0 updates them)
   int32_t cnt;
   int32_t pend_row, pend_col;  // Vogel: kinds of line the next step rescans
-  int32_t qtail;
   int32_t status;
-  int32_t nlevels;
+  int32_t level[3];   // tree build: whether a level reached anything, in turn
   int32_t idx;
   int32_t stop;       // deadline reached (rank 0 decides, the group follows)
-  int32_t pad0_[2];
+  int32_t pad0_[1];
   int32_t cnt2;       // Vogel, register mode: list count of the odd steps (cnt: the even ones)
   int32_t dlo[2];     // pivot: least depth of a cycle vertex (atomicMin), by pivot parity
   int32_t pad_[7];
@@ -152,12 +151,12 @@ __host__ __device__ inline size_t vogel_lds_bytes(int m, int n) {
          2 * align16(2 * (size_t)V) + align16((size_t)V);
 }
 // aux region in int32 units: max(tree-build scratch, path snapshot)
-//   build: start[V+1], vis[V], lvl[V+2], adj[2V] (int16), queue[V] (int16)
+//   build: cell ends, cell costs, depths, sizes, next positions, V each
 //   snapshot: for each side of the cycle, vertex, slot (int16), pre | size << 16 and flow (int32)
 //   of its vertices by depth, V entries each
 __host__ __device__ inline size_t aux_ints(int m, int n) {
   const size_t V = (size_t)(m + n);
-  const size_t build = (V + 1) + V + (V + 2) + V + (V + 1) / 2 + 8;
+  const size_t build = 5 * V;
   const size_t snap = 2 * (2 * ((V + 1) / 2 + 4) + 2 * (V + 4));
   return build > snap ? build : snap;
 }
@@ -1080,110 +1079,109 @@ __device__ __forceinline__ void set_dual(const TreeLds& t, int m, int x, int32_t
 }
 
 // ---------------------------------------------------------------------------
-// Basis tree from the m+n-1 basic cells: CSR adjacency (degree count, scan, fill --
-// the reference's determine_length / inclusive_scan / fill_Ea, parallel_kernels.cu:
-// 205-256, 294-319), then a level-synchronous BFS from vertex 0 that sets parent,
-// depth, slot, flow and the duals (x_child = c(row,col) - x_parent, DUAL_solver.cu:
-// 52-62), then subtree sizes bottom-up and preorder numbers top-down, level by level.
-// Returns false if the cells do not form a spanning tree.
+// Basis tree from the m+n-1 basic cells, rooted at vertex 0: level by level, every cell
+// not used yet whose one end has the level's depth hangs its other end below it (parent,
+// depth, slot and dual, x_child = c(row,col) - x_parent, DUAL_solver.cu:52-62; the
+// reference's CSR, parallel_kernels.cu:205-319, is not needed for that).  Then subtree
+// sizes bottom-up and preorder numbers top-down, again level by level: a vertex takes its
+// interval from its parent's next free position (siblings in any order: preorder numbers
+// only serve ancestor tests).  Returns false if the cells do not form a spanning tree: of
+// V - 1 cells that leave no vertex unreached none closes a cycle.
+// Bound: three passes of one barrier and one or two LDS round trips per level, 94 levels at
+// 505x475.  The cells' ends and costs are read from global memory once.  (A BFS over a CSR
+// read its cells' rows, columns, flows and costs from global memory level by level, with
+// two barriers each, after a serial scan of the degrees: 130 us at 500x480, 21 us at 13x9,
+// 2.9 ms at 4000x2000.)
+// scr: 5 V ints (aux_ints).
 // ---------------------------------------------------------------------------
 template <int G>
 __device__ __forceinline__ bool build_tree(const Ctx& C, gcint* brow, gcint* bcol, gcint* bflow, const TreeLds& t, int32_t* scr,
                            Shared& S) {
   const int m = C.m, V = C.V, tid = grank<G>();
-  int32_t* start = scr;                    // V+1
-  int32_t* vis = start + V + 1;            // V  (fill cursor, then visited flag, then size)
-  int32_t* lvl = vis + V;                  // V+2
-  int16_t* adj = (int16_t*)(lvl + V + 2);  // 2V
-  int16_t* queue = adj + 2 * V;            // V
-  for (int x = tid; x <= V; x += G) start[x] = 0;
-  gsync<G>();
+  int32_t* arc = scr;        // V-1: row << 16 | column vertex (-1: used)
+  int32_t* acost = arc + V;  // V-1
+  int32_t* dep = acost + V;  // V: depth, -1 unreached
+  int32_t* size = dep + V;   // V
+  int32_t* next = size + V;  // V: next free preorder position below the vertex
   int badCell = 0;
   for (int k = tid; k < V - 1; k += G) {
     const int r = brow[k], c = bcol[k];
-    if (r < 0 || r >= m || c < 0 || c >= C.n) { badCell = 1; continue; }  // guard
-    atomicAdd(&start[r + 1], 1);
-    atomicAdd(&start[m + c + 1], 1);
+    const bool bad = r < 0 || r >= m || c < 0 || c >= C.n;  // guard
+    badCell |= bad ? 1 : 0;
+    arc[k] = bad ? -1 : (int32_t)(((uint32_t)r << 16) | (uint32_t)(m + c));
+    acost[k] = bad ? 0 : cost_at(C, r, c);
   }
+  for (int x = tid; x < V; x += G) { dep[x] = x == 0 ? 0 : -1; size[x] = 1; }
   if (badCell) atomicAdd(&S.status, 1);
+  if (tid == 0) {
+    t.parent[0] = -1; t.slot[0] = -1; t.flow[0] = 0; set_dual(t, m, 0, 0);
+    S.level[0] = S.level[1] = S.level[2] = 0;
+  }
   gsync<G>();
   if (S.status != 0) return false;
-  if (tid == 0) {  // exclusive scan of the degrees
-    int32_t run = 0;
-    for (int x = 1; x <= V; ++x) { run += start[x]; start[x] = run; }
-  }
-  gsync<G>();
-  for (int x = tid; x < V; x += G) vis[x] = start[x];
-  gsync<G>();
-  for (int k = tid; k < V - 1; k += G) {
-    const int r = brow[k], c = bcol[k];
-    adj[atomicAdd(&vis[r], 1)] = (int16_t)k;
-    adj[atomicAdd(&vis[m + c], 1)] = (int16_t)k;
-  }
-  gsync<G>();
-  for (int x = tid; x < V; x += G) { vis[x] = 0; t.parent[x] = -1; t.depth[x] = 0; }
-  gsync<G>();
-  if (tid == 0) {
-    vis[0] = 1; queue[0] = 0; t.slot[0] = -1; t.flow[0] = 0; set_dual(t, m, 0, 0);
-    lvl[0] = 0; lvl[1] = 1; S.qtail = 1; S.nlevels = 1;
-  }
-  gsync<G>();
+  constexpr int U = 4;  // cells a rank looks at together
   int d = 0;
-  for (;;) {
-    const int b = lvl[d], e = lvl[d + 1];
-    if (b == e) break;  // uniform: written before the sync
-    for (int q = b + tid; q < e; q += G) {
-      const int x = queue[q];
-      const int px = t.parent[x];
-      const int32_t dx = dual_of(t, m, x);
-      for (int a = start[x]; a < start[x + 1]; ++a) {
-        const int k = adj[a];
-        const int r = brow[k], c = bcol[k];
-        const int y = x < m ? m + c : r;
-        if (y == px) continue;
-        if (atomicExch(&vis[y], 1) != 0) continue;  // a cycle in the cell set
-        t.parent[y] = (int16_t)x; t.depth[y] = (int16_t)(d + 1); t.slot[y] = (int16_t)k;
-        t.flow[y] = bflow[k];
-        set_dual(t, m, y, cost_at(C, r, c) - dx);
-        queue[atomicAdd(&S.qtail, 1)] = (int16_t)y;
+  for (;; ++d) {
+    // whether this level reached anything; the flag of the next level is cleared here: it
+    // was last read two barriers ago
+    int32_t* grown = &S.level[d % 3];
+    if (tid == 0) S.level[(d + 1) % 3] = 0;
+    for (int k0 = tid; k0 < V - 1; k0 += U * G) {
+      int32_t a[U], dr[U], dc[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) a[u] = k0 + u * G < V - 1 ? arc[k0 + u * G] : -1;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        dr[u] = lds_load(&dep[a[u] < 0 ? 0 : a[u] >> 16]);
+        dc[u] = lds_load(&dep[a[u] < 0 ? 0 : a[u] & 0xffff]);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool down = dr[u] == d && dc[u] < 0, up = dc[u] == d && dr[u] < 0;
+        if (a[u] >= 0 && (down | up)) {
+          const int k = k0 + u * G, r = a[u] >> 16, c = a[u] & 0xffff;
+          const int x = down ? r : c, y = down ? c : r;  // y hangs below x
+          t.parent[y] = (int16_t)x; t.slot[y] = (int16_t)k;
+          set_dual(t, m, y, acost[k] - dual_of(t, m, x));
+          lds_store(&dep[y], d + 1);
+          arc[k] = -1;
+          lds_store(grown, 1);
+        }
       }
     }
     gsync<G>();
-    if (tid == 0) { lvl[d + 2] = S.qtail; S.nlevels = d + 2; }
-    gsync<G>();
-    ++d;
+    if (lds_load(grown) == 0) break;  // uniform: written before the barrier
   }
-  const int nl = S.nlevels;  // levels 0..nl-2 are non-empty
-  const bool ok = S.qtail == V;
+  // depths 1 .. d are in use
+  bool reached = true;
+  for (int x = tid; x < V; x += G) reached = reached & (dep[x] >= 0);
+  if (!reached) atomicAdd(&S.status, 1);
   gsync<G>();
-  if (!ok) return false;
-  for (int x = tid; x < V; x += G) vis[x] = 1;
-  gsync<G>();
-  for (int dd = nl - 2; dd >= 1; --dd) {  // subtree sizes, deepest level first
-    for (int q = lvl[dd] + tid; q < lvl[dd + 1]; q += G) {
-      const int x = queue[q];
-      atomicAdd(&vis[t.parent[x]], vis[x]);
-    }
+  if (S.status != 0) {  // (the caller reports the forest; the status is its own)
+    gsync<G>();
+    if (tid == 0) S.status = 0;
+    gsync<G>();
+    return false;
+  }
+  for (int x = tid; x < V; x += G)
+    if (x > 0) t.flow[x] = bflow[t.slot[x]];
+  for (int dd = d; dd >= 1; --dd) {  // subtree sizes, deepest level first
+    for (int x = tid; x < V; x += G)
+      if (dep[x] == dd) atomicAdd(&size[t.parent[x]], size[x]);
     gsync<G>();
   }
-  if (tid == 0) t.pre(0) = 0;
+  if (tid == 0) { t.pre(0) = 0; next[0] = 1; }
   gsync<G>();
-  for (int dd = 0; dd < nl - 1; ++dd) {  // preorder, children in CSR order
-    for (int q = lvl[dd] + tid; q < lvl[dd + 1]; q += G) {
-      const int x = queue[q];
-      const int px = t.parent[x];
-      int run = t.pre(x) + 1;
-      for (int a = start[x]; a < start[x + 1]; ++a) {
-        const int k = adj[a];
-        const int y = x < m ? m + bcol[k] : brow[k];
-        if (y == px) continue;
-        t.pre(y) = (int16_t)run;
-        run += vis[y];
+  for (int dd = 1; dd <= d; ++dd) {
+    for (int x = tid; x < V; x += G)
+      if (dep[x] == dd) {
+        const int p = atomicAdd(&next[t.parent[x]], size[x]);
+        t.pre(x) = (int16_t)p;
+        next[x] = p + 1;
       }
-    }
     gsync<G>();
   }
-  for (int x = tid; x < V; x += G) t.size(x) = (int16_t)vis[x];
+  for (int x = tid; x < V; x += G) { t.size(x) = (int16_t)size[x]; t.depth[x] = (int16_t)dep[x]; }
   gsync<G>();
   return true;
 }
@@ -2238,10 +2236,8 @@ __device__ __forceinline__ void large_setup(DevInstance& D, char* region, size_t
   // (instances whose tree does not fit LDS); otherwise in LDS, saved to state per round
   const bool treeGlobal = P.tree_global != 0;
   char* gtree = (char*)uniform_ptr(D.state);
-  const TreeLds t = carve_tree(treeGlobal ? gtree : smem, C.m, C.n);
   const size_t treeBytes = tree_lds_bytes(C.m, C.n);
-  int32_t* aux = (!treeGlobal && treeBytes + 4 * aux_ints(C.m, C.n) <= avail) ? (int32_t*)(smem + treeBytes)
-                                                                              : uniform_ptr(D.scratch);
+  const bool auxLds = !treeGlobal && treeBytes + 4 * aux_ints(C.m, C.n) <= avail;
   const bool lead = grank<G>() == 0;
   if (lead) {
     S.status = 0;
@@ -2265,15 +2261,21 @@ __device__ __forceinline__ void large_setup(DevInstance& D, char* region, size_t
   gsync<G>();
   bool ok = S.status == 0;
   { const uint64_t t2 = now_ticks(); if (lead) S.tk[0] += (int64_t)(t2 - tp); tp = t2; }
-  if (ok) ok = build_tree<G>(C, brow, bcol, bflow, t, aux, S);
-  { const uint64_t t2 = now_ticks(); if (lead) S.tk[1] += (int64_t)(t2 - tp); tp = t2; }
-  if (ok) {
+  // one call for a tree and scratch in LDS, so that its accesses are LDS ones
+  auto finish = [&](const TreeLds& t, int32_t* aux) {
+    ok = build_tree<G>(C, brow, bcol, bflow, t, aux, S);
+    if (!ok) return;
     write_padding<G>(C);
     for (int j = C.n + grank<G>(); j < C.ld; j += G) t.dv[j] = 0;  // padding duals
     tree_index<G>(C, t, S);
-    // a tree in global memory stays where it is; the sweep grid reads its duals there
-    if (!treeGlobal) save_state<G>(smem, treeBytes, gl(uniform_ptr(D.state)));
+  };
+  if (ok) {
+    if (auxLds) finish(carve_tree(smem, C.m, C.n), (int32_t*)(smem + treeBytes));
+    else finish(carve_tree(treeGlobal ? gtree : smem, C.m, C.n), uniform_ptr(D.scratch));
   }
+  { const uint64_t t2 = now_ticks(); if (lead) S.tk[1] += (int64_t)(t2 - tp); tp = t2; }
+  // a tree in global memory stays where it is; the sweep grid reads its duals there
+  if (ok && !treeGlobal) save_state<G>(smem, treeBytes, gl(uniform_ptr(D.state)));
   if (lead) {
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
     D.iterations = 0; D.sweeps = 0; D.mode = 0;
