@@ -261,8 +261,14 @@ struct Server {
     int bigV = 0;
     for (int s : order)
       if (slots[s].m + slots[s].n > bigV) { bigV = slots[s].m + slots[s].n; maxm = slots[s].m; maxn = slots[s].n; }
-    // one engine configuration per slice, chosen for its largest request
-    const int cfg = pick_cfg(maxm, maxn, &opt, (int64_t)order.size());
+    // one engine configuration per slice, chosen for its largest request; a request of nearly
+    // its m+n can need a few bytes more (the padding of m and n) and then takes the slice to
+    // 1024 threads, whose snapshot may be in global memory
+    int cfg = pick_cfg(maxm, maxn, &opt, (int64_t)order.size());
+    for (int s : order) {
+      const int c = pick_cfg(slots[s].m, slots[s].n, &opt, (int64_t)order.size(), bigV);
+      if (cfg_threads(c) > cfg_threads(cfg)) cfg = c;
+    }
     for (int s : order) {
       bool dummy;
       lds = std::max(lds, cfg_group_bytes(cfg, slots[s].m, slots[s].n, &dummy));
