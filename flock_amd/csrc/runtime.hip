@@ -156,7 +156,7 @@ constexpr int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
 // size-class policy (tuned on MI355X; see autotune): instances with m+n up to
 // g_wave_max_v get one wavefront each, packed g_wave_pack per workgroup; larger ones
 // get a whole workgroup of 256 threads up to g_wg256_max_v, else 512 threads while the tree
-// and the pivot's snapshot fit LDS (m+n up to about 3600), else 1024.  A workgroup of 1024
+// and the pivot's snapshot fit LDS (m+n up to about 3700), else 1024.  A workgroup of 1024
 // loses at every size that 512 can take: its barriers cost 144 cycles instead of 48 and
 // four waves share each SIMD (61x1203 dantzig 8.4 against 6.2 ms, 100x2400 candidates 15.7
 // against 13.3 ms, 1800x1700 candidates 100 against 92 ms).

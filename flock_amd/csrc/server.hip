@@ -261,9 +261,9 @@ struct Server {
     int bigV = 0;
     for (int s : order)
       if (slots[s].m + slots[s].n > bigV) { bigV = slots[s].m + slots[s].n; maxm = slots[s].m; maxn = slots[s].n; }
-    // one engine configuration per slice, chosen for its largest request; a request of nearly
-    // its m+n can need a few bytes more (the padding of m and n) and then takes the slice to
-    // 1024 threads, whose snapshot may be in global memory
+    // one engine configuration per slice, chosen for its largest request; raised where another
+    // request needs more threads: LDS follows m and n padded apart, so it need not grow with
+    // m+n (at the present layout and 160 KB no two requests straddle the limit, m+n = 3704)
     int cfg = pick_cfg(maxm, maxn, &opt, (int64_t)order.size());
     for (int s : order) {
       const int c = pick_cfg(slots[s].m, slots[s].n, &opt, (int64_t)order.size(), bigV);
