@@ -71,13 +71,22 @@ struct Shared {
   uint64_t red1[3][16];  // one-barrier reductions (group_min1 / group_max1), by buffer
 };
 
+// Every reduction orders the group's memory accesses before it with those after it: a
+// workgroup's by its barrier, a wavefront's by a sync point of its own (its lane moves only
+// touch registers, so the compiler could otherwise move LDS accesses across them).
+template <int G>
+__device__ __forceinline__ void reduction_sync() {
+  if constexpr (G == kWave) gsync<G>();
+}
 template <int G>
 __device__ __forceinline__ uint64_t group_min_u64(uint64_t x, Shared& S) {
+  reduction_sync<G>();
   if constexpr (G == kWave) return wave_min_u64(x);
   else return block_min_u64<G>(x, S.red);
 }
 template <int G>
 __device__ __forceinline__ uint64_t group_max_u64(uint64_t x, Shared& S) {
+  reduction_sync<G>();
   if constexpr (G == kWave) return wave_max_u64(x);
   else return block_max_u64<G>(x, S.red);
 }
@@ -86,22 +95,26 @@ __device__ __forceinline__ uint64_t group_max_u64(uint64_t x, Shared& S) {
 // reductions on one buffer always have another barrier between them.
 template <int G, int kBuf>
 __device__ __forceinline__ uint64_t group_min1_u64(uint64_t x, Shared& S) {
+  reduction_sync<G>();
   if constexpr (G == kWave) return wave_min_u64(x);
   else return block_min1_u64<G>(x, S.red1[kBuf]);
 }
 template <int G, int kBuf>
 __device__ __forceinline__ uint64_t group_max1_u64(uint64_t x, Shared& S) {
+  reduction_sync<G>();
   if constexpr (G == kWave) return wave_max_u64(x);
   else return block_max1_u64<G>(x, S.red1[kBuf]);
 }
 // The same max on buffer 0 or 2 in turn, for a loop with no other barrier.
 template <int G>
 __device__ __forceinline__ uint64_t group_max_alt(uint64_t x, Shared& S, int odd) {
+  reduction_sync<G>();
   if constexpr (G == kWave) return wave_max_u64(x);
   else return block_max1_u64<G>(x, S.red1[2 * odd]);
 }
 template <int G>
 __device__ __forceinline__ int64_t group_sum_i64(int64_t x, Shared& S) {
+  reduction_sync<G>();
   if constexpr (G == kWave) return wave_sum_i64(x);
   else return block_sum_i64<G>(x, S.red);
 }

@@ -23,6 +23,15 @@
 #include <cstdlib>
 #include <vector>
 
+#if defined(__has_feature)
+#if __has_feature(thread_sanitizer)
+#define EMU_TSAN 1
+#include <linux/futex.h>
+#include <sys/syscall.h>
+#include <unistd.h>
+#endif
+#endif
+
 #define __device__
 #define __host__
 #define __global__
@@ -53,6 +62,29 @@ struct TagBarrier {
   }
 #else
   void wait(int who, int tag) { tags[who] = tag; bar.arrive_and_wait(); }
+#ifdef EMU_TSAN
+  // The rendezvous of a cross-lane operation: it moves register values and orders no memory
+  // access, so it must be no synchronisation in ThreadSanitizer's eyes.  Relaxed atomics and
+  // a bare futex: only the engine's own sync points order lanes' memory accesses.
+  int arrived = 0, generation = 0;
+  void meet(int who, int tag) {
+    const int seen = __atomic_load_n(&generation, __ATOMIC_RELAXED);
+    __atomic_store_n(&met[who], tag, __ATOMIC_RELAXED);
+    if (__atomic_add_fetch(&arrived, 1, __ATOMIC_RELAXED) == count) {
+      for (int i = 0; i < count; ++i)
+        if (__atomic_load_n(&met[i], __ATOMIC_RELAXED) != tag) {
+          std::fprintf(stderr, "emu: cross-lane operations differ: lane %d at %d, lane %d at %d\n", who, tag, i, met[i]);
+          std::abort();
+        }
+      __atomic_store_n(&arrived, 0, __ATOMIC_RELAXED);
+      __atomic_add_fetch(&generation, 1, __ATOMIC_RELAXED);
+      syscall(SYS_futex, &generation, FUTEX_WAKE_PRIVATE, count, nullptr, nullptr, 0);
+    } else {
+      while (__atomic_load_n(&generation, __ATOMIC_RELAXED) == seen)
+        syscall(SYS_futex, &generation, FUTEX_WAIT_PRIVATE, seen, nullptr, nullptr, 0);
+    }
+  }
+#endif
 #endif
   struct Check {
     TagBarrier* self;
@@ -66,6 +98,9 @@ struct TagBarrier {
   };
   int count;
   std::vector<int> tags;
+#ifdef EMU_TSAN
+  std::vector<int> met = std::vector<int>(count, 0);
+#endif
   std::barrier<Check> bar;
 };
 struct Lane {
@@ -88,12 +123,23 @@ inline Dim3 thread_idx() { return Dim3{lane_ctx.tid, 0, 0}; }
 inline void __threadfence_block() { std::atomic_thread_fence(std::memory_order_seq_cst); }
 inline void __threadfence() { std::atomic_thread_fence(std::memory_order_seq_cst); }
 
+namespace emu {
+inline void rendezvous(unsigned lane, int tag) {
+#ifdef EMU_TSAN
+  lane_ctx.wave->meet((int)lane, tag);
+#else
+  lane_ctx.wave->wait((int)lane, tag);
+#endif
+}
+inline void put(unsigned lane, uint64_t v) { __atomic_store_n(&lane_ctx.xchg[lane], v, __ATOMIC_RELAXED); }
+inline uint64_t get(unsigned lane) { return __atomic_load_n(&lane_ctx.xchg[lane % 64], __ATOMIC_RELAXED); }
+}  // namespace emu
 inline uint64_t emu_exchange(uint64_t v, unsigned src) {
   const unsigned lane = emu::lane_ctx.tid % 64;
-  emu::lane_ctx.xchg[lane] = v;
-  emu::lane_ctx.wave->wait((int)lane, -1);
-  const uint64_t r = emu::lane_ctx.xchg[src % 64];
-  emu::lane_ctx.wave->wait((int)lane, -2);
+  emu::put(lane, v);
+  emu::rendezvous(lane, -1);
+  const uint64_t r = emu::get(src);
+  emu::rendezvous(lane, -2);
   return r;
 }
 inline uint32_t __shfl_xor(uint32_t v, int mask, int width = 64) {
@@ -107,11 +153,11 @@ inline int __shfl(int v, int src, int width = 64) {
 // 64-lane ballot: every lane publishes its predicate, then reads all 64
 inline uint64_t __ballot(int pred) {
   const unsigned lane = emu::lane_ctx.tid % 64;
-  emu::lane_ctx.xchg[lane] = pred ? 1 : 0;
-  emu::lane_ctx.wave->wait((int)lane, -3);
+  emu::put(lane, pred ? 1 : 0);
+  emu::rendezvous(lane, -3);
   uint64_t m = 0;
-  for (int i = 0; i < 64; ++i) m |= (emu::lane_ctx.xchg[i] ? 1ull : 0ull) << i;
-  emu::lane_ctx.wave->wait((int)lane, -4);
+  for (unsigned i = 0; i < 64; ++i) m |= (emu::get(i) ? 1ull : 0ull) << i;
+  emu::rendezvous(lane, -4);
   return m;
 }
 // DPP moves used by the wavefront reductions: row_shr:k (0x111..0x11f), row_bcast:15

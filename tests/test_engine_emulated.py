@@ -6,7 +6,8 @@ lane on OS threads (tests/emu), checked against the oracle -- no GPU needed.
     step-bounded solves (the server's mode);
   * AddressSanitizer build: no out-of-bounds access of the engine's buffers;
   * ThreadSanitizer build: no data race between lanes (every cross-lane dependence
-    goes through a group sync), and the emulator's call-site-checked barriers prove
+    goes through a group sync; the rendezvous of a cross-lane operation counts as none,
+    also within one wavefront), and the emulator's call-site-checked barriers prove
     that all lanes of a group pass the same sequence of sync points.
 """
 import json
@@ -123,7 +124,12 @@ def test_emulated_engine_thread_sanitizer():
              {"m": 10, "n": 14, "seed": 4, "group": 64, "pricing": 1, "steps": 3},
              {"m": 13, "n": 16, "seed": 5, "group": 256, "pricing": 2},
              # 150 vertices on one wavefront: four window slots per rank in the re-root
-             {"m": 70, "n": 80, "seed": 11, "group": 64, "pricing": 1}]
+             {"m": 70, "n": 80, "seed": 11, "group": 64, "pricing": 1},
+             # one wavefront whose Vogel steps list many lines (equal costs), the multi-pivot
+             # rule's claims, a north-west corner start
+             {"m": 40, "n": 20, "seed": 12, "group": 64, "degenerate": True},
+             {"m": 21, "n": 17, "seed": 13, "group": 64, "pricing": 2},
+             {"m": 18, "n": 12, "seed": 14, "group": 64, "initial": 1}]
     check(run("tsan", cases))
 
 
