@@ -1275,6 +1275,7 @@ struct SweepShape {
     return w > 1 ? (uint32_t)(((uint64_t)p * magic) >> 32) : p;
   }
 };
+// w: at most a block, kSlots * G vectors
 template <int G>
 __device__ __forceinline__ SweepShape sweep_shape(int m, int w) {
   SweepShape s;
@@ -2147,7 +2148,8 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
   constexpr int K = kCands ? CandsPerRank<G>::value : 1;
   CandSet<K> cands;
   cands.clear();
-  const SweepShape shape = sweep_shape<G>(m, C.ld >> 2);
+  SweepShape shape{};
+  if constexpr (!SweepChunks<G>::value) shape = sweep_shape<G>(m, C.ld >> 2);
   int minor = 0;
   bool haveList = false;
   for (;;) {

@@ -107,6 +107,17 @@ def test_emulated_windowed_reroot_beyond_one_pass():
              {"m": 220, "n": 110, "seed": 75, "group": 64, "degenerate": True}]
     check(run("plain", cases))
 
+
+def test_emulated_wavefront_sweep_beyond_one_block():
+    """64-lane groups with rows longer than a sweep block (256 vectors, n > 1024): the row
+    is swept in chunks.  At, just past and well past the block's edge."""
+    cases = [{"m": 3, "n": n, "seed": n, "group": 64, "smax": 50000} for n in (1024, 1025, 1100)]
+    cases += [{"m": 2, "n": 1540, "seed": 82, "group": 64, "smax": 50000},
+              {"m": 5, "n": 1030, "seed": 83, "group": 64, "smax": 50000, "pricing": 1},
+              {"m": 2, "n": 1090, "seed": 84, "group": 64, "smax": 50000, "pricing": 2}]
+    check(run("plain", cases))
+
+
 def test_emulated_engine_address_sanitizer():
     cases = [{"m": 23, "n": 37, "seed": 1, "group": 64}, {"m": 13, "n": 11, "seed": 2, "group": 256},
              {"m": 30, "n": 30, "seed": 3, "group": 64, "pricing": 1, "steps": 5},
