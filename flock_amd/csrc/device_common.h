@@ -90,9 +90,11 @@ struct EngineParams {
   int32_t prio_count;       // the first prio_count queue positions (largest work first) run at raised wave priority
   int32_t tree_global;      // large-instance path: the basis tree lives in the state buffer (global memory)
   int32_t pad_;
-  // time slicing (server): when slice_ticks > 0, no instance is started and no pivot is
-  // begun later than slice_ticks device-clock ticks after *clock0 (the launch stamp the
-  // reset kernel writes); the kernel turns that into `deadline`
+  // time slicing (server): when slice_ticks > 0, no instance is started later than
+  // slice_ticks device-clock ticks after *clock0 (the launch stamp the reset kernel
+  // writes), and no pivot is begun later, or sweep's claim rounds with the multi-pivot
+  // rules; candidate pricing looks every fourth pivot.  Every call makes some progress.
+  // The kernel turns slice_ticks into `deadline`
   uint64_t slice_ticks;
   const uint64_t* clock0;
   uint64_t deadline;

@@ -2174,9 +2174,10 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
     }
     if (done >= budget) { status = 1; finished = true; break; }
     if (P.step_pivots > 0 && done >= P.step_pivots) break;
-    // one decision for the whole group, every fourth pivot (the clock, a barrier and, past
-    // the deadline, a read of the launch's counter); >= 1 pivot per call
-    if (P.deadline && done % 4 == 1) {
+    // one decision for the whole group, >= 1 pivot per call: after every sweep (where it
+    // costs little beside it), and on every fourth pivot of a candidate list (the clock, a
+    // barrier and, past the deadline, a read of the launch's counter)
+    if (P.deadline && done > 0 && (!kCands || done % 4 == 1)) {
       if (lead)
         S.stop = now_ticks() >= P.deadline &&
                  (!P.busy || __hip_atomic_load(P.busy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0);

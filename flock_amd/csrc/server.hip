@@ -7,9 +7,10 @@
 //      with the slice that is running;
 //   2. a slice is one persistent work-queue launch over every admitted, unfinished
 //      request (oldest first).  No request is started after the slice's deadline, and
-//      no pivot is begun after it once no request of the slice is still in its Vogel or
-//      tree build (those cannot stop, and the launch lasts until they end, so the other
-//      requests keep pivoting meanwhile); an unfinished request saves its basis tree to
+//      no pivot (candidate pricing: at most three) is begun after it once no request of
+//      the slice is still in its Vogel or tree build (those cannot stop, and the launch
+//      lasts until they end, so the other requests keep pivoting meanwhile); a request
+//      makes some progress in every slice; an unfinished one saves its basis tree to
 //      its slot and resumes from it in the next slice, so costs, trees and duals stay
 //      resident;
 //   3. after a slice, finished requests are gathered into one contiguous device buffer

@@ -23,7 +23,7 @@ def load_variant(variant: str):
     L.emu_solve.argtypes = [ctypes.c_int, ctypes.c_int, i32p, i32p, i32p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                             ctypes.c_int, ctypes.c_int64, ctypes.c_int, i32p, i32p, i32p, i32p,
                             ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
-                            ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]
+                            ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int64)]
     L.emu_large.argtypes = [ctypes.c_int, ctypes.c_int, i32p, i32p, i32p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                             i32p, i32p, i32p, i32p, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
                             ctypes.POINTER(ctypes.c_int32)]
@@ -58,12 +58,12 @@ def solve(L, cost, supply, demand, group=64, groups_per_wg=4, pricing=0, initial
     V = m + n
     br = np.zeros(V - 1, np.int32); bc = np.zeros(V - 1, np.int32); bf = np.zeros(V - 1, np.int32)
     du = np.zeros(V, np.int32)
-    obj, it = ctypes.c_int64(), ctypes.c_int64()
+    obj, it, sweeps = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
     st, steps = ctypes.c_int32(), ctypes.c_int32()
     r = L.emu_solve(m, n, cost.ravel(), np.ascontiguousarray(supply, np.int32), np.ascontiguousarray(demand, np.int32),
                     group, groups_per_wg, pricing, initial, max_it, step_pivots, br, bc, bf, du,
-                    ctypes.byref(obj), ctypes.byref(it), ctypes.byref(st), ctypes.byref(steps))
-    return dict(ret=r, objective=obj.value, iterations=it.value, status=st.value, steps=steps.value,
+                    ctypes.byref(obj), ctypes.byref(it), ctypes.byref(st), ctypes.byref(steps), ctypes.byref(sweeps))
+    return dict(ret=r, objective=obj.value, iterations=it.value, status=st.value, steps=steps.value, sweeps=sweeps.value,
                 rows=br, cols=bc, flows=bf, u=du[:m], v=du[m:])
 
 

@@ -296,7 +296,8 @@ extern "C" int emu_queue(int count, const int32_t* ms, const int32_t* ns, const 
 extern "C" int emu_solve(int m, int n, const int32_t* cost, const int32_t* supply, const int32_t* demand, int group,
                          int groups_per_wg, int pricing, int initial, int64_t max_it, int step_pivots,
                          int32_t* brow_out, int32_t* bcol_out, int32_t* bflow_out, int32_t* dual_out,
-                         int64_t* objective, int64_t* iterations, int32_t* status, int32_t* steps_out) {
+                         int64_t* objective, int64_t* iterations, int32_t* status, int32_t* steps_out,
+                         int64_t* sweeps_out) {
   const int V = m + n;
   const int ld = (n + 3) & ~3, ldT = (m + 3) & ~3;
   int32_t* c = exact<int32_t>((size_t)m * ld);
@@ -341,6 +342,7 @@ extern "C" int emu_solve(int m, int n, const int32_t* cost, const int32_t* suppl
   std::memcpy(bflow_out, bf, 4 * (size_t)(V - 1));
   std::memcpy(dual_out, du, 4 * (size_t)V);
   *objective = D.objective; *iterations = D.iterations; *status = D.status; *steps_out = steps;
+  *sweeps_out = D.sweeps;
   for (void* p : {(void*)c, (void*)cT, (void*)s, (void*)d, (void*)br, (void*)bc, (void*)bf, (void*)du, (void*)scr,
                   (void*)st, (void*)region})
     std::free(p);

@@ -108,6 +108,24 @@ def test_emulated_windowed_reroot_beyond_one_pass():
     check(run("plain", cases))
 
 
+@pytest.mark.parametrize("pricing", [0, 1, 2, 4])
+def test_emulated_expired_slice_deadline(pricing):
+    """A deadline that has passed stops a call after the least progress: one pivot, or one
+    sweep's claim rounds under the multi-pivot rules (the check comes after the next sweep,
+    so a call has two sweeps at most)."""
+    sys.path.insert(0, EMU)
+    import emu
+    emu.build()
+    L = emu.load_variant("plain")
+    inst = I.random_instance(np.random.default_rng(31), 40, 33, 50, 100)
+    o = oracle.solve(inst.cost, inst.supply, inst.demand)
+    r = emu.solve(L, inst.cost, inst.supply, inst.demand, group=64, pricing=pricing, step_pivots=-1)
+    assert r["status"] == 0 and r["objective"] == o.objective
+    assert r["sweeps"] <= 2 * r["steps"]
+    if pricing < 2:
+        assert r["iterations"] <= r["steps"]
+
+
 def test_emulated_wavefront_sweep_beyond_one_block():
     """64-lane groups with rows longer than a sweep block (256 vectors, n > 1024): the row
     is swept in chunks.  At, just past and well past the block's edge."""
