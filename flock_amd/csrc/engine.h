@@ -57,7 +57,8 @@ __device__ __forceinline__ void gsync() {
 // Scalars shared by one group; they sit at the start of the group's LDS region.
 struct Shared {
   uint64_t red[17];
-  int64_t tk[6];      // phase tick counters (rank 0 updates them)
+  int64_t tk[6];      // phase tick counters (rank 0 updates them), as DevInstance::ticks
+  int64_t reprice_ticks;  // samples of this call's candidate re-pricings
   int32_t cnt;
   int32_t pend_row, pend_col;  // Vogel: kinds of line the next step rescans
   int32_t status;
@@ -67,7 +68,7 @@ struct Shared {
   int32_t pad0_[1];
   int32_t cnt2;       // Vogel, register mode: list count of the odd steps (cnt: the even ones)
   int32_t dlo[2];     // pivot: least depth of a cycle vertex (atomicMin), by pivot parity
-  int32_t pad_[7];
+  int32_t pad_[5];
   uint64_t red1[3][16];  // one-barrier reductions (group_min1 / group_max1), by buffer
 };
 
@@ -1586,9 +1587,15 @@ template <int N>
 struct IntC { static constexpr int value = N; };
 
 // Phase timers: reading the clock takes 80 cycles and drains the LDS queue, and a pivot has
-// four readings, so every eighth pivot is timed and counted eight times.
+// four readings, so every eighth event of a kind is timed, the first one among them.  Events
+// are counted over the whole solve (pivots, Dantzig's sweeps) or from each sweep on
+// (candidate re-pricings), and the samples' sum is scaled to all of them at the end.
 constexpr int kTimedEvery = 8;
-__device__ __forceinline__ bool timed_pivot(int count) { return count % kTimedEvery == 0; }
+__device__ __forceinline__ bool timed_event(int count) { return count % kTimedEvery == 0; }
+__device__ __forceinline__ int64_t timed_events(int64_t events) { return (events + kTimedEvery - 1) / kTimedEvery; }
+__device__ __forceinline__ int64_t scale_samples(int64_t sum, int64_t events, int64_t timings) {
+  return timings > 0 ? (int64_t)((double)sum * ((double)events / (double)timings) + 0.5) : 0;
+}
 
 // kR: vertices each rank handles per pass, their LDS loads issued together.
 // kWideWin: the re-root's windowed form takes twice the slots per rank where kR is below
@@ -1598,7 +1605,7 @@ template <int G, int kR, class SN, bool kWideWin = false>
 __device__ __forceinline__ bool pivot_pass(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej, int32_t r,
                                            int count) {
   const int m = C.m, V = C.V, tid = grank<G>();
-  const bool timed = timed_pivot(count);
+  const bool timed = timed_event(count);
   uint64_t t0 = 0;
   if (timed) t0 = now_ticks();
   const int I = ei, J = m + ej;
@@ -1660,7 +1667,7 @@ __device__ __forceinline__ bool pivot_pass(const Ctx& C, const TreeLds& t, const
   uint64_t t1 = 0;
   if (timed) {
     t1 = now_ticks();
-    if (tid == 0) S.tk[4] += kTimedEvery * (int64_t)(t1 - t0);
+    if (tid == 0) S.tk[4] += (int64_t)(t1 - t0);
   }
   // the chain P[0] = a .. P[k] = q on q's side: snapshot entries dA .. dA + k
   const int qs = sideI ? 0 : 1;
@@ -1804,7 +1811,7 @@ __device__ __forceinline__ bool pivot_pass(const Ctx& C, const TreeLds& t, const
     for (int u = 0; u < kRW; ++u)
       if (xs[u] >= 0) t.vat[np[u]] = (int16_t)xs[u];
     if (tid == 0) S.dlo[sel ^ 1] = 0x7fffffff;
-    if (timed && tid == 0) S.tk[5] += kTimedEvery * (int64_t)(now_ticks() - t1);
+    if (timed && tid == 0) S.tk[5] += (int64_t)(now_ticks() - t1);
     return true;
   }
   for (int x0 = tid; x0 < V; x0 += kR * G) {
@@ -1900,12 +1907,13 @@ __device__ __forceinline__ bool pivot_pass(const Ctx& C, const TreeLds& t, const
   }
   if (tid == 0) S.dlo[sel ^ 1] = 0x7fffffff;
   gsync<G>();
-  if (timed && tid == 0) S.tk[5] += kTimedEvery * (int64_t)(now_ticks() - t1);
+  if (timed && tid == 0) S.tk[5] += (int64_t)(now_ticks() - t1);
   return true;
 }
 
-// count: a running count of pivots, its parity alternating from one pivot to the next.  Returns false, in every rank,
-// when the tree is corrupt.
+// count: the solve's pivots so far (modulo kTimedEvery, or counted on from there): one pivot
+// to the next it grows by one, so its parity alternates.  Returns false, in every rank, when
+// the tree is corrupt.
 template <int G, bool kWideWin = false, class SN>
 __device__ __forceinline__ bool pivot(const Ctx& C, const TreeLds& t, const SN& sn, Shared& S, int ei, int ej,
                                       int32_t r, int count) {
@@ -1929,13 +1937,13 @@ __device__ __forceinline__ bool pivot(const Ctx& C, const TreeLds& t, const SN& 
 // accepted cycle, its reduced cost and its theta unchanged; they pivot best first.  The
 // best candidate always wins.  Rounds repeat on the same candidates (re-priced) up to
 // minor_limit times or until none prices negative; then the caller sweeps again.  iter: the
-// pivots made before, maxIt: the budget.
+// pivots made before, maxIt: the budget, count: the pivot count at iter = 0.
 // `claim` needs V words (the pivot's snapshot region, free between pivots).  Returns
 // the pivots made (-1: the tree is corrupt); stops at the iteration budget.
 // ---------------------------------------------------------------------------
 template <int G, class SN>
 __device__ __forceinline__ int multi_pivot(const Ctx& C, const TreeLds& t, const SN& sn, uint32_t* claim,
-                                           Shared& S, const Cand& cand, int iter, int maxIt, int rounds) {
+                                           Shared& S, const Cand& cand, int iter, int maxIt, int rounds, int count) {
   const int m = C.m, V = C.V, tid = grank<G>();
   constexpr uint32_t kRange = (1u << 22) - 1;
   const int I = cand.row, J = m + cand.col;
@@ -1972,7 +1980,7 @@ __device__ __forceinline__ int multi_pivot(const Ctx& C, const TreeLds& t, const
       const uint64_t k = group_min_u64<G>(accepted ? reprice(C, t, cand) : kNoKey, S);
       if (k == kNoKey || key_val(k) >= 0) break;
       if (accepted && key_idx(k) == mine) { accepted = false; spent = true; }
-      if (!pivot<G>(C, t, sn, S, cell_row(k), cell_col(k), key_val(k), iter + done)) return -1;
+      if (!pivot<G>(C, t, sn, S, cell_row(k), cell_col(k), key_val(k), count + iter + done)) return -1;
       ++done; ++inRound;
     }
     if (inRound == 0) break;  // nothing prices negative any more (uniform)
@@ -2094,6 +2102,7 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
   const bool lead = grank<G>() == 0;
   if (lead) {
     S.status = 0;
+    if (kCands) S.reprice_ticks = 0;
     for (int k = 0; k < 6; ++k) S.tk[k] = fresh ? 0 : D.ticks[k];
     if (fresh) D.t_start = now_ticks();
   }
@@ -2145,6 +2154,10 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
   int32_t status = 0;
   bool finished = false;
   int32_t done = 0, sweeps = 0;  // pivots and full sweeps of this call
+  int32_t priced = 0, timings = 0;  // candidate re-pricings of this call's earlier lists, those timed
+  // the earlier calls' pivots and sweeps, modulo kTimedEvery
+  const int32_t count0 = uniform((int32_t)iter0 & (kTimedEvery - 1));
+  const int32_t scount0 = fresh ? 0 : uniform((int32_t)D.sweeps & (kTimedEvery - 1));
   constexpr int K = kCands ? CandsPerRank<G>::value : 1;
   CandSet<K> cands;
   cands.clear();
@@ -2155,18 +2168,19 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
   for (;;) {
     uint64_t key;
     if (kCands && haveList && minor < P.minor_limit) {
-      const bool timed = timed_pivot(done);
+      const bool timed = timed_event(minor);
       if (timed) tp = now_ticks();
       key = group_min1_u64<G, 0>(reprice_set(t, cands), S);
-      if (timed && lead) S.tk[3] += kTimedEvery * (int64_t)(now_ticks() - tp);
-      if (key_val(key) >= 0) { haveList = false; continue; }
+      if (timed && lead) S.reprice_ticks += (int64_t)(now_ticks() - tp);
       ++minor;
+      if (key_val(key) >= 0) { haveList = false; continue; }
     } else {
-      // (candidate sweeps are few and all timed)
-      const bool timed = kCands || timed_pivot(done);
+      if (kCands) { priced += minor; timings += timed_events(minor); }
+      // (the other rules time every sweep: mostly one serves many pivots)
+      const bool timed = kRule != kRuleDantzig || timed_event(scount0 + sweeps);
       if (timed) tp = now_ticks();
       key = sweep_argmin<G, K>(C, t, S, shape, cands);
-      if (timed && lead) S.tk[2] += (kCands ? 1 : kTimedEvery) * (int64_t)(now_ticks() - tp);
+      if (timed && lead) S.tk[2] += (int64_t)(now_ticks() - tp);
       ++sweeps;
       haveList = kCands;
       minor = 0;
@@ -2191,9 +2205,9 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
         const bool sw = P.pricing == 4;
         int made;
         if constexpr (kSnapLdsOnly)
-          made = multi_pivot<G>(C, t, snL, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit);
+          made = multi_pivot<G>(C, t, snL, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit, count0);
         else
-          made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit);
+          made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cands.get(0), done, budget, sw ? 1 : P.minor_limit, count0);
         if (made < 0) { status = 2; finished = true; break; }
         done = uniform(done + made);
         if (sw && made < 10) mode = 1;
@@ -2202,8 +2216,8 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
     }
     const int ei = cell_row(key), ej = cell_col(key);
     bool ok;
-    if (kSnapLdsOnly || auxLds) ok = pivot<G, (G < 1024)>(C, t, snL, S, ei, ej, key_val(key), done);
-    else ok = pivot<G, (G < 1024)>(C, t, sn, S, ei, ej, key_val(key), done);
+    if (kSnapLdsOnly || auxLds) ok = pivot<G, (G < 1024)>(C, t, snL, S, ei, ej, key_val(key), count0 + done);
+    else ok = pivot<G, (G < 1024)>(C, t, sn, S, ei, ej, key_val(key), count0 + done);
     if (!ok) { status = 2; finished = true; break; }
     ++done;
   }
@@ -2216,11 +2230,17 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
     // a fresh instance's counters start at zero (the launch's reset cleared them)
     if (finished) D.status = status;
     D.phase = finished ? 2 : 1;
-    D.iterations = iter0 + done;
-    D.sweeps = (fresh ? 0 : D.sweeps) + sweeps;
+    const int64_t allPivots = (fresh ? 0 : D.iterations) + done, allSweeps = (fresh ? 0 : D.sweeps) + sweeps;
+    D.iterations = allPivots;
+    D.sweeps = allSweeps;
     D.mode = mode;
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
-    if (finished) D.t_done = now_ticks();
+    if (kCands) D.ticks[3] = S.tk[3] + scale_samples(S.reprice_ticks, priced + minor, timings + timed_events(minor));
+    if (finished) {
+      if (kRule == kRuleDantzig) D.ticks[2] = scale_samples(S.tk[2], allSweeps, timed_events(allSweeps));
+      for (int k = 4; k < 6; ++k) D.ticks[k] = scale_samples(S.tk[k], allPivots, timed_events(allPivots));
+      D.t_done = now_ticks();
+    }
   }
   gsync<G>();
 }
@@ -2330,6 +2350,7 @@ __device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& g
   if (phase != 1) return;
   if (lead) {
     S.status = 0;
+    if (kCands) S.reprice_ticks = 0;
     for (int k = 0; k < 6; ++k) S.tk[k] = D.ticks[k];
   }
   pivot_init<G>(S);
@@ -2388,13 +2409,14 @@ __device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& g
         const bool sw = P.pricing == 4;
         const int made = multi_pivot<G>(C, t, sn, (uint32_t*)aux, S, cand, 0,
                                         maxIt - iter < 0x7fffffff ? (int)(maxIt - iter) : 0x7fffffff,
-                                        sw ? 1 : P.minor_limit);
+                                        sw ? 1 : P.minor_limit, (int)iter);
         if (made < 0) { status = 2; finished = true; }
         else iter += made;
         if (sw && made < 10) mode = 1;
       }
     }
   }
+  int priced = 0;  // candidate re-pricings of this round
   if (!finished && !multiDone) {
     int minor = 0;
     for (;;) {
@@ -2406,11 +2428,12 @@ __device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& g
       if (!ok) { status = 2; finished = true; break; }
       ++iter;
       if (!kCands || ++minor >= P.minor_limit) break;  // Dantzig: one pivot per sweep
-      const bool timed = timed_pivot((int)iter);
+      const bool timed = timed_event(minor - 1);
       uint64_t tp = 0;
       if (timed) tp = now_ticks();
       key = group_min1_u64<G, 0>(reprice_set(t, cs), S);
-      if (timed && lead) S.tk[3] += kTimedEvery * (int64_t)(now_ticks() - tp);
+      if (timed && lead) S.reprice_ticks += (int64_t)(now_ticks() - tp);
+      priced = minor;
       if (key_val(key) >= 0) break;  // list exhausted: next full sweep
     }
   }
@@ -2422,10 +2445,14 @@ __device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& g
   }
   if (lead) {
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
+    if (kCands) D.ticks[3] = S.tk[3] + scale_samples(S.reprice_ticks, priced, timed_events(priced));
     D.iterations = iter;
     D.mode = mode;
     D.sweeps = D.sweeps + 1;
-    if (finished) { D.status = status; D.phase = 2; D.t_done = now_ticks(); }
+    if (finished) {
+      for (int k = 4; k < 6; ++k) D.ticks[k] = scale_samples(S.tk[k], iter, timed_events(iter));
+      D.status = status; D.phase = 2; D.t_done = now_ticks();
+    }
   }
 }
 

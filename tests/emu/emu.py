@@ -23,10 +23,11 @@ def load_variant(variant: str):
     L.emu_solve.argtypes = [ctypes.c_int, ctypes.c_int, i32p, i32p, i32p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                             ctypes.c_int, ctypes.c_int64, ctypes.c_int, i32p, i32p, i32p, i32p,
                             ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
-                            ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int64)]
+                            ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int64),
+                            ctypes.c_int64 * 6]
     L.emu_large.argtypes = [ctypes.c_int, ctypes.c_int, i32p, i32p, i32p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                             i32p, i32p, i32p, i32p, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64),
-                            ctypes.POINTER(ctypes.c_int32)]
+                            ctypes.POINTER(ctypes.c_int32), ctypes.c_int64 * 6]
     L.emu_group_bytes.restype = ctypes.c_int64
     L.emu_group_bytes.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64]
     return L
@@ -60,11 +61,13 @@ def solve(L, cost, supply, demand, group=64, groups_per_wg=4, pricing=0, initial
     du = np.zeros(V, np.int32)
     obj, it, sweeps = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int64()
     st, steps = ctypes.c_int32(), ctypes.c_int32()
+    ticks = (ctypes.c_int64 * 6)()
     r = L.emu_solve(m, n, cost.ravel(), np.ascontiguousarray(supply, np.int32), np.ascontiguousarray(demand, np.int32),
                     group, groups_per_wg, pricing, initial, max_it, step_pivots, br, bc, bf, du,
-                    ctypes.byref(obj), ctypes.byref(it), ctypes.byref(st), ctypes.byref(steps), ctypes.byref(sweeps))
+                    ctypes.byref(obj), ctypes.byref(it), ctypes.byref(st), ctypes.byref(steps),
+                    ctypes.byref(sweeps), ticks)
     return dict(ret=r, objective=obj.value, iterations=it.value, status=st.value, steps=steps.value, sweeps=sweeps.value,
-                rows=br, cols=bc, flows=bf, u=du[:m], v=du[m:])
+                ticks=list(ticks), rows=br, cols=bc, flows=bf, u=du[:m], v=du[m:])
 
 
 def large(L, cost, supply, demand, pricing=0, vpt=0, tree_global=0):
@@ -77,8 +80,9 @@ def large(L, cost, supply, demand, pricing=0, vpt=0, tree_global=0):
     br = np.zeros(V - 1, np.int32); bc = np.zeros(V - 1, np.int32); bf = np.zeros(V - 1, np.int32)
     du = np.zeros(V, np.int32)
     obj, it, st = ctypes.c_int64(), ctypes.c_int64(), ctypes.c_int32()
+    ticks = (ctypes.c_int64 * 6)()
     rounds = L.emu_large(m, n, cost.ravel(), np.ascontiguousarray(supply, np.int32),
                          np.ascontiguousarray(demand, np.int32), pricing, vpt, tree_global, br, bc, bf, du, ctypes.byref(obj),
-                         ctypes.byref(it), ctypes.byref(st))
-    return dict(rounds=rounds, objective=obj.value, iterations=it.value, status=st.value, rows=br, cols=bc, flows=bf,
+                         ctypes.byref(it), ctypes.byref(st), ticks)
+    return dict(rounds=rounds, ticks=list(ticks), objective=obj.value, iterations=it.value, status=st.value, rows=br, cols=bc, flows=bf,
                 u=du[:m], v=du[m:])

@@ -297,7 +297,7 @@ extern "C" int emu_solve(int m, int n, const int32_t* cost, const int32_t* suppl
                          int groups_per_wg, int pricing, int initial, int64_t max_it, int step_pivots,
                          int32_t* brow_out, int32_t* bcol_out, int32_t* bflow_out, int32_t* dual_out,
                          int64_t* objective, int64_t* iterations, int32_t* status, int32_t* steps_out,
-                         int64_t* sweeps_out) {
+                         int64_t* sweeps_out, int64_t* ticks_out) {
   const int V = m + n;
   const int ld = (n + 3) & ~3, ldT = (m + 3) & ~3;
   int32_t* c = exact<int32_t>((size_t)m * ld);
@@ -343,11 +343,14 @@ extern "C" int emu_solve(int m, int n, const int32_t* cost, const int32_t* suppl
   std::memcpy(dual_out, du, 4 * (size_t)V);
   *objective = D.objective; *iterations = D.iterations; *status = D.status; *steps_out = steps;
   *sweeps_out = D.sweeps;
+  std::memcpy(ticks_out, D.ticks, sizeof D.ticks);
   for (void* p : {(void*)c, (void*)cT, (void*)s, (void*)d, (void*)br, (void*)bc, (void*)bf, (void*)du, (void*)scr,
                   (void*)st, (void*)region})
     std::free(p);
   return aux_in_lds ? 1 : 0;
 }
+
+extern "C" void emu_unit_clock(int on) { emu::unit_clock = on != 0; }
 
 extern "C" int64_t emu_group_bytes(int m, int n, int64_t cap) {
   bool in_lds = false;
@@ -362,7 +365,8 @@ extern "C" int64_t emu_group_bytes(int m, int n, int64_t cap) {
 // holds only the group's scalars).  Returns the rounds run.
 extern "C" int emu_large(int m, int n, const int32_t* cost, const int32_t* supply, const int32_t* demand, int pricing,
                          int vpt_override, int tree_global, int32_t* brow_out, int32_t* bcol_out, int32_t* bflow_out,
-                         int32_t* dual_out, int64_t* objective, int64_t* iterations, int32_t* status) {
+                         int32_t* dual_out, int64_t* objective, int64_t* iterations, int32_t* status,
+                         int64_t* ticks_out) {
   const bool setup_only = pricing < 0;  // stop after the set-up kernel: the basis out is Vogel's
   if (setup_only) pricing = 0;
   const int V = m + n;
@@ -426,6 +430,7 @@ extern "C" int emu_large(int m, int n, const int32_t* cost, const int32_t* suppl
   std::memcpy(bcol_out, D.basis_col, 4 * (size_t)(V - 1));
   std::memcpy(bflow_out, D.basis_flow, 4 * (size_t)(V - 1));
   std::memcpy(dual_out, D.dual, 4 * (size_t)V);
+  std::memcpy(ticks_out, D.ticks, sizeof D.ticks);
   *objective = D.objective; *iterations = D.iterations; *status = D.status;
   for (void* p : {(void*)c, (void*)D.costT, (void*)s, (void*)d, (void*)D.basis_row, (void*)D.basis_col,
                   (void*)D.basis_flow, (void*)D.dual, (void*)D.scratch, (void*)D.state, (void*)region, (void*)keys,

@@ -187,7 +187,14 @@ inline int __clz(int x) { return x == 0 ? 32 : __builtin_clz((unsigned)x); }
 #define __builtin_amdgcn_fence(order, scope) std::atomic_thread_fence(std::memory_order_seq_cst)
 #define __builtin_amdgcn_wave_barrier() (emu::lane_ctx.wave->wait((int)(emu::lane_ctx.tid % 64), __LINE__))
 
+// Unit clock (switched on by a test): a lane's clock is the number of its readings, so a
+// timed event lasts exactly one tick.
+namespace emu {
+inline bool unit_clock = false;
+inline uint64_t readings[1024];
+}  // namespace emu
 inline uint64_t wall_clock64() {
+  if (emu::unit_clock) return ++emu::readings[emu::lane_ctx.tid];
   return (uint64_t)std::chrono::duration_cast<std::chrono::nanoseconds>(
              std::chrono::steady_clock::now().time_since_epoch()).count() / 10;
 }

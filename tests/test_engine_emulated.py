@@ -126,6 +126,35 @@ def test_emulated_expired_slice_deadline(pricing):
         assert r["iterations"] <= r["steps"]
 
 
+@pytest.mark.parametrize("pricing", [0, 1, 2, 4])
+def test_emulated_phase_timers(pricing):
+    """Phase times with a clock that makes every timed event one tick: the counts they scale
+    to are the events', whether the solve is whole, stops after its first pivots, is cut into
+    steps or runs as the large-instance kernels."""
+    sys.path.insert(0, EMU)
+    import emu
+    emu.build()
+    L = emu.load_variant("plain")
+    inst = I.random_instance(np.random.default_rng(33), 29, 24, 50, 100)
+    L.emu_unit_clock(1)
+    try:
+        for kw in (dict(), dict(max_it=1), dict(max_it=9), dict(step_pivots=3)):
+            r = emu.solve(L, inst.cost, inst.supply, inst.demand, group=64, pricing=pricing, **kw)
+            t, it, sw = r["ticks"], r["iterations"], r["sweeps"]
+            assert t[:2] == [1, 1] and t[4:] == [it, it] and t[2] == sw, (kw, t, it, sw)
+            # a candidate pivot follows a sweep or a re-pricing; every list may end with one more
+            if pricing == 1:
+                assert it - sw <= t[3] <= it + sw, (kw, t, it, sw)
+            else:
+                assert t[3] == 0
+        r = emu.large(L, inst.cost, inst.supply, inst.demand, pricing=pricing, vpt=16)
+        t, it = r["ticks"], r["iterations"]
+        assert t[:2] == [1, 1] and t[4:] == [it, it] and t[2] == 0
+        assert it - r["rounds"] <= t[3] <= it if pricing == 1 else t[3] == 0
+    finally:
+        L.emu_unit_clock(0)
+
+
 def test_emulated_wavefront_sweep_beyond_one_block():
     """64-lane groups with rows longer than a sweep block (256 vectors, n > 1024): the row
     is swept in chunks.  At, just past and well past the block's edge."""
