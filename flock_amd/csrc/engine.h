@@ -1,6 +1,6 @@
 // engine.h -- a group of threads solves one balanced transportation instance end to end:
-//   transpose -> Vogel (or north-west corner) -> basis tree in LDS (level-synchronous
-//   BFS over CSR, which also yields the duals) -> loop { reduced-cost sweep fused with
+//   transpose -> Vogel (or north-west corner) -> basis tree in LDS (level by level over
+//   the basic cells, which also yields the duals) -> loop { reduced-cost sweep fused with
 //   argmin -> stepping-stone pivot with parallel cycle discovery and parallel subtree
 //   re-rooting } -> basis, duals, objective.
 //
@@ -62,7 +62,7 @@ struct Shared {
   int32_t cnt;
   int32_t pend_row, pend_col;  // Vogel: kinds of line the next step rescans
   int32_t status;
-  int32_t level[3];   // tree build: whether a level reached anything, in turn
+  int32_t level[3];   // tree build: vertices that a level reached, in turn
   int32_t idx;
   int32_t stop;       // deadline reached (rank 0 decides, the group follows)
   int32_t pad0_[1];
@@ -165,12 +165,13 @@ __host__ __device__ inline size_t vogel_lds_bytes(int m, int n) {
          2 * align16(2 * (size_t)V) + align16((size_t)V);
 }
 // aux region in int32 units: max(tree-build scratch, path snapshot)
-//   build: cell ends, cell costs, depths, sizes, next positions, V each
+//   build: cell ends, cell costs, depths, sizes, next positions, V each, the vertices by
+//   level and where each level starts (int16)
 //   snapshot: for each side of the cycle, vertex, slot (int16), pre | size << 16 and flow (int32)
 //   of its vertices by depth, V entries each
 __host__ __device__ inline size_t aux_ints(int m, int n) {
   const size_t V = (size_t)(m + n);
-  const size_t build = 5 * V;
+  const size_t build = 5 * V + 2 * (V / 2 + 1);
   const size_t snap = 2 * (2 * ((V + 1) / 2 + 4) + 2 * (V + 4));
   return build > snap ? build : snap;
 }
@@ -1097,16 +1098,19 @@ __device__ __forceinline__ void set_dual(const TreeLds& t, int m, int x, int32_t
 // not used yet whose one end has the level's depth hangs its other end below it (parent,
 // depth, slot and dual, x_child = c(row,col) - x_parent, DUAL_solver.cu:52-62; the
 // reference's CSR, parallel_kernels.cu:205-319, is not needed for that).  Then subtree
-// sizes bottom-up and preorder numbers top-down, again level by level: a vertex takes its
-// interval from its parent's next free position (siblings in any order: preorder numbers
-// only serve ancestor tests).  Returns false if the cells do not form a spanning tree: of
-// V - 1 cells that leave no vertex unreached none closes a cycle.
-// Bound: three passes of one barrier and one or two LDS round trips per level, 94 levels at
-// 505x475.  The cells' ends and costs are read from global memory once.  (A BFS over a CSR
-// read its cells' rows, columns, flows and costs from global memory level by level, with
-// two barriers each, after a serial scan of the degrees: 130 us at 500x480, 21 us at 13x9,
-// 2.9 ms at 4000x2000.)
-// scr: 5 V ints (aux_ints).
+// sizes bottom-up and preorder numbers top-down, again level by level, over the level's own
+// vertices (the first pass lists them): a vertex takes its interval from its parent's next
+// free position (siblings in any order: preorder numbers only serve ancestor tests).
+// Returns false if the cells do not form a spanning tree: of V - 1 cells that leave no
+// vertex unreached none closes a cycle.
+// Bound: three passes of one barrier and a few LDS round trips per level, and the first
+// pass's look at every cell.  Levels are few in Vogel's trees (94 at 505x475), about 0.66 V
+// in a square north-west corner one.  The cells' ends and costs are read from global memory
+// once.  A BFS over a CSR, reading its cells from global memory level by level with two
+// barriers each, took 146 us at 490x490 and 24.2 ms at 4500x4500 north-west corner (tree in
+// global memory); size and preorder passes over every vertex 39 us and 32.0 ms; this 34 us
+// and 19.0 ms (1000x1000 north-west corner: 3.4, 1.9 and 1.3 ms).
+// scr: aux_ints.
 // ---------------------------------------------------------------------------
 template <int G>
 __device__ __forceinline__ bool build_tree(const Ctx& C, gcint* brow, gcint* bcol, gcint* bflow, const TreeLds& t, int32_t* scr,
@@ -1117,6 +1121,8 @@ __device__ __forceinline__ bool build_tree(const Ctx& C, gcint* brow, gcint* bco
   int32_t* dep = acost + V;  // V: depth, -1 unreached
   int32_t* size = dep + V;   // V
   int32_t* next = size + V;  // V: next free preorder position below the vertex
+  int16_t* order = (int16_t*)(next + V);  // V: the vertices but the root, level by level
+  int16_t* start = order + 2 * (V / 2 + 1);  // V+1: where depth d's vertices start in it, d = 1 ..
   int badCell = 0;
   for (int k = tid; k < V - 1; k += G) {
     const int r = brow[k], c = bcol[k];
@@ -1134,12 +1140,12 @@ __device__ __forceinline__ bool build_tree(const Ctx& C, gcint* brow, gcint* bco
   gsync<G>();
   if (S.status != 0) return false;
   constexpr int U = 4;  // cells a rank looks at together
-  int d = 0;
+  int d = 0, placed = 0;  // vertices placed so far, the same in every rank
   for (;; ++d) {
-    // whether this level reached anything; the flag of the next level is cleared here: it
-    // was last read two barriers ago
+    // how many vertices this level reaches; the counter of the next level is cleared here:
+    // it was last read two barriers ago
     int32_t* grown = &S.level[d % 3];
-    if (tid == 0) S.level[(d + 1) % 3] = 0;
+    if (tid == 0) { S.level[(d + 1) % 3] = 0; start[d + 1] = (int16_t)placed; }
     for (int k0 = tid; k0 < V - 1; k0 += U * G) {
       int32_t a[U], dr[U], dc[U];
 #pragma unroll
@@ -1159,17 +1165,19 @@ __device__ __forceinline__ bool build_tree(const Ctx& C, gcint* brow, gcint* bco
           set_dual(t, m, y, acost[k] - dual_of(t, m, x));
           lds_store(&dep[y], d + 1);
           arc[k] = -1;
-          lds_store(grown, 1);
+          order[placed + atomicAdd(grown, 1)] = (int16_t)y;  // (a cell once: at most V - 1)
         }
       }
     }
     gsync<G>();
-    if (lds_load(grown) == 0) break;  // uniform: written before the barrier
+    const int reached = uniform(lds_load(grown));  // written before the barrier
+    if (reached == 0) break;
+    placed += reached;
   }
-  // depths 1 .. d are in use
-  bool reached = true;
-  for (int x = tid; x < V; x += G) reached = reached & (dep[x] >= 0);
-  if (!reached) atomicAdd(&S.status, 1);
+  // depths 1 .. d are in use, and start[1 .. d + 1] set
+  bool all = true;
+  for (int x = tid; x < V; x += G) all = all & (dep[x] >= 0);
+  if (!all) atomicAdd(&S.status, 1);
   gsync<G>();
   if (S.status != 0) {  // (the caller reports the forest; the status is its own)
     gsync<G>();
@@ -1179,20 +1187,28 @@ __device__ __forceinline__ bool build_tree(const Ctx& C, gcint* brow, gcint* bco
   }
   for (int x = tid; x < V; x += G)
     if (x > 0) t.flow[x] = bflow[t.slot[x]];
+  int at = d > 0 ? start[d] : 0, end = placed;
   for (int dd = d; dd >= 1; --dd) {  // subtree sizes, deepest level first
-    for (int x = tid; x < V; x += G)
-      if (dep[x] == dd) atomicAdd(&size[t.parent[x]], size[x]);
+    const int before = dd > 1 ? start[dd - 1] : 0;
+    for (int q = at + tid; q < end; q += G) {
+      const int x = order[q];
+      atomicAdd(&size[t.parent[x]], size[x]);
+    }
+    end = at; at = before;
     gsync<G>();
   }
   if (tid == 0) { t.pre(0) = 0; next[0] = 1; }
   gsync<G>();
+  at = 0; end = d > 1 ? start[2] : placed;
   for (int dd = 1; dd <= d; ++dd) {
-    for (int x = tid; x < V; x += G)
-      if (dep[x] == dd) {
-        const int p = atomicAdd(&next[t.parent[x]], size[x]);
-        t.pre(x) = (int16_t)p;
-        next[x] = p + 1;
-      }
+    const int after = dd + 1 < d ? start[dd + 2] : placed;
+    for (int q = at + tid; q < end; q += G) {
+      const int x = order[q];
+      const int p = atomicAdd(&next[t.parent[x]], size[x]);
+      t.pre(x) = (int16_t)p;
+      next[x] = p + 1;
+    }
+    at = end; end = after;
     gsync<G>();
   }
   for (int x = tid; x < V; x += G) { t.size(x) = (int16_t)size[x]; t.depth[x] = (int16_t)dep[x]; }

@@ -88,6 +88,10 @@ def test_emulated_engine_matches_oracle():
         cases.append({"m": size + 14, "n": size + 9, "seed": 13 + g, "group": g, "pricing": 4})
         cases.append({"m": size + 6, "n": size + 11, "seed": 14 + g, "group": g, "pricing": 4, "steps": 3})
         cases.append({"m": size, "n": size, "seed": 6 + g, "group": g, "initial": 1})
+        # few and many cells a level, one and two levels
+        cases.append({"m": 1, "n": size, "seed": 15 + g, "group": g, "initial": 1, "smax": 9999})
+        cases.append({"m": size, "n": 1, "seed": 16 + g, "group": g, "initial": 1, "smax": 9999})
+        cases.append({"m": 4, "n": 3 * size, "seed": 17 + g, "group": g, "initial": 1, "smax": 9999})
         cases.append({"m": size - 5, "n": size - 15, "seed": 7 + g, "group": g, "steps": 7})
         # time slices (negative steps: slice length in clock ticks), one pivot per call
         cases.append({"m": size - 3, "n": size - 8, "seed": 11 + g, "group": g, "steps": -1})

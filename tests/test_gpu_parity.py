@@ -256,6 +256,24 @@ def test_vogel_line_slots_exact(threads, m, n, cmax):
     assert np.array_equal(s.u.astype(np.int64), o.u) and np.array_equal(s.v.astype(np.int64), o.v)
 
 
+# deep trees: a north-west corner start's has about 0.66 (m+n) levels when m = n, one or two
+# at m = 1 or n = 1; scratch in LDS, in global memory, and with the tree in global memory
+@pytest.mark.parametrize("threads,m,n", [(0, 1, 1), (0, 1, 40), (0, 40, 1), (64, 90, 91), (256, 300, 299), (512, 700, 701),
+                                         (1024, 2100, 2050), (0, 2000, 2001), (0, 4100, 4001)])
+def test_northwest_corner_tree_exact(threads, m, n):
+    """The tree of a north-west corner start: basis, duals and flows after one Dantzig pivot
+    equal the oracle's."""
+    rng = np.random.default_rng(m * 7 + n)
+    inst = _rand(rng, m, n, cmax=60, smax=900)
+    say("nwc tree", threads, m, n)
+    s = F.solve(inst, pricing="dantzig", initial="nwc", threads=threads, max_iterations=1)
+    o = oracle.solve(inst.cost, inst.supply, inst.demand, initial="nwc", max_iterations=1)
+    assert s.iterations == o.iterations
+    assert np.array_equal(s.rows, o.rows) and np.array_equal(s.cols, o.cols)
+    assert np.array_equal(s.flows.astype(np.int64), o.flows)
+    assert np.array_equal(s.u.astype(np.int64), o.u) and np.array_equal(s.v.astype(np.int64), o.v)
+
+
 def test_batch_mixed_configurations():
     """One batch mixing wavefront and workgroup classes, candidates pricing."""
     rng = np.random.default_rng(8)
