@@ -16,7 +16,7 @@ LIB = os.path.join(LIB_DIR, "libflock_amd.so")
 CLI = os.path.join(LIB_DIR, "flock")
 SOURCES = ["csrc/queue_512.hip", "csrc/queue_1024.hip", "csrc/queue_256.hip", "csrc/queue_wave.hip",
            "csrc/large.hip", "csrc/runtime.hip", "csrc/server.hip", "csrc/uv_model.hip", "csrc/noalloc.hip"]
-HEADERS = ["csrc/device_common.h", "csrc/engine.h", "csrc/kernels.h", "csrc/queue_kernel.h", "csrc/runtime_internal.h",
+HEADERS = ["csrc/device_common.h", "csrc/engine.h", "csrc/kernels.h", "csrc/queue_kernel.h", "csrc/policy.h", "csrc/runtime_internal.h",
            "../include/flock_amd.h", "../include/flock/structs.h", "../include/flock/uv_model_parallel.h"]
 
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -216,15 +216,15 @@ void get_policy(int* wave_max_v, int* wave_pack, int* wg256_max_v) {
 }
 
 // The 256- and 512-thread engines need the tree and the pivot's snapshot in LDS.
-static bool snap_fits_lds(int m, int n) {
+bool snap_fits_lds(int m, int n) {
   return shared_bytes() + tree_lds_bytes(m, n) + 4 * aux_ints(m, n) <= g_lds_max;
 }
-static int pick_cfg_raw(int V, const flock_options* opt, int64_t count, int batch_v);
-int pick_cfg(int m, int n, const flock_options* opt, int64_t count, int batch_v) {
-  const int c = pick_cfg_raw(m + n, opt, count, batch_v);
+static int pick_cfg_raw(int V, const flock_options* opt, int64_t count, const BatchShape* batch);
+int pick_cfg(int m, int n, const flock_options* opt, int64_t count, const BatchShape* batch) {
+  const int c = pick_cfg_raw(m + n, opt, count, batch);
   return (c == 3 || c == 4) && !snap_fits_lds(m, n) ? 5 : c;
 }
-static int pick_cfg_raw(int V, const flock_options* opt, int64_t count, int batch_v) {
+static int pick_cfg_raw(int V, const flock_options* opt, int64_t count, const BatchShape* batch) {
   const int threads = opt ? opt->threads : 0;   // threads per instance
   const int pack = opt ? opt->team : 0;         // instances per workgroup for wave groups
   if (threads == 64 || (threads == 0 && V <= g_wave_max_v)) {
@@ -238,13 +238,12 @@ static int pick_cfg_raw(int V, const flock_options* opt, int64_t count, int batc
   // A batch of at most one instance per compute unit takes its largest instance's choice
   // for all: classes launch one after another (200 instances of [16,400], dantzig 9.1 ms in
   // two classes, 7.8 in one; candidates 5.4, 4.3).
-  const int P = std::max(V, batch_v);
+  const int P = std::max(V, batch ? batch->max_v : 0);
   if (count <= g_cus) return P <= g_few_256_max_v ? 3 : (P <= g_few_512_max_v ? 4 : 5);
-  // Dantzig, a sweep per pivot, wants the 512 threads' sweep (beyond the smallest instances)
-  // until the device is full four times over (ms at 256 / 512 threads: 300 of [16,400] 10.0 / 8.4, 800 of [100,300] 9.9 /
-  // 9.0, 1600 of [100,300] 16.3 / 17.3); candidates do not (800 of [100,300] 3.8 / 6.5).
+  // Dantzig wants 512 threads for some batches (see dantzig_wide); candidates do not (800 of
+  // [100,300] 3.8 / 6.5 ms).
   const bool dantzig = !opt || opt->pricing == FLOCK_PRICE_DANTZIG;
-  if (dantzig && count <= 4 * (int64_t)g_cus && P > g_few_256_max_v) return 4;
+  if (dantzig && batch && batch->max_v > g_few_256_max_v && batch->dantzig_wide(g_cus)) return 4;
   return V <= g_wg256_max_v ? 3 : 4;
 }
 
@@ -445,9 +444,9 @@ int Batch::plan(const flock_options* opt) {
   const int64_t pkey = (((int64_t)key * 1000003 + wm * 31 + wp * 7 + w2) * 1000003 + g_few_256_max_v) * 1000003 +
                        g_few_512_max_v;
   if (planned_for == pkey) return FLOCK_OK;
-  int batch_v = 0;  // the largest m+n that a 512-thread workgroup takes
+  BatchShape shape;
   for (const Offs& o : offs)
-    if (snap_fits_lds(o.m, o.n)) batch_v = std::max(batch_v, o.m + o.n);
+    if (snap_fits_lds(o.m, o.n)) shape.add(o.m + o.n);
   classes.clear();
   std::vector<int32_t>& grouped = class_order;  // kept alive: the upload below is asynchronous
   grouped.clear();
@@ -459,7 +458,7 @@ int Batch::plan(const flock_options* opt) {
       cl.cfg = c; cl.begin = (int)grouped.size(); cl.lds = 0;
       bool dummy;
       for (int k : sorted_order) {
-        if (pick_cfg(offs[k].m, offs[k].n, opt, n, batch_v) != c || class_bucket(c, offs[k].m + offs[k].n) != b) continue;
+        if (pick_cfg(offs[k].m, offs[k].n, opt, n, &shape) != c || class_bucket(c, offs[k].m + offs[k].n) != b) continue;
         grouped.push_back(k);
         cl.lds = std::max(cl.lds, cfg_group_bytes(c, offs[k].m, offs[k].n, &dummy));
       }

@@ -6,6 +6,7 @@
 
 #include "../../include/flock_amd.h"
 #include "device_common.h"
+#include "policy.h"
 
 namespace flock {
 
@@ -28,8 +29,9 @@ int size_bucket(int V);
 int class_bucket(int cfg, int V);
 int cfg_threads(int c);
 int cfg_group(int c);
-// batch_v: the m+n that decides for a small batch as a whole (0: each instance by its own)
-int pick_cfg(int m, int n, const flock_options* opt, int64_t count, int batch_v = 0);
+// batch: the whole batch's sizes (null: the instance decides alone)
+int pick_cfg(int m, int n, const flock_options* opt, int64_t count, const BatchShape* batch = nullptr);
+bool snap_fits_lds(int m, int n);
 size_t cfg_group_bytes(int cfg, int m, int n, bool* aux_in_lds);
 void set_policy(int wave_max_v, int wave_pack, int wg256_max_v);
 void get_policy(int* wave_max_v, int* wave_pack, int* wg256_max_v);

@@ -42,6 +42,28 @@ def test_dropin_caller_built_with_cpp14():
     assert os.path.exists(os.path.join(ROOT, "tests", "cpp", "_build", "dropin_caller"))
 
 
+@pytest.mark.parametrize("count,lo,hi,wide", [
+    # measured on 256 units: 512 threads faster
+    (512, 16, 400, 1), (1024, 16, 400, 1), (257, 16, 256, 1), (257, 100, 300, 1), (1024, 100, 300, 1),
+    (768, 210, 240, 1), (512, 400, 430, 1), (1024, 200, 300, 1), (1024, 16, 300, 1), (512, 50, 250, 1), (1600, 16, 400, 1),
+    # and slower, by up to 2.3 times, or no faster
+    (257, 130, 140, 0), (1024, 130, 140, 0), (512, 60, 130, 0), (1024, 16, 130, 0), (768, 100, 180, 0),
+    (1024, 16, 200, 0), (1024, 16, 256, 0), (768, 180, 220, 0), (257, 400, 430, 0), (1600, 100, 300, 0), (1600, 200, 300, 0),
+    (4096, 16, 400, 0)])
+def test_dantzig_batch_threads(tmp_path_factory, count, lo, hi, wide):
+    """The launch policy's choice for Dantzig batches of more instances than compute units,
+    on both sides of each of its lines."""
+    import subprocess
+    exe = str(tmp_path_factory.getbasetemp() / "policy_check")
+    if not os.path.exists(exe):
+        subprocess.run(["g++", "-std=c++14", "-O1", "-Wall", "-Werror", "-o", exe,
+                        os.path.join(ROOT, "tests", "cpp", "policy_check.cpp")], check=True)
+    rng = np.random.default_rng(lo + hi)
+    v = rng.integers(lo, hi + 1, size=(2, count)).sum(axis=0)
+    r = subprocess.run([exe], input=" ".join(map(str, [256, *v])), capture_output=True, text=True, check=True)
+    assert int(r.stdout) == wide
+
+
 REF_MAIN = "/root/reference/src/main.cpp"
 
 
