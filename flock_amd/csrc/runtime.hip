@@ -1052,18 +1052,47 @@ int flock_autotune(int32_t count, const flock_instance* inst, const flock_option
       flock_tuning t = best; t.minor_limit = ml;
       if ((st = consider(t))) break;
     }
+  // Candidates that differ in their launch classes.  One that launches just what the best
+  // so far does is not measured: noise would choose a value that only other batches see
+  // (a small batch's threads do not depend on wg256_max_v, for one).
+  flock::Batch* B = reinterpret_cast<flock::Batch*>(b);
+  struct Plan {
+    std::vector<int> classes;
+    std::vector<int32_t> order;
+    bool operator==(const Plan& o) const { return classes == o.classes && order == o.order; }
+  };
+  auto plan_of = [&](const flock_tuning& t, Plan* p) -> int {
+    int e = flock_tuning_set(&t);
+    if (e || (e = B->plan(opt))) return e;
+    HIP_TRY(hipStreamSynchronize(flock::lib_stream()));  // the order's upload, before it is planned again
+    p->classes.clear();
+    for (const flock::Batch::Class& c : B->classes) p->classes.insert(p->classes.end(), {c.cfg, c.begin, c.count});
+    p->order = B->class_order;
+    return FLOCK_OK;
+  };
+  Plan bestPlan;
+  if (!st) st = plan_of(best, &bestPlan);
+  auto consider_plan = [&](const flock_tuning& t) -> int {
+    Plan p;
+    int e = plan_of(t, &p);
+    if (e || p == bestPlan) return e;
+    const double before = bms;
+    if ((e = consider(t))) return e;
+    if (bms < before) bestPlan = p;
+    return FLOCK_OK;
+  };
   // instances per workgroup: the smallest instances on one wavefront each, 1, 2 or 4 per
   // workgroup (their classes launch before the workgroup classes, one after another)
   for (int wv : {64, 128, 256})
     for (int pack : {1, 2, 4}) {
       if (st) break;
       flock_tuning t = best; t.wave_max_v = wv; t.wave_pack = pack;
-      st = consider(t);
+      st = consider_plan(t);
     }
   if (!st)
     for (int wg : {400, 600, 1200, 8000}) {
       flock_tuning t = best; t.wg256_max_v = wg;
-      if ((st = consider(t))) break;
+      if ((st = consider_plan(t))) break;
     }
   // raised wave priority for the largest instances (the launch's critical path)
   if (!st)

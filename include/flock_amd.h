@@ -195,8 +195,13 @@ void flock_server_destroy(flock_server* s);
 /* ---- size-class policy (which engine configuration solves an instance) ----------
  * Instances with m+n <= wave_max_v get one 64-lane wavefront each, wave_pack (1, 2 or
  * 4) per workgroup; larger ones get a 256-thread workgroup up to wg256_max_v, else a
- * 512-thread workgroup while their basis tree fits its LDS (m+n up to about 3600), else
- * 1024 threads.  flock_autotune() measures candidates on a sample and installs
+ * 512-thread workgroup while their basis tree fits its LDS (m+n up to about 3700), else
+ * 1024 threads.  Two kinds of batch do not look at wg256_max_v: those of at most one
+ * instance per compute unit (few_256_max_v and few_512_max_v below), and with Dantzig
+ * pricing those whose largest instances set the time, or of up to four large instances
+ * per compute unit, which take 512 threads where that measures faster (unless their
+ * largest m+n is at most few_256_max_v).
+ * flock_autotune() measures candidates on a sample and installs
  * the fastest; flock_tuning_set/get read and write the policy directly. */
 typedef struct flock_tuning {
   int32_t wave_max_v;
@@ -205,14 +210,15 @@ typedef struct flock_tuning {
   int32_t minor_limit;      /* candidate pricing: minor iterations per full sweep     */
   /* launches of at most one instance per compute unit (the plain solver, small batches)
    * favour per-instance latency: 256 threads up to few_256_max_v, 512 up to
-   * few_512_max_v, else 1024 */
+   * few_512_max_v, else 1024.  A batch as a whole follows its largest m+n (of those that
+   * 512 threads take), so that it is one launch */
   int32_t few_256_max_v;
   int32_t few_512_max_v;
   /* must be 0 (team sweeps, where idle workgroups helped sweep one large matrix, are
    * not part of this library; large matrices take the graph path below) */
   int32_t team_min_cells;
   /* plain solves of matrices with at least this many cells (four times as many with
-   * candidate pricing, for m+n up to about 3600) run as a graph of sweep-grid and
+   * candidate pricing, for m+n up to about 3700) run as a graph of sweep-grid and
    * pivot-round kernels (0: never) */
   int32_t graph_min_cells;
   /* per mille (0..1000) of each launch's instances, largest first, whose workgroups run at
@@ -236,7 +242,7 @@ int flock_tuning_set(const flock_tuning* t);
  * workgroup (a wavefront per instance, 1, 2 or 4 per workgroup, for the smallest
  * instances) and the raised-priority share), checks that every candidate returns the
  * same objectives, installs the fastest and returns it in *out with its batch time in
- * *best_ms. */
+ * *best_ms.  Thresholds that do not change the sample's launches keep their values. */
 int flock_autotune(int32_t count, const flock_instance* inst, const flock_options* opt, flock_tuning* out,
                    double* best_ms);
 

@@ -539,6 +539,22 @@ def test_autotune_installs_a_policy_with_identical_objectives():
         F.set_tuning(**before)
 
 
+@pytest.mark.parametrize("pricing,count,lo,hi", [("dantzig", 40, 20, 120), ("candidates", 40, 20, 120),
+                                                 ("dantzig", 300, 60, 215)])
+def test_autotune_keeps_thresholds_the_sample_does_not_depend_on(pricing, count, lo, hi):
+    """A batch of at most one instance per compute unit, and a Dantzig batch that takes 512
+    threads for its largest instances, launch the same whatever wg256_max_v is."""
+    rng = np.random.default_rng(count + hi)
+    insts = [_rand(rng, int(m), int(n), cmax=500, smax=900) for m, n in rng.integers(lo, hi + 1, size=(count, 2))]
+    before = F.get_tuning()
+    say("autotune thresholds", pricing, count)
+    try:
+        tuning, _ = F.autotune(insts, pricing=pricing)
+        assert tuning["wg256_max_v"] == before["wg256_max_v"]
+    finally:
+        F.set_tuning(**before)
+
+
 def test_autotune_large_picks_a_tile_shape_with_the_same_optimum():
     """flock_autotune_large tries every sweep tile shape on one large instance, requires the
     same objective from each (it fails otherwise) and installs the fastest; the installed
