@@ -492,9 +492,17 @@ int Batch::download_desc() {
   return FLOCK_OK;
 }
 
-int Batch::download_outputs() {
+int Batch::download_outputs(const flock_result* res) {
   h_out.resize(out_bytes);
-  HIP_TRY(hipMemcpyAsync(h_out.data(), (const char*)base + out_off, out_bytes, hipMemcpyDeviceToHost, g_stream));
+  for (int k0 = 0; k0 < n; ++k0) {  // one copy for every run of instances that ask
+    if (!wants_arrays(res[k0])) continue;
+    int k1 = k0;
+    while (k1 + 1 < n && wants_arrays(res[k1 + 1])) ++k1;
+    const size_t begin = offs[k0].brow, end = offs[k1].dual + 4 * (size_t)(offs[k1].m + offs[k1].n);
+    HIP_TRY(hipMemcpyAsync(h_out.data() + (begin - out_off), (const char*)base + begin, end - begin, hipMemcpyDeviceToHost,
+                           g_stream));
+    k0 = k1;
+  }
   HIP_TRY(hipStreamSynchronize(g_stream));
   return FLOCK_OK;
 }
@@ -889,7 +897,7 @@ int flock_solve(const flock_instance* inst, const flock_options* opt, flock_resu
   st = flock::large_runner()->run(b, P);
   if (st) { res->status = st; return st; }
   HIP_TRY(hipEventRecord(e1, flock::lib_stream()));
-  if ((st = b.download_desc()) || (flock::Batch::wants_arrays(*res) && (st = b.download_outputs()))) {
+  if ((st = b.download_desc()) || (flock::Batch::wants_arrays(*res) && (st = b.download_outputs(res)))) {
     res->status = st;
     return st;
   }
@@ -943,10 +951,11 @@ double flock_batch_last_ms(const flock_batch* bb) {
 int flock_batch_results(flock_batch* bb, flock_result* res) {
   flock::Batch* b = reinterpret_cast<flock::Batch*>(bb);
   if (!b || !res) return flock::set_error(FLOCK_E_INVALID, "null batch/result");
+  std::lock_guard<std::mutex> lk(b->results_mu);  // several threads may read one batch's results
   int st = b->download_desc();
   bool arrays = false;
   for (int k = 0; k < b->n; ++k) arrays = arrays || flock::Batch::wants_arrays(res[k]);
-  if (!st && arrays) st = b->download_outputs();
+  if (!st && arrays) st = b->download_outputs(res);
   if (st) return st;
   for (int k = 0; k < b->n; ++k) b->fill_result(k, &res[k]);
   return FLOCK_OK;

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <vector>
 
 #include "../../include/flock_amd.h"
@@ -73,6 +74,7 @@ struct Batch {
   std::vector<int32_t> class_order;
   size_t out_off = 0, out_bytes = 0;  // every instance's basis and duals, contiguous
   std::vector<char> h_out;            // their host copy (download_outputs)
+  std::mutex results_mu;              // hdesc, h_t0 and h_out while results are read
   int64_t planned_for = -1;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0;
@@ -85,7 +87,8 @@ struct Batch {
   int plan(const flock_options* opt);
   int run(const EngineParams& P, int grid_cap);
   int download_desc();
-  int download_outputs();
+  // the basis and duals of the instances whose results ask for arrays
+  int download_outputs(const flock_result* res);
   // needs download_desc(), and download_outputs() where the result asks for arrays
   void fill_result(int k, flock_result* r);
   static bool wants_arrays(const flock_result& r) {

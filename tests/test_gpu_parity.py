@@ -234,6 +234,46 @@ def test_batch_packed_copies(sizes):
         assert np.array_equal(s.flow_list, np.stack([s.rows[pos], s.cols[pos], s.flows[pos]], axis=1))
 
 
+def test_batch_results_for_some_instances_and_from_threads():
+    """Arrays only where a result asks for them (runs of askers at both ends and alone), and
+    one batch's results read by several threads at a time."""
+    import threading
+    rng = np.random.default_rng(77)
+    insts = [_rand(rng, int(m), int(n), cmax=300) for m, n in rng.integers(1, 60, size=(40, 2))]
+    say("some results")
+    b = F.Batch(insts)
+    b.run(pricing="dantzig")
+    whole = b.results()
+    ask = {0, 1, 5, 17, 18, 19, 39}
+    res = (F._Result * len(insts))()
+    keep = {}
+    for k in ask:
+        res[k], keep[k] = F._result_buffers(insts[k].m, insts[k].n)
+    assert F.lib().flock_batch_results(b._h, res) == 0
+    for k, w in enumerate(whole):
+        assert res[k].objective == w.objective and res[k].n_flows == w.n_flows
+        if k in ask:
+            s = F._solution(res[k], keep[k])
+            for f in ("rows", "cols", "flows", "u", "v", "flow_list"):
+                assert np.array_equal(getattr(s, f), getattr(w, f)), (k, f)
+    got = [None] * 8
+
+    def read(i):
+        got[i] = [b.results() for _ in range(5)]
+    ts = [threading.Thread(target=read, args=(i,)) for i in range(len(got))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for runs in got:
+        for sols in runs:
+            for s, w in zip(sols, whole):
+                assert s.objective == w.objective
+                for f in ("rows", "cols", "flows", "u", "v", "flow_list"):
+                    assert np.array_equal(getattr(s, f), getattr(w, f))
+    b.close()
+
+
 # Vogel's register mode: m+n at the edges of 4 and 8 lines per rank, with few distinct costs
 # (one covered line lists many others) and with many
 VOGEL_EDGES = [(64, 100, 156), (64, 100, 157), (256, 23, 1000), (256, 24, 1000), (256, 1000, 25), (512, 48, 2000),
