@@ -257,7 +257,9 @@ def _result_buffers(m: int, n: int):
 
 def _batch_buffers(insts, res):
     """Result arrays of a whole batch: one allocation per field, each instance's arrays
-    slices of it (six allocations per instance otherwise).  Sets the pointers in `res`."""
+    slices of it (six allocations per instance otherwise).  An array kept from one solution
+    therefore keeps the whole batch's; copy it to let the others go.  Sets the pointers in
+    `res`."""
     ms = [inst.m for inst in insts]
     ns = [inst.n for inst in insts]
     slots = sum(ms) + sum(ns) - len(insts)
@@ -335,6 +337,8 @@ class Batch:
         return lib().flock_batch_last_ms(self._h)
 
     def results(self, full: bool = True) -> list[Solution]:
+        """Solutions of the last run.  Their arrays (full=True) are slices of one allocation
+        per field for the whole batch: copy one to keep it without the others."""
         n = len(self.insts)
         res = (_Result * n)()
         bufs = _batch_buffers(self.insts, res) if full else None

@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -301,6 +302,16 @@ EngineParams make_params(const flock_options* opt) {
   return P;
 }
 
+// Grows a host buffer; an error code instead of an exception at the C entry points.
+static int host_buffer(std::vector<char>& buf, size_t size) {
+  try {
+    if (buf.size() < size) buf.resize(size);
+  } catch (const std::bad_alloc&) {
+    return set_error(FLOCK_E_DEVICE, "out of host memory (%zu bytes)", size);
+  }
+  return FLOCK_OK;
+}
+
 // ---------------------------------------------------------------------------
 // batch layout in one device allocation
 // ---------------------------------------------------------------------------
@@ -405,7 +416,8 @@ int Batch::upload(const flock_instance* inst, char* pinned, size_t pinned_cap) {
         if (k1 > k0 && e - begin > kUploadPiece) break;
         end = e; ++k1;
       }
-      if (piece.size() < end - begin) piece.resize(end - begin);
+      const int st = host_buffer(piece, end - begin);
+      if (st) return st;
       for (int k = k0; k < k1; ++k) {
         const Offs& o = offs[k];
         char* c = piece.data() + (o.cost - begin);
@@ -493,7 +505,8 @@ int Batch::download_desc() {
 }
 
 int Batch::download_outputs(const flock_result* res) {
-  h_out.resize(out_bytes);
+  const int st = host_buffer(h_out, out_bytes);
+  if (st) return st;
   for (int k0 = 0; k0 < n; ++k0) {  // one copy for every run of instances that ask
     if (!wants_arrays(res[k0])) continue;
     int k1 = k0;

@@ -153,7 +153,8 @@ int flock_batch_create(int32_t count, const flock_instance* inst, flock_batch** 
 int flock_batch_run(flock_batch* b, const flock_options* opt);
 /* Device time of the last run in ms (HIP events around the launch). */
 double flock_batch_last_ms(const flock_batch* b);
-/* Copy results of the last run to the host (res[k] for instance k). */
+/* Copy results of the last run to the host (res[k] for instance k).  Arrays come over only
+ * for instances whose res[k] asks for some, through a host copy that the handle keeps. */
 int flock_batch_results(flock_batch* b, flock_result* res);
 void flock_batch_free(flock_batch* b);
 
