@@ -111,13 +111,6 @@ struct EngineParams {
 // ---------------------------------------------------------------------------
 // reductions
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t x, int mask) {
-  uint32_t lo = (uint32_t)x, hi = (uint32_t)(x >> 32);
-  lo = __shfl_xor(lo, mask, kWave);
-  hi = __shfl_xor(hi, mask, kWave);
-  return ((uint64_t)hi << 32) | lo;
-}
-
 // DPP lane moves (GFX9 data-parallel primitives).  row_shr:k (0x110 + k) moves lane
 // i - k of the same 16-lane row into lane i; row_bcast:15 (0x142) moves lane 15 of row r
 // into every lane of row r + 1; row_bcast:31 (0x143) moves lane 31 into rows 2 and 3.
@@ -150,7 +143,7 @@ __device__ __forceinline__ uint64_t wave_reduce_u64(uint64_t x, uint64_t idn, Op
   x = op(x, dpp_u64<0x143, 0xc>(idn, x));
   return readlane_u64(x, 63);
 }
-// 32-bit wavefront min / sum, same DPP pattern on one register.
+// 32-bit wavefront min / max, same DPP pattern on one register.
 template <int kCtrl, int kRowMask>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t old, uint32_t src) {
   return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, kCtrl, kRowMask, 0xf, false);
@@ -166,13 +159,11 @@ __device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t x, uint32_t idn, Op
   return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
 }
 struct MaxU32 { __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return b > a ? b : a; } };
-struct AddU32 { __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return a + b; } };
-// Max and sum have identity 0, which is what a DPP move with bound_ctrl writes into lanes
+// Max has identity 0, which is what a DPP move with bound_ctrl writes into lanes
 // without a source, so the compiler folds each move into the operation (v_max_u32_dpp,
 // one instruction per step).  Min is taken as the complement of the max of complements.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) { return wave_reduce_u32(x, 0u, MaxU32{}); }
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) { return ~wave_max_u32(~x); }
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t x) { return wave_reduce_u32(x, 0u, AddU32{}); }
 
 struct AddU64 { __device__ __forceinline__ uint64_t operator()(uint64_t a, uint64_t b) const { return a + b; } };
 
@@ -224,22 +215,6 @@ __device__ __forceinline__ uint64_t block_min_u64(uint64_t x, uint64_t* red) {
   if (w == 0) {
     uint64_t y = l < W ? red[l] : kNoKey;
     y = wave_min_u64(y);
-    if (l == 0) red[W] = y;
-  }
-  __syncthreads();
-  return red[W];
-}
-
-template <int T>
-__device__ __forceinline__ uint64_t block_max_u64(uint64_t x, uint64_t* red) {
-  constexpr int W = T / kWave;
-  x = wave_max_u64(x);
-  const int w = threadIdx.x / kWave, l = threadIdx.x % kWave;
-  if (l == 0) red[w] = x;
-  __syncthreads();
-  if (w == 0) {
-    uint64_t y = l < W ? red[l] : 0ull;
-    y = wave_max_u64(y);
     if (l == 0) red[W] = y;
   }
   __syncthreads();

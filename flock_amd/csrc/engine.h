@@ -85,12 +85,6 @@ __device__ __forceinline__ uint64_t group_min_u64(uint64_t x, Shared& S) {
   if constexpr (G == kWave) return wave_min_u64(x);
   else return block_min_u64<G>(x, S.red);
 }
-template <int G>
-__device__ __forceinline__ uint64_t group_max_u64(uint64_t x, Shared& S) {
-  reduction_sync<G>();
-  if constexpr (G == kWave) return wave_max_u64(x);
-  else return block_max_u64<G>(x, S.red);
-}
 // One-barrier variants for the solve loop.  Buffer use: 0 candidate re-pricing and
 // Vogel's penalty argmax, 1 the pivot's leaving arc, 2 the full sweep; consecutive
 // reductions on one buffer always have another barrier between them.

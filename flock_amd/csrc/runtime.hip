@@ -204,8 +204,6 @@ int size_bucket(int V) {
 // several groups into one workgroup, so they are split by size bucket to keep small
 // instances dense.  Workgroup configurations launch once per configuration.
 int class_bucket(int cfg, int V) { return kCfgs[cfg].group == 64 ? size_bucket(V) : 0; }
-int cfg_threads(int c) { return kCfgs[c].threads; }
-int cfg_group(int c) { return kCfgs[c].group; }
 
 void set_policy(int wave_max_v, int wave_pack, int wg256_max_v) {
   if (wave_max_v >= 0) g_wave_max_v = std::min(wave_max_v, 2048);

@@ -28,8 +28,6 @@ int validate_instance(const flock_instance* in, int max_v = kMaxVertices);
 int num_cfgs();
 int size_bucket(int V);
 int class_bucket(int cfg, int V);
-int cfg_threads(int c);
-int cfg_group(int c);
 // batch: the whole batch's sizes (null: the instance decides alone)
 int pick_cfg(int m, int n, const flock_options* opt, int64_t count, const BatchShape* batch = nullptr);
 bool snap_fits_lds(int m, int n);

@@ -262,17 +262,12 @@ struct Server {
     int bigV = 0;
     for (int s : order)
       if (slots[s].m + slots[s].n > bigV) { bigV = slots[s].m + slots[s].n; maxm = slots[s].m; maxn = slots[s].n; }
-    // one engine configuration per slice, chosen for its largest request; raised where another
-    // request needs more threads: LDS follows m and n padded apart, so it need not grow with
-    // m+n (at the present layout and 160 KB no two requests straddle the limit, m+n = 3704)
+    // one engine configuration per slice, chosen for its largest request: what fits the
+    // 512-thread engine's LDS is m+n <= 3704, however m and n share it
     BatchShape shape;
     for (int s : order)
       if (snap_fits_lds(slots[s].m, slots[s].n)) shape.add(slots[s].m + slots[s].n);
-    int cfg = pick_cfg(maxm, maxn, &opt, (int64_t)order.size(), &shape);
-    for (int s : order) {
-      const int c = pick_cfg(slots[s].m, slots[s].n, &opt, (int64_t)order.size(), &shape);
-      if (cfg_threads(c) > cfg_threads(cfg)) cfg = c;
-    }
+    const int cfg = pick_cfg(maxm, maxn, &opt, (int64_t)order.size(), &shape);
     for (int s : order) {
       bool dummy;
       lds = std::max(lds, cfg_group_bytes(cfg, slots[s].m, slots[s].n, &dummy));

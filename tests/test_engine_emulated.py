@@ -130,6 +130,20 @@ def test_emulated_expired_slice_deadline(pricing):
         assert r["iterations"] <= r["steps"]
 
 
+def test_lds_limit_depends_on_the_vertex_count_alone():
+    """The tree and snapshot fit a workgroup's 160 KB for every instance of m+n <= 3704 and
+    for none above, so that the largest request of a server slice decides for all."""
+    sys.path.insert(0, EMU)
+    import emu
+    emu.build()
+    L = emu.load_variant("plain")
+    cap = 160 * 1024
+    for V in (3696, 3700, 3704, 3705, 3708, 3720):
+        got = {L.emu_group_bytes(m, V - m, cap) for m in range(1, V)}
+        # without the snapshot in LDS a region holds the tree alone, 20 of 44 bytes a vertex
+        assert all(40 * V < b <= cap for b in got) if V <= 3704 else all(b < 30 * V for b in got), V
+
+
 @pytest.mark.parametrize("pricing", [0, 1, 2, 4])
 def test_emulated_phase_timers(pricing):
     """Phase times with a clock that makes every timed event one tick: the counts they scale
