@@ -73,7 +73,7 @@ struct DevInstance {
   // device wall-clock ticks spent per phase (thread 0's view, summed over steps):
   // 0 transpose+Vogel, 1 tree build + duals, 2 full sweeps, 3 candidate re-pricing,
   // 4 pivot cycle discovery + leaving arc, 5 pivot flow update + re-rooting.  Where only
-  // samples are timed (4, 5, and 2 with Dantzig pricing) they hold the samples' sum until
+  // samples are timed (4, 5, and 2 but for candidate pricing) they hold the samples' sum until
   // the instance is done, then the sum scaled to every event
   int64_t ticks[6];
   uint64_t t_start;         // device wall clock when the instance's solve began / ended

@@ -1598,13 +1598,14 @@ struct IntC { static constexpr int value = N; };
 
 // Phase timers: reading the clock takes 80 cycles and drains the LDS queue, and a pivot has
 // four readings, so every eighth event of a kind is timed, the first one among them.  Events
-// are counted over the whole solve (pivots, Dantzig's sweeps) or from each sweep on
-// (candidate re-pricings), and the samples' sum is scaled to all of them at the end.
+// are counted over the whole solve (pivots, and sweeps but the candidate rule's few, which
+// are all timed) or over one call (candidate re-pricings), and the samples' sum is scaled to
+// all of them at the end.
 constexpr int kTimedEvery = 8;
 __device__ __forceinline__ bool timed_event(int count) { return count % kTimedEvery == 0; }
-__device__ __forceinline__ int64_t timed_events(int64_t events) { return (events + kTimedEvery - 1) / kTimedEvery; }
-__device__ __forceinline__ int64_t scale_samples(int64_t sum, int64_t events, int64_t timings) {
-  return timings > 0 ? (int64_t)((double)sum * ((double)events / (double)timings) + 0.5) : 0;
+__device__ __forceinline__ int64_t scale_samples(int64_t sum, int64_t events) {
+  const double samples = (double)((events + kTimedEvery - 1) / kTimedEvery);
+  return events > 0 ? (int64_t)((double)sum * ((double)events / samples) + 0.5) : 0;
 }
 
 // kR: vertices each rank handles per pass, their LDS loads issued together.
@@ -2164,7 +2165,7 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
   int32_t status = 0;
   bool finished = false;
   int32_t done = 0, sweeps = 0;  // pivots and full sweeps of this call
-  int32_t priced = 0, timings = 0;  // candidate re-pricings of this call's earlier lists, those timed
+  int32_t priced = 0;            // candidate re-pricings of this call's earlier lists
   // the earlier calls' pivots and sweeps, modulo kTimedEvery
   const int32_t count0 = uniform((int32_t)iter0 & (kTimedEvery - 1));
   const int32_t scount0 = fresh ? 0 : uniform((int32_t)D.sweeps & (kTimedEvery - 1));
@@ -2178,16 +2179,15 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
   for (;;) {
     uint64_t key;
     if (kCands && haveList && minor < P.minor_limit) {
-      const bool timed = timed_event(minor);
+      const bool timed = timed_event(priced + minor);
       if (timed) tp = now_ticks();
       key = group_min1_u64<G, 0>(reprice_set(t, cands), S);
       if (timed && lead) S.reprice_ticks += (int64_t)(now_ticks() - tp);
       ++minor;
       if (key_val(key) >= 0) { haveList = false; continue; }
     } else {
-      if (kCands) { priced += minor; timings += timed_events(minor); }
-      // (the other rules time every sweep: mostly one serves many pivots)
-      const bool timed = kRule != kRuleDantzig || timed_event(scount0 + sweeps);
+      priced += minor;
+      const bool timed = kCands || timed_event(scount0 + sweeps);
       if (timed) tp = now_ticks();
       key = sweep_argmin<G, K>(C, t, S, shape, cands);
       if (timed && lead) S.tk[2] += (int64_t)(now_ticks() - tp);
@@ -2245,10 +2245,10 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
     D.sweeps = allSweeps;
     D.mode = mode;
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
-    if (kCands) D.ticks[3] = S.tk[3] + scale_samples(S.reprice_ticks, priced + minor, timings + timed_events(minor));
+    if (kCands) D.ticks[3] = S.tk[3] + scale_samples(S.reprice_ticks, priced + minor);
     if (finished) {
-      if (kRule == kRuleDantzig) D.ticks[2] = scale_samples(S.tk[2], allSweeps, timed_events(allSweeps));
-      for (int k = 4; k < 6; ++k) D.ticks[k] = scale_samples(S.tk[k], allPivots, timed_events(allPivots));
+      if (!kCands) D.ticks[2] = scale_samples(S.tk[2], allSweeps);
+      for (int k = 4; k < 6; ++k) D.ticks[k] = scale_samples(S.tk[k], allPivots);
       D.t_done = now_ticks();
     }
   }
@@ -2455,12 +2455,12 @@ __device__ __forceinline__ void large_round(DevInstance& D, const DevInstance& g
   }
   if (lead) {
     for (int k = 0; k < 6; ++k) D.ticks[k] = S.tk[k];
-    if (kCands) D.ticks[3] = S.tk[3] + scale_samples(S.reprice_ticks, priced, timed_events(priced));
+    if (kCands) D.ticks[3] = S.tk[3] + scale_samples(S.reprice_ticks, priced);
     D.iterations = iter;
     D.mode = mode;
     D.sweeps = D.sweeps + 1;
     if (finished) {
-      for (int k = 4; k < 6; ++k) D.ticks[k] = scale_samples(S.tk[k], iter, timed_events(iter));
+      for (int k = 4; k < 6; ++k) D.ticks[k] = scale_samples(S.tk[k], iter);
       D.status = status; D.phase = 2; D.t_done = now_ticks();
     }
   }

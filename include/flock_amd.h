@@ -103,7 +103,7 @@ typedef struct flock_result {
    * [0] transpose + Vogel, [1] tree build + duals, [2] full reduced-cost sweeps,
    * [3] candidate re-pricing, [4] pivot cycle discovery + leaving arc,
    * [5] pivot flow update + subtree re-rooting (incremental duals).  [3] to [5], and [2]
-   * with Dantzig pricing, are estimates: the first and every eighth re-pricing, pivot or
+   * but for candidate pricing, are estimates: the first and every eighth re-pricing, pivot or
    * sweep is timed, and the sum scaled to all of them.  Plain solves on the graph path do
    * not time their sweeps ([2] is 0) */
   double phase_us[6];
