@@ -159,8 +159,8 @@ constexpr int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
 // get a whole workgroup of 256 threads up to g_wg256_max_v, else 512 threads while the tree
 // and the pivot's snapshot fit LDS (m+n up to about 3700), else 1024.  A workgroup of 1024
 // loses at every size that 512 can take: its barriers cost 144 cycles instead of 48 and
-// four waves share each SIMD (61x1203 dantzig 8.4 against 6.2 ms, 100x2400 candidates 15.7
-// against 13.3 ms, 1800x1700 candidates 100 against 92 ms).
+// four waves share each SIMD (device ms at 1024 / 512: 61x1203 dantzig 8.2 / 5.3, 470x500
+// dantzig 24.7 / 17.7, 100x2400 candidates 12.3 / 9.9, 1800x1700 candidates 104 / 98).
 static int g_wave_max_v = 0;
 static int g_wave_pack = 4;
 static int g_wg256_max_v = 2000;
@@ -171,7 +171,7 @@ static int g_prio_permille = 0;
 // large-instance path: 16-byte cost vectors per thread in one tile of the sweep grid
 // (256 threads per tile), i.e. the tile shape; tiles = ceil(vectors / (256 * this))
 static int g_sweep_vectors = 4;
-static int g_large_threads = 512;  // large-instance setup / round workgroup (512 or 1024)
+static int g_large_threads = 512;  // large-instance round workgroup (512 or 1024)
 static int g_large_minor_limit = 64;  // large-instance path's candidate minor limit (0: g_minor_limit)
 // launches of at most one instance per compute unit: 256 threads up to the first, 512 up to
 // the second (where they fit LDS), else 1024
@@ -180,10 +180,11 @@ static int g_few_512_max_v = kMaxVertices;
 // plain solves of matrices with at least this many cells take the graph path; with
 // candidate pricing, where a sweep serves tens of pivots, at least kCandGraphFactor times
 // as many if the 512-thread engine can take them (device ms, engine against graph path:
-// dantzig 420x430 15.3 / 15.1, 500x500 18.9 / 16.3; candidates 800x800 17.8 / 19.8, 1000x1000
-// 28.4 / 28.0, 1300x1300 49.4 / 46.5, 1800x1700 92 / 72)
+// dantzig 420x430 14.1 / 13.6, 500x500 18.1 / 15.0; candidates, the sum of three cost ranges,
+// 600x600 30.9 / 32.0, 300x2000 46.5 / 48.2, 700x700 38.7 / 38.3, 800x800 48.1 / 45.2, 950x1000
+// 65.7 / 55.4, 250x3400 66.8 / 57.1; 1300x1300 46.0 / 37.4 alone)
 static int g_graph_min_cells = 250000;
-constexpr int kCandGraphFactor = 4;
+constexpr int kCandGraphFactor = 2;
 
 // the kernels' pricing rule (the switch rule starts with multi-pivot rounds)
 static int rule_of(const EngineParams& P) {
@@ -235,12 +236,12 @@ static int pick_cfg_raw(int V, const flock_options* opt, int64_t count, const Ba
   if (threads == 512) return 4;
   if (threads == 1024) return 5;
   // A batch of at most one instance per compute unit takes its largest instance's choice
-  // for all: classes launch one after another (200 instances of [16,400], dantzig 9.1 ms in
-  // two classes, 7.8 in one; candidates 5.4, 4.3).
+  // for all: classes launch one after another (200 instances of [16,400], dantzig 15.0 ms in
+  // two classes, 13.9 in one; candidates 7.1, 6.0).
   const int P = std::max(V, batch ? batch->max_v : 0);
   if (count <= g_cus) return P <= g_few_256_max_v ? 3 : (P <= g_few_512_max_v ? 4 : 5);
   // Dantzig wants 512 threads for some batches (see dantzig_wide); candidates do not (800 of
-  // [100,300] 3.8 / 6.5 ms).
+  // [100,300] 4.1 ms at 256, 7.5 at 512).
   const bool dantzig = !opt || opt->pricing == FLOCK_PRICE_DANTZIG;
   if (dantzig && batch && batch->max_v > g_few_256_max_v && batch->dantzig_wide(g_cus)) return 4;
   return V <= g_wg256_max_v ? 3 : 4;
@@ -567,8 +568,9 @@ namespace flock {
 // ---------------------------------------------------------------------------
 constexpr int kRoundsPerGraph = 32;
 constexpr int kLargeTiles = 1024;   // sweep workgroups at most
-// setup / round workgroup: 1024 threads, or 512 (g_large_threads) for instances whose
-// tree stays in LDS and whose m+n is at most 2048 (four vertices per rank in a pivot)
+// round workgroup: 1024 threads, or 512 (g_large_threads) for instances whose tree stays in
+// LDS and whose m+n is at most 2048 (four vertices per rank in a pivot); the set-up's has a
+// rule of its own (in run)
 constexpr int kLargeSmallMaxV = 2048;
 
 struct LargeRunner {
@@ -1162,7 +1164,7 @@ int flock_autotune_large(const flock_instance* inst, const flock_options* opt, f
     if ((st = measure(t, &ms))) break;
     if (ms < bms) { bms = ms; best = t; }
   }
-  for (int th : {512, 1024}) {  // set-up / round workgroup, at the best tile shape
+  for (int th : {512, 1024}) {  // round workgroup, at the best tile shape
     if (st || th == best.large_threads) continue;
     flock_tuning t = best; t.large_threads = th;
     double ms = 0;

@@ -218,7 +218,7 @@ typedef struct flock_tuning {
   /* must be 0 (team sweeps, where idle workgroups helped sweep one large matrix, are
    * not part of this library; large matrices take the graph path below) */
   int32_t team_min_cells;
-  /* plain solves of matrices with at least this many cells (four times as many with
+  /* plain solves of matrices with at least this many cells (twice as many with
    * candidate pricing, for m+n up to about 3700) run as a graph of sweep-grid and
    * pivot-round kernels (0: never) */
   int32_t graph_min_cells;
@@ -249,7 +249,7 @@ int flock_autotune(int32_t count, const flock_instance* inst, const flock_option
 
 /* Autotuner of the large-instance path: solves `inst` (at least graph_min_cells cells, or
  * m+n > 8000) on the graph path with each sweep tile shape (1, 2, 4, 8
- * vectors per thread), then at the best shape with the other set-up / round workgroup
+ * vectors per thread), then at the best shape with the other round workgroup
  * size (512 or 1024 threads), then (candidate pricing) with the path's minor limit at
  * 32, 64 and 128, two solves each, checks that the objectives agree, installs the
  * fastest and returns it in *out with its solve time (device ms) in *best_ms. */

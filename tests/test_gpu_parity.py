@@ -562,6 +562,17 @@ def test_instances_too_large_for_256_thread_lds_use_the_1024_engine():
         F.set_tuning(**before)
 
 
+@pytest.mark.parametrize("m,n", [(707, 707), (708, 707), (2500, 200), (131, 3590)])
+def test_candidates_on_both_sides_of_the_graph_threshold(m, n):
+    """Just under and over 500 000 cells, and an instance whose snapshot does not fit the
+    512-thread engine's LDS (graph path from 250 000 cells): the oracle's optimum, certified."""
+    inst = I.random_instance(np.random.default_rng(m + n), m, n, 1000, 100 * max(m, n))
+    say("graph threshold", m, n)
+    s = F.solve(inst, pricing="candidates")
+    assert s.status == 0 and certify(inst, s) == (0, s.objective)
+    assert s.objective == oracle.solve(inst.cost, inst.supply, inst.demand).objective
+
+
 def test_autotune_installs_a_policy_with_identical_objectives():
     """flock_autotune measures policies on a sample, requires identical objectives from
     every one (it fails otherwise), and installs the fastest."""
