@@ -41,17 +41,17 @@ __device__ __forceinline__ int grank() {
   return r;
 }
 
+// One wavefront executes in lockstep; this orders its LDS/global accesses for the compiler
+// and the memory model at wavefront scope.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 template <int G>
 __device__ __forceinline__ void gsync() {
-  if constexpr (G == kWave) {
-    // one wavefront executes in lockstep; this orders its LDS/global accesses for the
-    // compiler and the memory model at wavefront scope
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  } else {
-    __syncthreads();
-  }
+  if constexpr (G == kWave) wave_sync();
+  else __syncthreads();
 }
 
 // Scalars shared by one group; they sit at the start of the group's LDS region.
@@ -475,6 +475,7 @@ __device__ __forceinline__ void wave_book_track(gcshort* book, gcint* data, int 
                                                 const uint8_t* crossCov, int lane, int b, TRK* out, uint8_t* nt,
                                                 uint32_t& k1, uint32_t& k2) {
   int at = *pos, found = 0, first = -1;
+  wave_sync();  // every lane has the position before lane 0 moves it
   uint32_t r0 = ~0u, r1 = ~0u;  // this lane's key if it holds rank 0 / rank 1
   while (at < len && found <= kTrack) {
     const int q = at + lane;
@@ -523,6 +524,7 @@ __device__ __forceinline__ void row_book_track(gcshort* book, gcint* data, int l
                                                uint32_t& k2) {
   const int shift = lane & ~15, sl = lane & 15;
   int at = *pos, found = 0, first = -1;
+  wave_sync();  // every lane has the position before a row's first lane moves it
   uint32_t r0 = ~0u, r1 = ~0u;
   for (;;) {
     const bool on = active && at < len && found <= kTrack;

@@ -205,7 +205,12 @@ def test_emulated_engine_thread_sanitizer():
              # rule's claims, a north-west corner start
              {"m": 40, "n": 20, "seed": 12, "group": 64, "degenerate": True},
              {"m": 21, "n": 17, "seed": 13, "group": 64, "pricing": 2},
-             {"m": 18, "n": 12, "seed": 14, "group": 64, "initial": 1}]
+             {"m": 18, "n": 12, "seed": 14, "group": 64, "initial": 1},
+             # the large-instance kernels: Vogel on books with equal costs (more listed lines
+             # than wavefronts) and with few, the tree in LDS and in global memory
+             {"m": 13, "n": 11, "seed": 15, "group": 256, "cmax": 1, "large": True, "vpt": 4},
+             {"m": 9, "n": 14, "seed": 16, "group": 256, "cmax": 2, "large": True, "vpt": 8, "tree_global": 2, "pricing": 1},
+             {"m": 12, "n": 8, "seed": 17, "group": 256, "large": True, "vpt": 4, "tree_global": 1, "pricing": 2}]
     check(run("tsan", cases))
 
 
