@@ -2203,7 +2203,7 @@ __device__ __forceinline__ void solve_instance(DevInstance& D, char* region, siz
     // one decision for the whole group, >= 1 pivot per call: after every sweep (where it
     // costs little beside it), and on every fourth pivot of a candidate list (the clock, a
     // barrier and, past the deadline, a read of the launch's counter)
-    if (P.deadline && done > 0 && (!kCands || done % 4 == 1)) {
+    if (P.deadline && (kCands ? done % 4 == 1 : done > 0)) {
       if (lead)
         S.stop = now_ticks() >= P.deadline &&
                  (!P.busy || __hip_atomic_load(P.busy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0);
